@@ -35,10 +35,11 @@ HOST_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-Wall"]
 
 SOURCES = ["errors.cpp", "synth.cpp", "quant.hip", "gemm.hip", "model.hip", "sampler.hip"]
 
-# Per-source device flags. quant.hip: MFMA results straight into VGPRs (the
-# GEMV kernels consume each result at once; in AGPRs every one of them costs a
-# v_accvgpr_read). The GEMM keeps the default: its accumulator tiles live in AGPRs.
-EXTRA_FLAGS = {"quant.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+# Per-source device flags. quant.hip, gemm.hip: MFMA results straight into
+# VGPRs (the GEMV kernels consume each result at once, the row products fold
+# theirs into f32 sums; in AGPRs every one of them costs a v_accvgpr_read).
+EXTRA_FLAGS = {"quant.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+               "gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def _deps(src: str) -> list[str]:

@@ -1,29 +1,22 @@
 // quantized_matmul_rows (crates/mivi-quant/src/lib.rs:143-357) for gfx950.
 //
-// batch == 1 is exactly the matvec path (lib.rs:171-182). Q4_K and Q6_K with
-// at least kMfmaMinBatch rows run on the matrix cores:
+// batch == 1 is exactly the matvec path (lib.rs:171-182). From kMfmaMinBatch
+// rows on (rows_route below) the products run on the matrix cores:
 //
-//   gemm_prep_kernel   one workgroup per input row: scales the row by a power
-//                      of two 2^-e (so that |x| <= 1), splits it into fp16
-//                      hi + lo (x = hi + lo to about 2^-22 relative) and forms
-//                      the fp32 sums of each 32-value sub-block, also split;
-//   gemm_q4k_kernel    64 x 256 output tiles (input rows x weight rows),
-//                      v_mfma_f32_32x32x16_f16. The
-//                      B operand is sc*q of the Q4_K sub-block, an integer
-//                      <= 945 and so exact in fp16; one MFMA chain per 256-value
-//                      super-block gives sum(sc q x), folded into the fp32
-//                      accumulator as acc += d * C. The min term of
-//                      q4_k_m.rs:24-63, dmin * sum_sub m_sub * X_sub, runs on
-//                      the same MFMA shape with B = m (K = 8 sub-blocks padded
-//                      to 16) and is subtracted the same way. The row scale
-//                      2^e is applied at the store.
-//   gemm_q6k_kernel    the same tiles for Q6_K: B = q (exact in fp16), the
-//                      per-sub-block scale d * sc applied to each k-step's
-//                      chain (one 32 x 32 x 16 product per 16-value
-//                      sub-block).
+//   gemm_prep_kernel   one wave per input row: the prologue, then the row
+//                      split into 16-bit planes in MFMA operand order (fp16
+//                      hi + lo under a power-of-two row scale; bf16 hi + mid
+//                      + lo for bf16 weights);
+//   gemm_rows_kernel   v_mfma_f32_32x32x16 with both operands loaded straight
+//                      from memory into registers, one wave per 64 x 64
+//                      outputs and share of the depth.
 //
-// Other formats, and fewer rows, run the batched GEMV (the inputs as its
-// columns).
+// Every weight enters the products exactly (Q4_K: sc * q, an integer <= 945;
+// Q6_K and Q8_0: the integer q, its scale applied to the f32 sums; F16 and
+// BF16: the value itself), so the inputs' split and the f32 sums are the only
+// roundings. Other formats and shapes, and fewer rows, run the batched GEMV
+// (the inputs as its columns).
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 #include <vector>
@@ -40,141 +33,208 @@ using namespace mivi;
 
 namespace {
 
-constexpr int kMfmaMinBatch = 16;
-constexpr int kTm = 64;             // input rows of a GEMM tile
-constexpr int kTk = 64;             // k-tile: one Q4_K group (a sub-block pair)
-constexpr int kXs = kTk + 8;        // padded LDS row (halves) of an x or B tile
+constexpr int kMfmaMinBatch = 16;     // K-quants at the depths of the batched GEMVs
+constexpr int kMfmaMinBatchRows = 4;  // shapes with one GEMV launch per input
+constexpr int kMfmaMinBatchQ8 = 6;    // the same, Q8_0
+constexpr int kTk = 64;  // k-tile of the packed copy: one Q4_K group (a sub-block pair)
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // ---------------------------------------------------------------- prep
-// grid = Mp rows, 256 threads, K = 8 * 256 * r (thread t owns values
-// [8t, 8t + 8) of each 2048-value stretch). Row m < M is v = pro(X row m)
-// with X row m at X + m * ldx: PRO_NONE v = x; PRO_RMSNORM v = (x * s) * w,
-// s = 1/sqrt(mean(x^2) + eps) (norm.rs:38-72); PRO_SWIGLU v = silu(x) * x2
-// (math.rs:87-95, X2 row m at X2 + m * ldx). Then e = exponent with
-// max|v| * 2^-e <= 1; xh/xl = fp16 hi/lo of v * 2^-e; sh/sl = fp16 hi/lo of
-// each 32-value sub-block sum of v * 2^-e (fp32). Rows >= M are zero.
-typedef _Float16 half8p __attribute__((ext_vector_type(8)));
-// R > 0: K = 2048 R, the thread's 8 R values (and norm weights or up values)
-// loaded once and held in registers through both reductions; R = 0: any K,
-// each pass re-reading them. The same operations in the same order either way.
-template <int R>
-__global__ void __launch_bounds__(256) gemm_prep_kernel(const float* __restrict__ X, const float* __restrict__ X2,
+// Row m of the activations, v = pro(X row m) with X row m at X + m * ldx
+// (PRO_NONE v = x; PRO_RMSNORM v = (x * s) * w, s = 1/sqrt(mean(x^2) + eps)
+// (norm.rs:38-72); PRO_SWIGLU v = silu(x) * x2 (math.rs:87-95), X2 row m at
+// X2 + m * ldx), into the A operand of the row products.
+//
+// fp16 planes (P = 2): the row scaled by the power of two that puts its
+// largest finite |v| in [2^14, 2^15) (so the lo part of a value within 2^-15
+// of the largest is no denormal) and split v = hi + lo, each rounded to
+// nearest: v to about 2^-24 relative. bf16 planes (P = 3, bf16 weights, whose
+// range fp16 does not cover): v = hi + mid + lo unscaled. An infinite value
+// keeps its hi part only (no inf - inf).
+// Operand order: per 32 rows and 16-value k-step, one 1 KB block per plane,
+// lane l = m % 32 + 32 h holding the values 16 ks + 8 h .. + 7 (16 bytes) of
+// row m, at ((m / 32) * (K / 16) + ks) * P + plane) KB. Rows >= M are zero.
+// Q4_K also takes the 32-value sub-block sums of the scaled row, times 2^-5
+// (a sum may reach 2^20, past fp16's range), as fp16 hi / lo: per 32 rows and
+// super-block a 1 KB block, lane m % 32 the eight hi parts, lane m % 32 + 32
+// the lo parts.
+//
+// One wave per row, eight rows per workgroup: an operand line of 128 bytes
+// holds eight consecutive rows' chunks of eight values, so the workgroup
+// writes whole lines (through LDS). One row per workgroup wrote every line in
+// eight pieces from eight workgroups, each a partial write to memory: 18 us at
+// 512 x 8192 against 6 here. Lane l owns the chunks l + 64 j; J > 0: at most J
+// of them, held in registers through both reductions; J = 0: any K, the row
+// re-read by each pass. vec: rows (and norm weights) 16-byte aligned.
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+constexpr int kStepBytes = 1024;  // one operand block: 32 rows x 16 values of 16 bits
+constexpr int kPrepRows = 8;
+
+template <int J, int P>
+__global__ void __launch_bounds__(512) gemm_prep_kernel(const float* __restrict__ X, const float* __restrict__ X2,
                                                         const float* __restrict__ norm_w, float eps, int pro,
-                                                        int64_t ldx, int M, int K, _Float16* __restrict__ xh,
-                                                        _Float16* __restrict__ xl, _Float16* __restrict__ sh,
-                                                        _Float16* __restrict__ sl, float* __restrict__ rowscale) {
-    __shared__ float red[4];
-    const int m = blockIdx.x;
+                                                        int64_t ldx, int M, int K, int vec, uint8_t* __restrict__ xa,
+                                                        uint8_t* __restrict__ xs, float* __restrict__ rowscale) {
+    constexpr int C = 4;  // chunks of a lane per write pass
+    __shared__ __attribute__((aligned(16))) uint8_t buf[C * P * 64 * kPrepRows * 16];
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int m = kPrepRows * blockIdx.x + w;
     const bool live = m < M;
     const float* x = X + (live ? m : 0) * ldx;
     const float* x2 = pro == PRO_SWIGLU ? X2 + (live ? m : 0) * ldx : nullptr;
-    auto block_red = [&](float v, bool is_max) {
-        v = is_max ? wave_max(v) : wave_sum(v);
-        __syncthreads();
-        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-        __syncthreads();
-        return is_max ? fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])) : (red[0] + red[1]) + (red[2] + red[3]);
-    };
-    // the 8 values [i, i + 8) of a row as two 16-byte loads
     auto load8 = [&](const float* p, int i, float (&v)[8]) {
-        const f32x4 a = *(const f32x4*)(p + i), b = *(const f32x4*)(p + i + 4);
-        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-    };
-    constexpr int RR = R > 0 ? R : 1;
-    float xr[RR][8], wr[RR][8];  // R > 0: x and (norm w | up) of stretch r
-    if constexpr (R > 0) {
+        if (vec) {
+            const f32x4 a = *(const f32x4*)(p + i), b = *(const f32x4*)(p + i + 4);
+            v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+        } else {
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-#pragma unroll
-            for (int q = 0; q < 8; q++) { xr[r][q] = 0.f; wr[r][q] = 0.f; }
-            if (live) {
-                load8(x, 2048 * r + 8 * threadIdx.x, xr[r]);
-                if (pro == PRO_RMSNORM) load8(norm_w, 2048 * r + 8 * threadIdx.x, wr[r]);
-                else if (pro == PRO_SWIGLU) load8(x2, 2048 * r + 8 * threadIdx.x, wr[r]);
-            }
+            for (int q = 0; q < 8; q++) v[q] = p[i + q];
         }
-    }
+    };
+    const int nj = J > 0 ? J : (K + 511) / 512;
+    constexpr int JJ = J > 0 ? J : 1;
+    float v[JJ][8];
     float scale = 1.0f;
+    // chunk j of the prologue's input: x, or silu(x) * x2
+    auto input = [&](int j, float (&o)[8]) {
+        const int i = 8 * (lane + 64 * j);
+#pragma unroll
+        for (int q = 0; q < 8; q++) o[q] = 0.f;
+        if (!live || i >= K) return;
+        load8(x, i, o);
+        if (pro == PRO_SWIGLU) {
+            float u[8];
+            load8(x2, i, u);
+#pragma unroll
+            for (int q = 0; q < 8; q++) o[q] = silu_f(o[q]) * u[q];
+        }
+    };
+    auto normed = [&](int j, float (&o)[8]) {
+        const int i = 8 * (lane + 64 * j);
+        if (pro != PRO_RMSNORM || !live || i >= K) return;
+        float g[8];
+        load8(norm_w, i, g);
+#pragma unroll
+        for (int q = 0; q < 8; q++) o[q] = o[q] * scale * g[q];
+    };
+    if constexpr (J > 0) {
+#pragma unroll
+        for (int j = 0; j < J; j++) input(j, v[j]);
+    }
     if (pro == PRO_RMSNORM) {
         float ss = 0.f;
-        if constexpr (R > 0) {
 #pragma unroll
-            for (int r = 0; r < R; r++)
+        for (int j = 0; j < nj; j++) {
+            float (&o)[8] = v[J > 0 ? j : 0];
+            if (J == 0) input(j, o);
 #pragma unroll
-                for (int q = 0; q < 8; q++) ss = fmaf(xr[r][q], xr[r][q], ss);
-        } else if (live) {
-            for (int i = 8 * threadIdx.x; i < K; i += 8 * 256) {
-                float v[8];
-                load8(x, i, v);
-#pragma unroll
-                for (int q = 0; q < 8; q++) ss = fmaf(v[q], v[q], ss);
-            }
+            for (int q = 0; q < 8; q++) ss = fmaf(o[q], o[q], ss);
         }
-        ss = block_red(ss, false);
+        ss = wave_sum(ss);
         scale = 1.0f / sqrtf(ss / (float)K + eps);
     }
-    auto values = [&](int r, int i, float (&v)[8]) {  // pro(x)[i .. i + 8), i = 2048 r + 8 t
-        float w[8];
-        if constexpr (R > 0) {
+    if constexpr (J > 0) {
 #pragma unroll
-            for (int q = 0; q < 8; q++) { v[q] = xr[r][q]; w[q] = wr[r][q]; }
-        } else {
-            load8(x, i, v);
-            if (pro == PRO_RMSNORM) load8(norm_w, i, w);
-            else if (pro == PRO_SWIGLU) load8(x2, i, w);
+        for (int j = 0; j < J; j++) normed(j, v[j]);
+    }
+    float inv = 1.0f;
+    if constexpr (P == 2) {
+        float mx = 0.f;
+#pragma unroll
+        for (int j = 0; j < nj; j++) {
+            float (&o)[8] = v[J > 0 ? j : 0];
+            if (J == 0) { input(j, o); normed(j, o); }
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                const float av = fabsf(o[q]);
+                mx = av <= 3.40282347e38f ? fmaxf(mx, av) : mx;
+            }
         }
-        if (pro == PRO_RMSNORM) {
+        mx = wave_max(mx);
+        // max * 2^-e in [2^14, 2^15); e >= -110 keeps 2^-e finite
+        int e = 0;
+        if (mx > 0.f) {
+            frexpf(mx, &e);
+            e = max(e - 15, -110);
+        }
+        inv = ldexpf(1.0f, -e);
+        if (lane == 0) rowscale[m] = live ? ldexpf(1.0f, e) : 0.f;
+    } else if (lane == 0) {
+        rowscale[m] = live ? 1.0f : 0.f;
+    }
+    // chunk j as planes into buf: [chunk of the pass][plane][lane][row], the
+    // rows of a lane permuted by the lane so that the writes of a wave hit
+    // distinct banks
+    auto split = [&](int j, int c, float (&o)[8]) {
+        const int i = 8 * (lane + 64 * j);
+        uint8_t* dst = buf + ((c * P * 64 + lane) * kPrepRows + (w ^ (lane & 7))) * 16;
+        constexpr int PS = 64 * kPrepRows * 16;
+        if constexpr (P == 2) {
+            half8 hv, lv;
+            float sum = 0.f;
 #pragma unroll
-            for (int q = 0; q < 8; q++) v[q] = v[q] * scale * w[q];
-        } else if (pro == PRO_SWIGLU) {
+            for (int q = 0; q < 8; q++) {
+                const float s = o[q] * inv;  // exact: power-of-two scaling
+                hv[q] = (_Float16)s;
+                const float rest = s - (float)hv[q];
+                lv[q] = fabsf(s) <= 3.40282347e38f ? (_Float16)rest : (_Float16)0.0f;
+                sum += s;
+            }
+            *(half8*)dst = hv;
+            *(half8*)(dst + PS) = lv;
+            if (xs) {
+                // 4 consecutive lanes hold one 32-value sub-block
+                sum += __shfl_xor(sum, 1, 64);
+                sum += __shfl_xor(sum, 2, 64);
+                if ((lane & 3) == 0 && i < K) {
+                    sum *= 0.03125f;
+                    const _Float16 h = (_Float16)sum;
+                    uint8_t* sp = xs + ((size_t)(m >> 5) * (K / 256) + i / 256) * kStepBytes + 16 * (m & 31) + 2 * ((i / 32) & 7);
+                    *(_Float16*)sp = h;
+                    *(_Float16*)(sp + 512) = (_Float16)(sum - (float)h);
+                }
+            }
+        } else {
+            bf16x8 b[3];
 #pragma unroll
-            for (int q = 0; q < 8; q++) v[q] = silu_f(v[q]) * w[q];
+            for (int q = 0; q < 8; q++) {
+                b[0][q] = (__bf16)o[q];
+                const bool fin = fabsf((float)b[0][q]) <= 3.40282347e38f;
+                const float r1 = fin ? o[q] - (float)b[0][q] : 0.f;
+                b[1][q] = (__bf16)r1;
+                b[2][q] = (__bf16)(r1 - (float)b[1][q]);
+            }
+#pragma unroll
+            for (int p = 0; p < 3; p++) *(bf16x8*)(dst + p * PS) = b[p];
         }
     };
-    // stretch r of the thread: values [2048 r + 8 t, + 8)
-    auto more = [&](int r) { return R > 0 ? r < R : 2048 * r + 8 * (int)threadIdx.x < K; };
-    float mx = 0.f;
-    if (live)
-        for (int r = 0; more(r); r++) {  // (R > 0: unrolled, the registers indexed statically)
-            const int i = 2048 * r + 8 * threadIdx.x;
-            float v[8];
-            values(r, i, v);
+    const int r = threadIdx.x & 7, l8 = threadIdx.x >> 3;  // the thread's row and chunk lane when writing
+    const int mw = kPrepRows * blockIdx.x + r;
+    uint8_t* xrow = xa + ((size_t)(mw >> 5) * (K / 16) * P) * kStepBytes + 16 * (mw & 31);
 #pragma unroll
-            for (int q = 0; q < 8; q++) mx = fmaxf(mx, fabsf(v[q]));
+    for (int j0 = 0; j0 < nj; j0 += C) {
+        if (j0) __syncthreads();
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            const int j = j0 + c;
+            if (J > 0 && j >= J) break;
+            float (&o)[8] = v[J > 0 ? j : 0];
+            if (J == 0) { input(j, o); normed(j, o); }
+            split(j, c, o);
         }
-    mx = block_red(mx, true);
-    // 2^-e with max * 2^-e in [1/2, 1); e = 0 for an all-zero row
-    int e = 0;
-    if (mx > 0.f && mx <= 3.40282347e38f) frexpf(mx, &e);
-    const float inv = ldexpf(1.0f, -e);
-    if (threadIdx.x == 0) rowscale[m] = live ? ldexpf(1.0f, e) : 0.f;
-    for (int r = 0; more(r); r++) {
-        const int i = 2048 * r + 8 * threadIdx.x;
-        float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (live) values(r, i, v);
+        __syncthreads();
+        const int k8 = l8 + 64 * j0;
 #pragma unroll
-        for (int q = 0; q < 8; q++) v[q] *= inv;  // exact: power-of-two scaling
-        half8p hv, lv;
-        float sum = 0.f;
+        for (int c = 0; c < C; c++) {
+            const int k = k8 + 64 * c;
+            if (8 * k >= K) break;
+            uint8_t* d = xrow + (size_t)(k >> 1) * P * kStepBytes + (k & 1) * 512;
 #pragma unroll
-        for (int q = 0; q < 8; q++) {
-            hv[q] = (_Float16)v[q];
-            lv[q] = (_Float16)(v[q] - (float)hv[q]);
-            sum += v[q];
-        }
-        *(half8p*)(xh + (size_t)m * K + i) = hv;
-        *(half8p*)(xl + (size_t)m * K + i) = lv;
-        // 4 consecutive threads hold one 32-value sub-block
-        sum += __shfl_xor(sum, 1, 64);
-        sum += __shfl_xor(sum, 2, 64);
-        if ((threadIdx.x & 3) == 0) {
-            const _Float16 h = (_Float16)sum;
-            sh[(size_t)m * (K / 32) + i / 32] = h;
-            sl[(size_t)m * (K / 32) + i / 32] = (_Float16)(sum - (float)h);
+            for (int p = 0; p < P; p++)
+                *(u32x4*)(d + p * kStepBytes) = *(const u32x4*)(buf + (((c * P + p) * 64 + l8) * kPrepRows + (r ^ (l8 & 7))) * 16);
         }
     }
 }
@@ -191,253 +251,10 @@ __device__ __forceinline__ void scale_min_k4(const uint8_t* q, int j, uint32_t& 
     }
 }
 
-// The 6-bit scale of sub-block j (0..7) from a block header held in
-// registers (dwords 1..3 = the 12 scale bytes), get_scale_min_k4 of
-// q4_k_m.rs:11-22 with byte selects by shifts, so j may vary at run time.
-__device__ __forceinline__ uint32_t scale_k4(const u32x4& hdr, int j) {
-    const int sh = 8 * (j & 3);
-    const uint32_t a = (hdr.y >> sh) & 0xFFu;  // q[j & 3]
-    const uint32_t c = (hdr.w >> sh) & 0xFFu;  // q[8 + (j & 3)]
-    return j < 4 ? (a & 63u) : ((c & 0xFu) | ((a >> 6) << 4));
-}
-
-// 8 nibbles (bytes of w0, w1; low or high nibble) times sc, as exact fp16
-__device__ __forceinline__ half8 nib8_times(uint32_t w0, uint32_t w1, bool high, _Float16 sc) {
-    uint32_t t0 = high ? (w0 >> 4) & 0x0F0F0F0Fu : w0 & 0x0F0F0F0Fu;
-    uint32_t t1 = high ? (w1 >> 4) & 0x0F0F0F0Fu : w1 & 0x0F0F0F0Fu;
-    // fp16 1024 + q has bit pattern 0x6400 | q: bytes [q, 0x64]
-    const uint32_t p0 = __builtin_amdgcn_perm(0x64646464u, t0, 0x07010700u);  // q0, q1
-    const uint32_t p1 = __builtin_amdgcn_perm(0x64646464u, t0, 0x07030702u);  // q2, q3
-    const uint32_t p2 = __builtin_amdgcn_perm(0x64646464u, t1, 0x07010700u);
-    const uint32_t p3 = __builtin_amdgcn_perm(0x64646464u, t1, 0x07030702u);
-    const half2v off = {(_Float16)-1024.0f, (_Float16)-1024.0f};
-    const half2v s2 = {sc, sc};
-    half2v h0 = (__builtin_bit_cast(half2v, p0) + off) * s2;
-    half2v h1 = (__builtin_bit_cast(half2v, p1) + off) * s2;
-    half2v h2 = (__builtin_bit_cast(half2v, p2) + off) * s2;
-    half2v h3 = (__builtin_bit_cast(half2v, p3) + off) * s2;
-    return half8{h0.x, h0.y, h1.x, h1.y, h2.x, h2.y, h3.x, h3.y};
-}
-
-// The outputs of one lane, 2 x 16 registers: acc[i][r] is row row(i, r),
-// column col(i); y (=|+=) acc * rowscale[row]. Every row scale and (with
-// accumulate) every old value is loaded before the first store: the stores
-// could alias later loads as far as the compiler knows, and each load would
-// otherwise wait for the store before it and then for its own memory trip.
-template <class RowF, class ColF>
-__device__ __forceinline__ void gemm_store(float* __restrict__ Y, int64_t ldy, int M, int N,
-                                           const float* __restrict__ rowscale, const f32x16 (&acc)[2], RowF row,
-                                           ColF col, int accumulate) {
-    float rs[2][16], old[2][16];
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const int n = col(i);
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int m = row(i, r);
-            const bool in = m < M && n < N;
-            rs[i][r] = in ? rowscale[m] : 0.f;
-            old[i][r] = in && accumulate ? Y[m * ldy + n] : 0.f;
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const int n = col(i);
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int m = row(i, r);
-            if (m < M && n < N) {
-                const float v = acc[i][r] * rs[i][r];
-                Y[m * ldy + n] = accumulate ? old[i][r] + v : v;  // one writer per output
-            }
-        }
-    }
-}
-
-// grid = (ceil(N / 256), Mp / 64), 512 threads = 8 waves: wave w computes
-// input rows 32 (w & 1) .. +32 of the tile against weight rows 64 (w >> 1)
-// .. +64 (two 32 x 32 MFMA tiles). Per 64-value k-tile the workgroup stages x
-// (fp16 hi and lo, 16 KB, shared by the eight waves) and builds the fp16 B
-// operand sc*q once into LDS (two threads per weight row, from qs bytes and
-// scales held in registers), so no wave repeats another's conversion. LDS
-// holds two k-tiles: while the waves run the products of tile t from one
-// buffer they build tile t + 1 in the other, so a k-tile costs one barrier,
-// and each tile's bytes are loaded two tiles ahead into one of three
-// register stages. 120 KB of LDS: one workgroup (eight waves) per CU.
-constexpr int kGT = 512;  // threads of a GEMM workgroup
-constexpr int kGN = 256;  // weight rows of its tile
-
-struct GemmStage {
-    u32x4 xh, xl;       // x chunk of 8 values: input row tid/8, chunk tid%8
-    u32x4 qs, hdr, ps;  // 16 qs bytes of weight row bn; its block header; sub-block sums (tid < 128)
-};
-
-struct GemmBuf {
-    _Float16 Xh[kTm][kXs];
-    _Float16 Xl[kTm][kXs];
-    _Float16 Bt[kGN][kXs];  // sc * q of the k-tile, weight-row major
-};
-
-__global__ void __launch_bounds__(kGT) gemm_q4k_kernel(const uint8_t* __restrict__ W, int N, int K,
-                                                       const _Float16* __restrict__ xh,
-                                                       const _Float16* __restrict__ xl,
-                                                       const _Float16* __restrict__ sh,
-                                                       const _Float16* __restrict__ sl,
-                                                       const float* __restrict__ rowscale, float* __restrict__ Y,
-                                                       int M, int64_t ldy, int accumulate) {
-    __shared__ __attribute__((aligned(16))) GemmBuf buf[2];
-    // per super-block (by its parity): d, dmin, scales (rows 20 B apart, so
-    // the 32 rows a wave reads fall in distinct banks); sub-block sums of x
-    __shared__ __attribute__((aligned(16))) uint8_t Wh[2][kGN][20];
-    __shared__ __attribute__((aligned(16))) _Float16 Sh[2][kTm][8];
-    __shared__ __attribute__((aligned(16))) _Float16 Sl[2][kTm][8];
-    const int n0 = blockIdx.x * kGN, m0 = blockIdx.y * kTm;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave & 1, wn = wave >> 1;
-    const int nb = K / 256;
-    const size_t rb = (size_t)nb * 144;
-    const int li = lane & 31, lh = lane >> 5;
-    // B building: weight row bn of the tile, qs bytes [16 bc, 16 bc + 16) of
-    // the group; each 16 threads cover 8 rows x 2 halves, eight consecutive
-    // lanes on eight rows (their LDS rows 144 B apart hit distinct banks)
-    const int bn = 8 * (tid >> 4) + (tid & 7), bc = (tid >> 3) & 1;
-    const uint8_t* brow = W + (size_t)(n0 + bn < N ? n0 + bn : N - 1) * rb;
-    const int xr = tid >> 3, xc = tid & 7;  // x staging: row xr, values 8 xc .. +8 of the k-tile
-
-    f32x16 acc[2], c1[2];
-#pragma unroll
-    for (int nt = 0; nt < 2; nt++) {
-        acc[nt] = f32x16{};
-        c1[nt] = f32x16{};
-    }
-
-    const int ntiles = K / kTk;
-    auto load_tile = [&](GemmStage& S, int t) {
-        const int k0 = t * kTk;
-        const size_t o = (size_t)(m0 + xr) * K + k0 + 8 * xc;
-        S.xh = *(const u32x4*)(xh + o);
-        S.xl = *(const u32x4*)(xl + o);
-        const int b = k0 / 256, g = (k0 % 256) / 64;
-        S.qs = *(const u32x4*)(brow + (size_t)b * 144 + 16 + 32 * g + 16 * bc);
-        if (g == 0) {
-            S.hdr = *(const u32x4*)(brow + (size_t)b * 144);
-            if (tid < 2 * kTm) {
-                const int rr = tid >> 1, half = tid & 1;
-                S.ps = half ? *(const u32x4*)(sl + (size_t)(m0 + rr) * (K / 32) + 8 * b)
-                            : *(const u32x4*)(sh + (size_t)(m0 + rr) * (K / 32) + 8 * b);
-            }
-        }
-    };
-    u32x4 hdr = {};  // this thread's weight row header of the super-block being built
-    auto store_tile = [&](const GemmStage& S, int t) {
-        GemmBuf& B = buf[t & 1];
-        *(u32x4*)&B.Xh[xr][8 * xc] = S.xh;
-        *(u32x4*)&B.Xl[xr][8 * xc] = S.xl;
-        const int g = t & 3, p = (t >> 2) & 1;
-        if (g == 0) {
-            hdr = S.hdr;
-            if (bc == 0) {
-                uint32_t* w = (uint32_t*)&Wh[p][bn][0];
-                w[0] = S.hdr.x; w[1] = S.hdr.y; w[2] = S.hdr.z; w[3] = S.hdr.w;
-            }
-            if (tid < 2 * kTm) {
-                if (tid & 1) *(u32x4*)&Sl[p][tid >> 1][0] = S.ps;
-                else *(u32x4*)&Sh[p][tid >> 1][0] = S.ps;
-            }
-        }
-        // values 16bc .. 16bc+15 of sub-blocks 2g (low nibbles) and 2g+1 (high)
-        const _Float16 s0 = (_Float16)(float)scale_k4(hdr, 2 * g), s1 = (_Float16)(float)scale_k4(hdr, 2 * g + 1);
-        *(half8*)&B.Bt[bn][16 * bc] = nib8_times(S.qs.x, S.qs.y, false, s0);
-        *(half8*)&B.Bt[bn][16 * bc + 8] = nib8_times(S.qs.z, S.qs.w, false, s0);
-        *(half8*)&B.Bt[bn][32 + 16 * bc] = nib8_times(S.qs.x, S.qs.y, true, s1);
-        *(half8*)&B.Bt[bn][32 + 16 * bc + 8] = nib8_times(S.qs.z, S.qs.w, true, s1);
-    };
-
-    const int ar = 32 * wm + li;  // this lane's A row (input row of the tile)
-    auto compute = [&](int t) {
-        const GemmBuf& B = buf[t & 1];
-#pragma unroll
-        for (int s = 0; s < 4; s++) {
-            // k-step s: values 16s .. 16s+15 of the group; lane half lh holds 8 of them
-            const half8 a_h = *(const half8*)&B.Xh[ar][16 * s + 8 * lh];
-            const half8 a_l = *(const half8*)&B.Xl[ar][16 * s + 8 * lh];
-            half8 bq[2];
-#pragma unroll
-            for (int nt = 0; nt < 2; nt++) bq[nt] = *(const half8*)&B.Bt[64 * wn + 32 * nt + li][16 * s + 8 * lh];
-#pragma unroll
-            for (int nt = 0; nt < 2; nt++) c1[nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_h, bq[nt], c1[nt], 0, 0, 0);
-#pragma unroll
-            for (int nt = 0; nt < 2; nt++) c1[nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_l, bq[nt], c1[nt], 0, 0, 0);
-        }
-        if ((t & 3) == 3) {
-            // end of super-block: acc += d * C, then the min term
-            // dmin * sum_sub m_sub * X_sub on the same MFMA shape
-            const int p = (t >> 2) & 1;
-            float d[2], dm[2];
-            half8 bm[2];
-#pragma unroll
-            for (int nt = 0; nt < 2; nt++) {
-                const int r = 64 * wn + 32 * nt + li;
-                const uint32_t w0 = *(const uint32_t*)&Wh[p][r][0];
-                d[nt] = half_bits_to_f32(w0);
-                dm[nt] = half_bits_to_f32(w0 >> 16);
-                // B[k][n] = m of sub-block k for k < 8, 0 for k = 8..15 (lane half 1)
-                half8 v = {};
-                if (lh == 0) {
-#pragma unroll
-                    for (int j = 0; j < 8; j++) {
-                        uint32_t sc, mm;
-                        scale_min_k4(&Wh[p][r][4], j, sc, mm);
-                        v[j] = (_Float16)(float)mm;
-                    }
-                }
-                bm[nt] = v;
-            }
-#pragma unroll
-            for (int nt = 0; nt < 2; nt++) {
-                acc[nt] += d[nt] * c1[nt];
-                c1[nt] = f32x16{};
-            }
-            const half8 s_h = lh == 0 ? *(const half8*)&Sh[p][ar][0] : half8{};
-            const half8 s_l = lh == 0 ? *(const half8*)&Sl[p][ar][0] : half8{};
-#pragma unroll
-            for (int nt = 0; nt < 2; nt++) {
-                f32x16 c2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(s_h, bm[nt], f32x16{}, 0, 0, 0);
-                c2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(s_l, bm[nt], c2, 0, 0, 0);
-                acc[nt] -= dm[nt] * c2;
-            }
-        }
-    };
-    // three register stages with fixed roles (no dynamic indexing): at step t
-    // the stage holding tile t + 1 is built into LDS and tile t + 2 loads
-    // into the stage tile t - 1 used
-    GemmStage S0, S1, S2;
-    load_tile(S0, 0);
-    if (1 < ntiles) load_tile(S1, 1);
-    store_tile(S0, 0);
-    __syncthreads();
-    auto step = [&](GemmStage& Snext, GemmStage& Sfar, int t) {
-        if (t + 2 < ntiles) load_tile(Sfar, t + 2);
-        compute(t);
-        if (t + 1 < ntiles) store_tile(Snext, t + 1);  // the other buffer: every wave is past tile t - 1
-        __syncthreads();
-    };
-    for (int t = 0; t < ntiles; t += 3) {
-        step(S1, S2, t);
-        if (t + 1 < ntiles) step(S2, S0, t + 1);
-        if (t + 2 < ntiles) step(S0, S1, t + 2);
-    }
-    // store: D[i][j] in lane j + 32*((i/4)%2), register 4*(i/8) + i%4
-    gemm_store(
-        Y, ldy, M, N, rowscale, acc, [&](int, int r) { return m0 + 32 * wm + 8 * (r / 4) + 4 * lh + (r % 4); },
-        [&](int nt) { return n0 + 64 * wn + 32 * nt + li; }, accumulate);
-}
-
-
 // ------------------------------------------------ Q4_K B operand converted once
 //
 // launch_pack_q4k_gemm layout of a rows x cols Q4_K matrix (rows % 32 == 0,
-// cols % 256 == 0), read by gemm_q4k_b16_kernel:
+// cols % 256 == 0), read by gemm_rows_kernel<RF_Q4P>:
 //   B section: per 32-row tile nt and 64-value k-tile kt (Q4_K group g = kt %
 //   4 of super-block kt / 4: sub-block 2g from the low nibbles of its 32 code
 //   bytes, 2g + 1 from the high ones), per k-step s (values 16s .. 16s + 15
@@ -447,8 +264,8 @@ __global__ void __launch_bounds__(kGT) gemm_q4k_kernel(const uint8_t* __restrict
 //   H section (after the rows * cols * 2 bytes of B): per (nt, super-block
 //   sb), 640 bytes: the 32 rows' d | dmin << 16 (their header's first dword),
 //   then their 8 sub-block mins as fp16 (16 bytes a row).
-// The values are those gemm_q4k_kernel builds in LDS for every tile of
-// input rows; here they are built once and every k-step's B is one
+// The values are those gemm_rows_kernel<RF_Q4> forms in registers for every
+// tile of input rows; here they are built once and every k-step's B is one
 // contiguous 1 KB load.
 constexpr int kGemmHBytes = 640;
 
@@ -495,304 +312,542 @@ __global__ void __launch_bounds__(256) pack_q4k_gemm_kernel(const uint8_t* __res
     }
 }
 
-// gemm_q4k_kernel's tiles (64 input rows x 256 weight rows, 512 threads) on
-// the converted B: wave w takes weight rows 32 w .. 32 w + 31 of the tile for
-// all 64 input rows (two 32 x 32 MFMA tiles), its B operands loaded straight
-// into registers (one 1 KB load per k-step), only x (fp16 hi and lo) staged
-// in LDS. Four register stages in a ring, k-tile t + 3 loading while t
-// computes, unrolled by four so that the tiles that start a super-block
-// (and bring its header and sub-block sums) are known at compile time:
-// every load is unconditional (the last tiles re-read tile KT - 1), so the
-// compiler counts them exactly and waits only for the tile in hand. The
-// same MFMA chains in the same order as gemm_q4k_kernel: the same results,
-// bit for bit.
-struct GemmStageB {
-    u32x4 xh, xl, ps;  // x chunk of 8 values (input row tid/8, chunk tid%8); sub-block sums (super-block start)
-    u32x4 b[4];        // the wave's B operand of each k-step
-};
 
-__global__ void __launch_bounds__(kGT) gemm_q4k_b16_kernel(const uint8_t* __restrict__ Wg, int N, int K,
-                                                           const _Float16* __restrict__ xh,
-                                                           const _Float16* __restrict__ xl,
-                                                           const _Float16* __restrict__ sh,
-                                                           const _Float16* __restrict__ sl,
-                                                           const float* __restrict__ rowscale,
-                                                           float* __restrict__ Y, int M, int64_t ldy, int accumulate) {
-    __shared__ __attribute__((aligned(16))) _Float16 Xh[2][kTm][kXs];
-    __shared__ __attribute__((aligned(16))) _Float16 Xl[2][kTm][kXs];
-    __shared__ __attribute__((aligned(16))) _Float16 Sh[2][kTm][8];
-    __shared__ __attribute__((aligned(16))) _Float16 Sl[2][kTm][8];
-    const int n0 = blockIdx.x * kGN, m0 = blockIdx.y * kTm;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int li = lane & 31, lh = lane >> 5;
-    const int KT = K / kTk, NB = K / 256;  // KT: a multiple of 32 (K % 2048 == 0)
-    // this wave's 32-row tile (past N: the last one, loaded and not stored)
-    const bool live = n0 + 32 * wave < N;
-    const int nt = live ? (n0 >> 5) + wave : N / 32 - 1;
-    const uint8_t* Bw = Wg + (size_t)nt * KT * 4096 + 16 * lane;
-    const uint8_t* Hw = Wg + (size_t)N * K * 2 + (size_t)nt * NB * kGemmHBytes;
-    const int xr = tid >> 3, xc = tid & 7;
-    const int pr = (tid >> 1) & (kTm - 1);  // sub-block sums: row pr, hi (even) or lo (odd)
-    const _Float16* ps_src = ((tid & 1) ? sl : sh) + (size_t)(m0 + pr) * (K / 32);
+// ------------------------------------------------------------ the product
+// Weight formats of the row products: Q4_K in the operand layout of
+// launch_pack_q4k_gemm (below), or rows as the file holds them.
+enum RowsFmt : int { RF_Q4P, RF_Q4, RF_Q6, RF_Q8, RF_F16, RF_BF16 };
 
-    f32x16 acc[2], c1[2];
-#pragma unroll
-    for (int mt = 0; mt < 2; mt++) {
-        acc[mt] = f32x16{};
-        c1[mt] = f32x16{};
+// f(std::integral_constant<int, I>) for I = I0 .. N - 1, unrolled at compile
+// time (register arrays indexed by I stay in registers)
+template <int I0, int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (I0 < N) {
+        f(std::integral_constant<int, I0>{});
+        static_for<I0 + 1, N>(f);
     }
-    uint32_t hd = 0, hd_n = 0;  // the lane's row: d | dmin << 16 of the super-block computing, of the next
-    u32x4 hm = {}, hm_n = {};   // their 8 mins (fp16)
-    // SB: t starts a super-block (t % 4 == 0): its sub-block sums into the
-    // stage, its header into hd_n / hm_n
-    auto load = [&](GemmStageB& S, int t, auto SB) {
-        t = t < KT ? t : KT - 4 + (t & 3);  // (KT % 4 == 0: keeps t % 4)
-        const size_t o = (size_t)(m0 + xr) * K + t * kTk + 8 * xc;
-        S.xh = *(const u32x4*)(xh + o);
-        S.xl = *(const u32x4*)(xl + o);
-#pragma unroll
-        for (int s = 0; s < 4; s++) S.b[s] = *(const u32x4*)(Bw + ((size_t)t * 4 + s) * 1024);
-        if constexpr (decltype(SB)::value) {
-            S.ps = *(const u32x4*)(ps_src + 8 * (t >> 2));
-            const uint8_t* h = Hw + (size_t)(t >> 2) * kGemmHBytes;
-            hd_n = *(const uint32_t*)(h + 4 * li);
-            hm_n = *(const u32x4*)(h + 128 + 16 * li);
-        }
-    };
-    auto store_x = [&](const GemmStageB& S, int t) {
-        const int bf = t & 1;
-        *(u32x4*)&Xh[bf][xr][8 * xc] = S.xh;
-        *(u32x4*)&Xl[bf][xr][8 * xc] = S.xl;
-        if ((t & 3) == 0 && tid < 2 * kTm) {
-            const int p = (t >> 2) & 1;
-            if (tid & 1) *(u32x4*)&Sl[p][pr][0] = S.ps;
-            else *(u32x4*)&Sh[p][pr][0] = S.ps;
-        }
-    };
-    auto compute = [&](const GemmStageB& S, int t) {
-        const int bf = t & 1;
-#pragma unroll
-        for (int s = 0; s < 4; s++) {
-            const half8 bq = __builtin_bit_cast(half8, S.b[s]);
-            half8 a_h[2], a_l[2];
-#pragma unroll
-            for (int mt = 0; mt < 2; mt++) {
-                a_h[mt] = *(const half8*)&Xh[bf][32 * mt + li][16 * s + 8 * lh];
-                a_l[mt] = *(const half8*)&Xl[bf][32 * mt + li][16 * s + 8 * lh];
-            }
-#pragma unroll
-            for (int mt = 0; mt < 2; mt++) c1[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_h[mt], bq, c1[mt], 0, 0, 0);
-#pragma unroll
-            for (int mt = 0; mt < 2; mt++) c1[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_l[mt], bq, c1[mt], 0, 0, 0);
-        }
-        if ((t & 3) == 3) {
-            // end of super-block: acc += d * C, then the min term on the same MFMA shape
-            const int p = (t >> 2) & 1;
-            const float d = half_bits_to_f32(hd), dm = half_bits_to_f32(hd >> 16);
-            const half8 bm = lh == 0 ? __builtin_bit_cast(half8, hm) : half8{};
-#pragma unroll
-            for (int mt = 0; mt < 2; mt++) {
-                acc[mt] += d * c1[mt];
-                c1[mt] = f32x16{};
-            }
-#pragma unroll
-            for (int mt = 0; mt < 2; mt++) {
-                const half8 s_h = lh == 0 ? *(const half8*)&Sh[p][32 * mt + li][0] : half8{};
-                const half8 s_l = lh == 0 ? *(const half8*)&Sl[p][32 * mt + li][0] : half8{};
-                f32x16 c2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(s_h, bm, f32x16{}, 0, 0, 0);
-                c2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(s_l, bm, c2, 0, 0, 0);
-                acc[mt] -= dm * c2;
-            }
-        }
-    };
-    GemmStageB S0, S1, S2, S3;
-    load(S0, 0, std::true_type{});
-    hd = hd_n;
-    hm = hm_n;
-    load(S1, 1, std::false_type{});
-    load(S2, 2, std::false_type{});
-    store_x(S0, 0);
-    __syncthreads();
-    // step t: tile t computes from Sc (its x already in LDS), tile t + 1's x
-    // goes into the other LDS buffer from Sn, tile t + 3 loads into Sf (the
-    // stage tile t - 1 used); the step that loads a super-block's first tile
-    // (t % 4 == 1) brings its header, taken over after the last k-tile of
-    // the super-block before it
-    auto step = [&](const GemmStageB& Sc, const GemmStageB& Sn, GemmStageB& Sf, int t, auto SB) {
-        load(Sf, t + 3, SB);
-        compute(Sc, t);
-        if ((t & 3) == 3) {
-            hd = hd_n;
-            hm = hm_n;
-        }
-        if (t + 1 < KT) store_x(Sn, t + 1);
-        __syncthreads();
-    };
-    for (int t = 0; t < KT; t += 4) {
-        step(S0, S1, S3, t, std::false_type{});
-        step(S1, S2, S0, t + 1, std::true_type{});
-        step(S2, S3, S1, t + 2, std::false_type{});
-        step(S3, S0, S2, t + 3, std::false_type{});
-    }
-    if (!live) return;
-    // store: D[i][j] in lane j + 32*((i/4)%2), register 4*(i/8) + i%4
-    gemm_store(
-        Y, ldy, M, N, rowscale, acc, [&](int mt, int r) { return m0 + 32 * mt + 8 * (r / 4) + 4 * lh + (r % 4); },
-        [&](int) { return n0 + 32 * wave + li; }, accumulate);
 }
 
-
-// Q6_K (q6_k.rs:8-43: y = (d * sc) * q, q = code - 32, one int8 scale per
-// 16-value sub-block) on the same tiles as gemm_q4k_kernel. The B operand
-// is q itself, exact in fp16; sc * q (up to 4096 in magnitude) is not
-// always exact in fp16, so the scale is applied per sub-block instead: a
-// 32 x 32 x 16 product is exactly one sub-block, so each k-step's chain (x
-// hi, then x lo) starts from zero and is folded into the fp32 accumulator as
-// acc += (d * sc) * C, the factor per weight row (lane) and sub-block.
-// Blocks are 210 bytes (2-byte aligned): the code bytes of a k-tile pair
-// (ql low nibbles and qh bits 0-3, then the high nibbles and bits 4-7 of the
-// same bytes) are loaded once per pair with ld16_a2.
-struct GemmStage6 {
-    u32x4 xh, xl;             // x chunk of 8 values: input row tid/8, chunk tid%8
-    u32x4 ql0, ql1, qh, scw;  // weight row bn: ql / qh bytes of the k-tile pair; the 16 scales
-    uint32_t d;               // and d (first k-tile of a super-block)
+struct RowsSeg {
+    const uint8_t* W;  // weight rows (RF_Q4P: the operand copy)
+    float* y;
+    int n;             // rows
+    int t0;            // its first column tile of the launch
 };
 
-struct GemmBuf6 {
-    _Float16 Xh[kTm][kXs];
-    _Float16 Xl[kTm][kXs];
-    _Float16 Bq[kGN][kXs];  // q = code - 32 of the k-tile, weight-row major
+struct RowsArgs {
+    RowsSeg seg[3];
+    int nseg, ntiles, mtiles;  // column tiles (all segments), row tiles
+    int K, M;
+    const uint8_t* xa;         // gemm_prep_kernel's operands of the rows
+    const uint8_t* xs;
+    const float* rowscale;
+    int64_t ldy;
+    int accumulate;            // y += result
 };
 
-// four 6-bit codes (nibbles of ql at bit 4p, two qh bits at 4p + 2j) as
-// fp16 q = code - 32: 1024 + code has the bits 0x6400 | code
-__device__ __forceinline__ void q6_codes8(uint32_t l0, uint32_t l1, uint32_t h0, uint32_t h1, int p, int j,
-                                          _Float16* dst) {
-    const uint32_t sn = 4u * (uint32_t)p, sh = 4u * (uint32_t)p + 2u * (uint32_t)j;
-    const uint32_t c0 = ((l0 >> sn) & 0x0F0F0F0Fu) | (((h0 >> sh) & 0x03030303u) << 4);
-    const uint32_t c1 = ((l1 >> sn) & 0x0F0F0F0Fu) | (((h1 >> sh) & 0x03030303u) << 4);
-    const uint32_t p0 = __builtin_amdgcn_perm(0x64646464u, c0, 0x07010700u);
-    const uint32_t p1 = __builtin_amdgcn_perm(0x64646464u, c0, 0x07030702u);
-    const uint32_t p2 = __builtin_amdgcn_perm(0x64646464u, c1, 0x07010700u);
-    const uint32_t p3 = __builtin_amdgcn_perm(0x64646464u, c1, 0x07030702u);
-    const half2v off = {(_Float16)-1056.0f, (_Float16)-1056.0f};
-    const half2v h0v = __builtin_bit_cast(half2v, p0) + off, h1v = __builtin_bit_cast(half2v, p1) + off;
-    const half2v h2v = __builtin_bit_cast(half2v, p2) + off, h3v = __builtin_bit_cast(half2v, p3) + off;
-    *(half8*)dst = half8{h0v.x, h0v.y, h1v.x, h1v.y, h2v.x, h2v.y, h3v.x, h3v.y};
+// The 6-bit scale and min of sub-block j (compile time) from the 12 scale
+// bytes (header dwords y, z, w), get_scale_min_k4 of q4_k_m.rs:11-22.
+__device__ __forceinline__ uint32_t q4_scale(const u32x4& h, int j) {
+    const int sh = 8 * (j & 3);
+    return j < 4 ? (h.y >> sh) & 63u : ((h.w >> sh) & 0xFu) | (((h.y >> (sh + 6)) & 3u) << 4);
+}
+__device__ __forceinline__ uint32_t q4_min(const u32x4& h, int j) {
+    const int sh = 8 * (j & 3);
+    return j < 4 ? (h.z >> sh) & 63u : ((h.w >> (sh + 4)) & 0xFu) | (((h.z >> (sh + 6)) & 3u) << 4);
+}
+__device__ __forceinline__ _Float16 u2h(uint32_t v) { return (_Float16)(uint16_t)v; }
+
+// Eight bytes c (each 0 .. 255) as fp16 1024 + c: the bits 0x6400 | c.
+__device__ __forceinline__ void bytes_1024(uint32_t t0, uint32_t t1, half2v (&h)[4]) {
+    h[0] = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, t0, 0x07010700u));
+    h[1] = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, t0, 0x07030702u));
+    h[2] = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, t1, 0x07010700u));
+    h[3] = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, t1, 0x07030702u));
+}
+// c - off: the difference of two fp16 integers below 2048 is exact
+__device__ __forceinline__ void bytes_to_half(uint32_t t0, uint32_t t1, float off, half2v (&h)[4]) {
+    const half2v o = {(_Float16)(-1024.0f - off), (_Float16)(-1024.0f - off)};
+    bytes_1024(t0, t1, h);
+#pragma unroll
+    for (int e = 0; e < 4; e++) h[e] += o;
+}
+__device__ __forceinline__ u32x4 pack_half(const half2v (&h)[4]) {
+    return u32x4{__builtin_bit_cast(uint32_t, h[0]), __builtin_bit_cast(uint32_t, h[1]),
+                 __builtin_bit_cast(uint32_t, h[2]), __builtin_bit_cast(uint32_t, h[3])};
 }
 
-__global__ void __launch_bounds__(kGT) gemm_q6k_kernel(const uint8_t* __restrict__ W, int N, int K,
-                                                       const _Float16* __restrict__ xh,
-                                                       const _Float16* __restrict__ xl,
-                                                       const float* __restrict__ rowscale, float* __restrict__ Y,
-                                                       int M, int64_t ldy, int accumulate) {
-    __shared__ __attribute__((aligned(16))) GemmBuf6 buf[2];
-    // per super-block (by its parity): the 16 int8 scales and d of each
-    // weight row (rows 20 B apart, so the 32 rows a wave reads fall in
-    // distinct banks)
-    __shared__ __attribute__((aligned(16))) uint8_t Wh[2][kGN][20];
-    const int n0 = blockIdx.x * kGN, m0 = blockIdx.y * kTm;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave & 1, wn = wave >> 1;
-    const size_t rb = (size_t)(K / 256) * 210;
+// 16 bytes at byte v (per lane) + s (uniform) of a buffer: the address takes
+// one register for all the loads of a wave. Past the buffer's end: zeros.
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+__device__ __forceinline__ rsrc_t buffer_of(const uint8_t* p, size_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)bytes, 0x00027000);
+}
+__device__ __forceinline__ u32x4 buf16(rsrc_t r, int v, int s) {
+    return __builtin_amdgcn_raw_buffer_load_b128(r, v, s, 0);
+}
+
+template <bool BF>
+__device__ __forceinline__ f32x16 mfma16(const u32x4& a, const u32x4& b, const f32x16& c) {
+    if constexpr (BF)
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0, 0);
+}
+
+typedef uint32_t u32x4_a2g __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x2_a2g __attribute__((ext_vector_type(2), aligned(2)));
+
+template <int FMT, int WN, int KQ, int MT, bool MID>
+__global__ void __launch_bounds__(256, 1) gemm_rows_kernel(const RowsArgs a) {
+    static_assert(WN * KQ == 4 && (MT == 1 || MT == 2), "four waves");
+    static_assert(WN == 1 || FMT == RF_Q4P || FMT == RF_Q4 || FMT == RF_Q6, "wide groups take K-quants");
+    constexpr bool BF = FMT == RF_BF16, Q4 = FMT == RF_Q4P || FMT == RF_Q4;
+    constexpr int P = BF ? 3 : 2;
+    constexpr bool SH = WN > 1;            // the input planes of a k-tile shared through LDS
+    constexpr bool CONV = FMT == RF_Q4 || FMT == RF_Q6 || FMT == RF_Q8;  // weights become fp16 in registers
+    constexpr int AB = KQ * MT * 4 * P;    // their 1 KB blocks: [depth share][32 rows][k-step][plane]
+    constexpr int ABUF = SH ? 4 : 1;
+    constexpr int SMEM = SH ? ABUF * AB * kStepBytes : 16;
+    constexpr int RED = KQ > 1 ? 4 * MT * 2 * 16 * 64 * 4 : 16;
+    __shared__ __attribute__((aligned(16))) uint8_t smem[SMEM > RED ? SMEM : RED];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int li = lane & 31, lh = lane >> 5;
-    const int bn = 8 * (tid >> 4) + (tid & 7), bc = (tid >> 3) & 1;
-    const uint8_t* brow = W + (size_t)(n0 + bn < N ? n0 + bn : N - 1) * rb;
-    const int xr = tid >> 3, xc = tid & 7;
-
-    f32x16 acc[2];
-#pragma unroll
-    for (int nt = 0; nt < 2; nt++) acc[nt] = f32x16{};
-
-    const int ntiles = K / kTk;
-    auto load_tile = [&](GemmStage6& S, int t) {
-        const int k0 = t * kTk;
-        const size_t o = (size_t)(m0 + xr) * K + k0 + 8 * xc;
-        S.xh = *(const u32x4*)(xh + o);
-        S.xl = *(const u32x4*)(xl + o);
-        const int b = k0 / 256, g = (k0 % 256) / 64, h = g >> 1;
-        const uint8_t* blk = brow + (size_t)b * 210;
-        // branch-free: both k-tiles of a pair load the pair's bytes, every
-        // k-tile the block's scales and d (used at its first k-tile)
-        S.ql0 = ld16_a2(blk + 64 * h + 16 * bc);
-        S.ql1 = ld16_a2(blk + 64 * h + 32 + 16 * bc);
-        S.qh = ld16_a2(blk + 128 + 32 * h + 16 * bc);
-        S.scw = ld16_a2(blk + 192);
-        S.d = ld_u16(blk + 208);
-    };
-    auto store_tile = [&](const GemmStage6& S, int t) {
-        GemmBuf6& B = buf[t & 1];
-        *(u32x4*)&B.Xh[xr][8 * xc] = S.xh;
-        *(u32x4*)&B.Xl[xr][8 * xc] = S.xl;
-        const int g = t & 3, p = g & 1, sp = (t >> 2) & 1;
-        const u32x4 ql0 = S.ql0, ql1 = S.ql1, qh = S.qh;
-        if (g == 0 && bc == 0) {
-            uint32_t* w = (uint32_t*)&Wh[sp][bn][0];
-            w[0] = S.scw.x; w[1] = S.scw.y; w[2] = S.scw.z; w[3] = S.scw.w; w[4] = S.d;
-        }
-        // values 16 bc .. +15 of the tile's two 32-value quarters (codes of
-        // ql0 / ql1 with the qh bit pairs 2p, 2p + 1)
-        q6_codes8(ql0.x, ql0.y, qh.x, qh.y, p, 0, &B.Bq[bn][16 * bc]);
-        q6_codes8(ql0.z, ql0.w, qh.z, qh.w, p, 0, &B.Bq[bn][16 * bc + 8]);
-        q6_codes8(ql1.x, ql1.y, qh.x, qh.y, p, 1, &B.Bq[bn][32 + 16 * bc]);
-        q6_codes8(ql1.z, ql1.w, qh.z, qh.w, p, 1, &B.Bq[bn][32 + 16 * bc + 8]);
-    };
-
-    const int ar = 32 * wm + li;
-    auto compute = [&](int t) {
-        const GemmBuf6& B = buf[t & 1];
-        const int g = t & 3, sp = (t >> 2) & 1;
-        // d * sc of this lane's two weight rows for the tile's four sub-blocks
-        float ds[2][4];
-#pragma unroll
-        for (int nt = 0; nt < 2; nt++) {
-            const int r = 64 * wn + 32 * nt + li;
-            const uint32_t scs = *(const uint32_t*)&Wh[sp][r][4 * g];
-            const float d = half_bits_to_f32(*(const uint32_t*)&Wh[sp][r][16]);
-#pragma unroll
-            for (int s = 0; s < 4; s++) ds[nt][s] = d * (float)(int)(int8_t)(scs >> (8 * s));
-        }
-        // k-step s: sub-block 4g + s, its chain (x hi, then x lo) scaled into acc
-#pragma unroll
-        for (int s = 0; s < 4; s++) {
-            const half8 a_h = *(const half8*)&B.Xh[ar][16 * s + 8 * lh];
-            const half8 a_l = *(const half8*)&B.Xl[ar][16 * s + 8 * lh];
-            half8 bq[2];
-#pragma unroll
-            for (int nt = 0; nt < 2; nt++) bq[nt] = *(const half8*)&B.Bq[64 * wn + 32 * nt + li][16 * s + 8 * lh];
-            f32x16 c[2];
-#pragma unroll
-            for (int nt = 0; nt < 2; nt++) c[nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_h, bq[nt], f32x16{}, 0, 0, 0);
-#pragma unroll
-            for (int nt = 0; nt < 2; nt++) c[nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_l, bq[nt], c[nt], 0, 0, 0);
-#pragma unroll
-            for (int nt = 0; nt < 2; nt++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) acc[nt][r] = fmaf(ds[nt][s], c[nt][r], acc[nt][r]);
-        }
-    };
-    // two register stages (gemm_q4k_kernel's three would not fit the
-    // registers), each loaded two k-tiles ahead: at step t the stage holding
-    // tile t + 1 is built into LDS and then reloaded with tile t + 3
-    GemmStage6 S0, S1;
-    load_tile(S0, 0);
-    if (1 < ntiles) load_tile(S1, 1);
-    store_tile(S0, 0);
-    if (2 < ntiles) load_tile(S0, 2);
-    __syncthreads();
-    auto step = [&](GemmStage6& Snext, int t) {  // Snext holds tile t + 1
-        compute(t);
-        if (t + 1 < ntiles) store_tile(Snext, t + 1);  // the other buffer: every wave is past tile t - 1
-        if (t + 3 < ntiles) load_tile(Snext, t + 3);
-        __syncthreads();
-    };
-    for (int t = 0; t < ntiles; t += 2) {
-        step(S1, t);
-        if (t + 1 < ntiles) step(S0, t + 1);
+    const int wn = wave % WN, kq = wave / WN;
+    // tile: with a multiple of eight column tiles, the row tiles of a column
+    // tile follow each other on one XCD (workgroup id % 8), so its weights
+    // come into one L2
+    int tn, tm;
+    if ((a.ntiles & 7) == 0) {
+        const int slot = blockIdx.x >> 3;
+        tn = (slot / a.mtiles) * 8 + (blockIdx.x & 7);
+        tm = slot % a.mtiles;
+    } else {
+        tn = blockIdx.x % a.ntiles;
+        tm = blockIdx.x / a.ntiles;
     }
-    gemm_store(
-        Y, ldy, M, N, rowscale, acc, [&](int, int r) { return m0 + 32 * wm + 8 * (r / 4) + 4 * lh + (r % 4); },
-        [&](int nt) { return n0 + 64 * wn + 32 * nt + li; }, accumulate);
+    const int sg = a.nseg > 2 && tn >= a.seg[2].t0 ? 2 : a.nseg > 1 && tn >= a.seg[1].t0 ? 1 : 0;
+    const uint8_t* W = a.seg[sg].W;
+    const int N = a.seg[sg].n;
+    const int c0 = ((tn - a.seg[sg].t0) * WN + wn) * 64;  // the wave's first column (weight row)
+    const int K = a.K, KS = K / 16, NB = K / 256;
+    const int nsb = (NB - kq + KQ - 1) / KQ;  // the wave's super-blocks kq, kq + KQ, ...
+    const int nbt = SH ? (NB + KQ - 1) / KQ : nsb;
+
+    // the 64 (32) input rows: per 32 rows KS * P blocks
+    const int a_mt = KS * P * kStepBytes;
+    const rsrc_t Ar = buffer_of(a.xa + (size_t)(tm * MT) * a_mt, (size_t)MT * a_mt);
+    const rsrc_t Sr = buffer_of(Q4 ? a.xs + (size_t)(tm * MT) * NB * kStepBytes : a.xa, (size_t)MT * NB * kStepBytes);
+    const int l16 = 16 * lane;
+    const uint8_t* Bb[2];   // the lane's row
+    rsrc_t Br[2], Hr[2];    // RF_Q4P: the column tile's blocks, its headers
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        if constexpr (FMT == RF_Q4P) {
+            const int nt = min(c0 / 32 + j, N / 32 - 1);  // (past N: the last tile, computed and not stored)
+            Br[j] = buffer_of(W + (size_t)nt * KS * kStepBytes, (size_t)KS * kStepBytes);
+            Hr[j] = buffer_of(W + (size_t)N * K * 2 + (size_t)nt * NB * kGemmHBytes, (size_t)NB * kGemmHBytes);
+        } else {
+            const size_t rb = FMT == RF_Q4 ? (size_t)NB * 144 : FMT == RF_Q6 ? (size_t)NB * 210
+                              : FMT == RF_Q8 ? (size_t)(K / 32) * 34 : (size_t)K * 2;
+            Bb[j] = W + (size_t)min(c0 + 32 * j + li, N - 1) * rb;
+        }
+    }
+
+    // Register rings. B (and A when each wave reads its own): slot s holds
+    // k-step s of a unit of eight (128 values) and takes the next unit's
+    // k-step s once it is used. Shared A: k-tile t + 4 loads while t computes,
+    // t + 2 goes into LDS, the fragments are read a pair of k-steps ahead.
+    u32x4 A[SH ? 4 : 8][MT][P];     // own: by slot; shared: fragments, two pairs of k-steps
+    constexpr int SC = SH ? AB * kStepBytes / 4096 : 1;  // 16-byte chunks of a k-tile per thread
+    u32x4 st[2][SC];
+    u32x4 B[8][2];                  // operand blocks, F16 / BF16 values
+    u32x2 C8[8][2];                 // Q8_0: the k-step's eight quants
+    u32x2 Cq[2][2][FMT == RF_Q6 ? 6 : 4];  // Q4_K / Q6_K: code bytes of the unit (by its half)
+    uint32_t Dq[2][2][4];           // Q8_0: block scales of the unit
+    u32x4 hd[2], hdn[2];            // super-block headers: Q4_K header or mins, Q6_K scales; the next one's
+    uint32_t dd[2], ddn[2];         // d | dmin << 16 (RF_Q4P), d (Q6_K)
+    u32x4 sm[MT], smn[MT];          // Q4_K: sub-block sums
+    f32x16 acc[MT][2], mid[MT][2], c[MT][2];
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[i][j] = f32x16{};
+
+    // shared A: thread's chunks of k-tile g of the depth shares' super-blocks
+    // b (share q: super-block q + KQ b, past the end a re-read of the last)
+    auto stage_load = [&](int b, int g, u32x4 (&r)[SC]) {
+#pragma unroll
+        for (int k = 0; k < SC; k++) {
+            // a chunk's block row (share, 32 rows) is uniform over the workgroup:
+            // a k-tile of 32 rows is 4 P KB, P chunks of the 256 threads
+            const int q = k / (MT * P), i = (k / P) % MT;
+            const int sb = min(q + KQ * b, q + KQ * ((NB - q - 1) / KQ));
+            r[k] = buf16(Ar, 16 * (int)threadIdx.x, i * a_mt + (16 * sb + 4 * g) * (P * kStepBytes) + (k % P) * 4096);
+        }
+    };
+    auto stage_store = [&](const u32x4 (&r)[SC], int buf) {
+#pragma unroll
+        for (int k = 0; k < SC; k++) *(u32x4*)(smem + buf * (AB * kStepBytes) + k * 4096 + 16 * threadIdx.x) = r[k];
+    };
+    auto frag = [&](int buf, int s, int i, int p) {  // k-step s of the k-tile in buf
+        return *(const u32x4*)(smem + (buf * AB + ((kq * MT + i) * 4 + s) * P + p) * kStepBytes + 16 * lane);
+    };
+    auto load_step = [&](int ks, auto S) {  // k-step ks (its unit's slot S)
+        constexpr int s = decltype(S)::value;
+        if constexpr (!SH) {
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+#pragma unroll
+                for (int p = 0; p < P; p++)
+                    A[s][i][p] = buf16(Ar, l16, i * a_mt + (ks * P + p) * kStepBytes);
+        }
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            if constexpr (FMT == RF_Q4P) B[s][j] = buf16(Br[j], l16, ks * kStepBytes);
+            else if constexpr (FMT == RF_F16 || BF) B[s][j] = *(const u32x4_a2g*)(Bb[j] + (size_t)ks * 32 + 16 * lh);
+            else if constexpr (FMT == RF_Q8)
+                C8[s][j] = *(const u32x2_a2g*)(Bb[j] + (size_t)(ks >> 1) * 34 + 2 + 16 * (ks & 1) + 8 * lh);
+        }
+    };
+    // what a unit (half H of super-block sb) takes beside its k-steps
+    auto load_unit = [&](int sb, auto H) {
+        constexpr int h = decltype(H)::value;
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            if constexpr (FMT == RF_Q4) {
+                const uint8_t* q = Bb[j] + (size_t)sb * 144 + 16 + 64 * h + 8 * lh;
+#pragma unroll
+                for (int g = 0; g < 4; g++) Cq[h][j][g] = *(const u32x2_a2g*)(q + 16 * g);
+            } else if constexpr (FMT == RF_Q6) {
+                const uint8_t* q = Bb[j] + (size_t)sb * 210 + 8 * lh;
+#pragma unroll
+                for (int g = 0; g < 4; g++) Cq[h][j][g] = *(const u32x2_a2g*)(q + 64 * h + 16 * g);
+#pragma unroll
+                for (int g = 0; g < 2; g++) Cq[h][j][4 + g] = *(const u32x2_a2g*)(q + 128 + 32 * h + 16 * g);
+            } else if constexpr (FMT == RF_Q8) {
+#pragma unroll
+                for (int g = 0; g < 4; g++) Dq[h][j][g] = ld_u16(Bb[j] + (size_t)(8 * sb + 4 * h + g) * 34);
+            }
+        }
+    };
+    auto load_head = [&](int sb) {
+        if constexpr (FMT == RF_Q4P || FMT == RF_Q4 || FMT == RF_Q6) {
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                if constexpr (FMT == RF_Q4P) {
+                    ddn[j] = __builtin_amdgcn_raw_buffer_load_b32(Hr[j], 4 * li, sb * kGemmHBytes, 0);
+                    hdn[j] = buf16(Hr[j], 16 * li, sb * kGemmHBytes + 128);
+                } else if constexpr (FMT == RF_Q4) {
+                    hdn[j] = *(const u32x4_a2g*)(Bb[j] + (size_t)sb * 144);
+                } else {
+                    hdn[j] = *(const u32x4_a2g*)(Bb[j] + (size_t)sb * 210 + 192);
+                    ddn[j] = ld_u16(Bb[j] + (size_t)sb * 210 + 208);
+                }
+            }
+        }
+        if constexpr (Q4) {
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+                smn[i] = buf16(Sr, l16, (i * NB + sb) * kStepBytes);
+        }
+    };
+    auto take_head = [&]() {
+#pragma unroll
+        for (int j = 0; j < 2; j++) { hd[j] = hdn[j]; dd[j] = ddn[j]; }
+#pragma unroll
+        for (int i = 0; i < MT; i++) sm[i] = smn[i];
+    };
+    // the B operand of k-step S of half H, column tile j
+    auto operand = [&](auto H, auto S, int j, const u32x4& head) -> u32x4 {
+        constexpr int h = decltype(H)::value, s = decltype(S)::value;
+        if constexpr (FMT == RF_Q4) {
+            // group 2h + s / 4; sub-block 2 * group + (s / 2) % 2 (low or high nibbles)
+            constexpr int sub = 2 * (2 * h + s / 4) + ((s >> 1) & 1);
+            const u32x2 q = Cq[h][j][2 * (s / 4) + (s & 1)];
+            const uint32_t t0 = (s >> 1) & 1 ? (q.x >> 4) & 0x0F0F0F0Fu : q.x & 0x0F0F0F0Fu;
+            const uint32_t t1 = (s >> 1) & 1 ? (q.y >> 4) & 0x0F0F0F0Fu : q.y & 0x0F0F0F0Fu;
+            // sc * q = sc * (1024 + q) - 1024 sc in one exact fma (sc * q <= 945)
+            const _Float16 sc = u2h(q4_scale(head, sub));
+            const half2v s2 = {sc, sc}, o2 = s2 * half2v{(_Float16)-1024.0f, (_Float16)-1024.0f};
+            half2v v[4];
+            bytes_1024(t0, t1, v);
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = __builtin_elementwise_fma(v[e], s2, o2);
+            return pack_half(v);
+        } else if constexpr (FMT == RF_Q6) {
+            // quarter s / 2 of the half: ql bytes 32 (quarter % 2) + 16 (s % 2), nibble quarter / 2, qh bits 2 quarter
+            constexpr int qt = s >> 1;
+            const u32x2 l = Cq[h][j][2 * (qt & 1) + (s & 1)], u = Cq[h][j][4 + (s & 1)];
+            auto code = [&](uint32_t lo, uint32_t hi) {
+                const uint32_t n = qt >= 2 ? (lo >> 4) & 0x0F0F0F0Fu : lo & 0x0F0F0F0Fu;
+                const uint32_t b = qt == 0 ? hi << 4 : qt == 1 ? hi << 2 : qt == 2 ? hi : hi >> 2;
+                return n | (b & 0x30303030u);
+            };
+            half2v v[4];
+            bytes_to_half(code(l.x, u.x), code(l.y, u.y), 32.0f, v);
+            return pack_half(v);
+        } else if constexpr (FMT == RF_Q8) {
+            half2v v[4];
+            bytes_to_half(C8[s][j].x ^ 0x80808080u, C8[s][j].y ^ 0x80808080u, 128.0f, v);
+            return pack_half(v);
+        } else {
+            return B[s][j];
+        }
+    };
+
+    const int kql = min(kq, NB - 1);  // (a share without super-blocks loads the last one's)
+    if (nbt > 0) {
+        load_head(kql);
+        load_unit(kql, std::integral_constant<int, 0>{});
+        if constexpr (SH) {
+            u32x4 s0[SC], s1[SC];
+            stage_load(0, 0, s0);
+            stage_load(0, 1, s1);
+            stage_load(0, 2, st[0]);
+            stage_load(0, 3, st[1]);
+            static_for<0, 8>([&](auto S) { load_step(16 * kql + decltype(S)::value, S); });
+            stage_store(s0, 0);
+            stage_store(s1, 1);
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+#pragma unroll
+                    for (int p = 0; p < P; p++) A[u][i][p] = frag(0, u, i, p);
+        } else {
+            static_for<0, 8>([&](auto S) { load_step(16 * kql + decltype(S)::value, S); });
+        }
+        take_head();
+    }
+    u32x4 bq[2][2];  // the pair's B operands; CONV: formed a pair ahead, beside the products
+    if constexpr (CONV) {
+        if (nbt > 0)
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                bq[0][j] = operand(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, j, hd[j]);
+                bq[1][j] = operand(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{}, j, hd[j]);
+            }
+    }
+    for (int b = 0; b < nbt; b++) {
+        const bool live = b < nsb;  // (wave-uniform; a share may have one super-block fewer)
+        const int sb = live ? kq + KQ * b : kql, sbn = b + 1 < nsb ? sb + KQ : sb;  // (past the end: re-read)
+        static_for<0, 4>([&](auto G) {
+            constexpr int g = decltype(G)::value, h = g / 2;
+            using Hc = std::integral_constant<int, h>;
+            const int usb = h == 0 ? sb : sbn;  // the next unit: half 1 - h of super-block usb
+            if constexpr (g % 2 == 0) {
+                load_unit(usb, std::integral_constant<int, 1 - h>{});
+                if constexpr (h == 1) load_head(sbn);
+            }
+            if constexpr (SH) {
+                stage_store(st[g & 1], (g + 2) & 3);
+                stage_load(b + 1, g, st[g & 1]);
+            }
+            static_for<0, 2>([&](auto R) {
+                constexpr int pr = decltype(R)::value, s0 = 4 * (g & 1) + 2 * pr;  // slots s0, s0 + 1
+                using S0 = std::integral_constant<int, s0>;
+                using S1 = std::integral_constant<int, s0 + 1>;
+                constexpr int f0 = SH ? 2 * pr : s0;  // where the pair's A is
+                if constexpr (SH) {  // the next pair's fragments
+#pragma unroll
+                    for (int u = 0; u < 2; u++)
+#pragma unroll
+                        for (int i = 0; i < MT; i++)
+#pragma unroll
+                            for (int p = 0; p < P; p++)
+                                A[2 * (1 - pr) + u][i][p] = frag((g + pr) & 3, pr == 0 ? 2 + u : u, i, p);
+                }
+                u32x4 bn[2][2];
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    if constexpr (CONV) {
+                        // the next pair (of the next super-block after the last)
+                        constexpr int np = (2 * g + pr + 1) & 7;
+                        using Hn = std::integral_constant<int, np / 4>;
+                        const u32x4& head = np == 0 ? hdn[j] : hd[j];
+                        bn[0][j] = operand(Hn{}, std::integral_constant<int, 2 * (np & 3)>{}, j, head);
+                        bn[1][j] = operand(Hn{}, std::integral_constant<int, 2 * (np & 3) + 1>{}, j, head);
+                    } else {
+                        bq[0][j] = operand(Hc{}, S0{}, j, hd[j]);
+                        bq[1][j] = operand(Hc{}, S1{}, j, hd[j]);
+                    }
+                }
+                // Chains start from zero: every k-step for Q6_K (one
+                // sub-block), every pair for Q8_0 (one block), otherwise
+                // every k-tile, or every super-block without MID (Q4_K).
+                // Within a pair the small parts come first, so only the hi
+                // parts round at the chain's full size.
+#pragma unroll
+                for (int q = 0; q < 2 * P; q++) {
+                        // (Q8_0, whose chain is one pair: k-step by k-step,
+                        // hi then lo, measured closer to the 64-bit result)
+                        const int p = FMT == RF_Q8 ? q % P : P - 1 - q / 2, u = FMT == RF_Q8 ? q / P : q % 2;
+                        if (FMT == RF_Q6 && u == 1) continue;
+                        const bool first = q == 0 && (FMT == RF_Q6 || FMT == RF_Q8 || (pr == 0 && (MID || g == 0)));
+#pragma unroll
+                        for (int i = 0; i < MT; i++)
+#pragma unroll
+                            for (int j = 0; j < 2; j++)
+                                c[i][j] = mfma16<BF>(A[f0 + u][i][p], bq[u][j], first ? f32x16{} : c[i][j]);
+                }
+                f32x16 (&sum)[MT][2] = MID ? mid : acc;
+                auto fold = [&](int u) {  // sum (+)= f * c
+#pragma unroll
+                    for (int j = 0; j < 2; j++) {
+                        float f = 1.0f;
+                        if constexpr (FMT == RF_Q6) {
+                            const uint32_t w = g == 0 ? hd[j].x : g == 1 ? hd[j].y : g == 2 ? hd[j].z : hd[j].w;
+                            f = half_bits_to_f32(dd[j]) * sbyte_f32(w, 2 * pr + u);
+                        } else if constexpr (FMT == RF_Q8) {
+                            f = half_bits_to_f32(Dq[h][j][s0 >> 1]);
+                        }
+                        const bool start = MID && g == 0 && u == 0 && (pr == 0 || !(FMT == RF_Q6 || FMT == RF_Q8));
+#pragma unroll
+                        for (int i = 0; i < MT; i++) {
+                            if constexpr (FMT == RF_Q6 || FMT == RF_Q8) {
+                                if (start) sum[i][j] = f * c[i][j];
+                                else
+#pragma unroll
+                                    for (int r = 0; r < 16; r++) sum[i][j][r] = fmaf(f, c[i][j][r], sum[i][j][r]);
+                            } else {
+                                if (start) sum[i][j] = c[i][j];
+                                else sum[i][j] += c[i][j];
+                            }
+                        }
+                    }
+                };
+                if constexpr (FMT == RF_Q6) {
+                    fold(0);
+#pragma unroll
+                    for (int p = P - 1; p >= 0; p--)
+#pragma unroll
+                        for (int i = 0; i < MT; i++)
+#pragma unroll
+                            for (int j = 0; j < 2; j++)
+                                c[i][j] = mfma16<BF>(A[f0 + 1][i][p], bq[1][j], p == P - 1 ? f32x16{} : c[i][j]);
+                    fold(1);
+                } else if constexpr (FMT == RF_Q8) {
+                    fold(0);
+                } else if constexpr (MID && pr == 1) {
+                    fold(0);
+                }
+                load_step(16 * usb + 8 * (1 - h) + s0, S0{});
+                load_step(16 * usb + 8 * (1 - h) + s0 + 1, S1{});
+                if constexpr (CONV)
+#pragma unroll
+                    for (int j = 0; j < 2; j++) { bq[0][j] = bn[0][j]; bq[1][j] = bn[1][j]; }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            if constexpr (SH) __syncthreads();
+        });
+        if (live) {
+            if constexpr (Q4) {
+                // end of the super-block: acc += d * sums, then the min term
+                // dmin * sum_sub m_sub * X_sub as one product over K = 16: the
+                // eight hi sums in the lower lane half, the lo sums in the upper
+                // one, the mins in both
+                u32x4 bm[2];
+                float d[2], dm[2];
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    if constexpr (FMT == RF_Q4P) {
+                        bm[j] = hd[j];
+                        d[j] = half_bits_to_f32(dd[j]);
+                        dm[j] = half_bits_to_f32(dd[j] >> 16);
+                    } else {
+                        half2v v[4];
+#pragma unroll
+                        for (int e = 0; e < 4; e++) v[e] = half2v{u2h(q4_min(hd[j], 2 * e)), u2h(q4_min(hd[j], 2 * e + 1))};
+                        bm[j] = pack_half(v);
+                        d[j] = half_bits_to_f32(hd[j].x);
+                        dm[j] = half_bits_to_f32(hd[j].x >> 16);
+                    }
+                    dm[j] *= 32.0f;  // exact: the sums are times 2^-5
+                }
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+#pragma unroll
+                    for (int j = 0; j < 2; j++) {
+                        const f32x16 c2 = mfma16<false>(sm[i], bm[j], f32x16{});
+#pragma unroll
+                        for (int r = 0; r < 16; r++) {
+                            const float cs = MID ? mid[i][j][r] : c[i][j][r];
+                            acc[i][j][r] = fmaf(-dm[j], c2[r], fmaf(d[j], cs, acc[i][j][r]));
+                        }
+                    }
+            } else if constexpr (MID) {
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+#pragma unroll
+                    for (int j = 0; j < 2; j++) acc[i][j] += mid[i][j];
+            }
+        }
+        take_head();
+    }
+
+    // the KQ partial sums of the tile, added in a fixed order: wave kq takes
+    // register groups [G0, G0 + 4 / KQ) of four rows
+    constexpr int NG = 4 / KQ;
+    const int g0 = kq * NG;
+    float* red = (float*)smem;  // [wave][32 rows, column tile, register][lane]
+    constexpr int RW = MT * 2 * 16 * 64;
+    if constexpr (KQ > 1) {
+        if constexpr (SH) __syncthreads();  // (the last k-tile's fragments are read)
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) red[wave * RW + ((i * 2 + j) * 16 + r) * 64 + lane] = acc[i][j][r];
+        __syncthreads();
+    }
+    // D[i][j] in lane j + 32 * ((i / 4) % 2), register 4 * (i / 8) + i % 4.
+    // Every row scale and (with accumulate) every old value is loaded before
+    // the first store: a store could alias a later load as far as the
+    // compiler knows, which would make each element wait for its own trip.
+    float* y = a.seg[sg].y;
+    float v[MT][2][NG][4], old[MT][2][NG][4];
+    f32x4 rs[MT][NG];
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int g = 0; g < NG; g++) {
+            const int m = 32 * (tm * MT + i) + 8 * (g0 + g) + 4 * lh;
+            rs[i][g] = *(const f32x4*)(a.rowscale + m);
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const int n = c0 + 32 * j + li;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    old[i][j][g][e] = a.accumulate && m + e < a.M && n < N ? y[(m + e) * a.ldy + n] : 0.f;
+                    if constexpr (KQ == 1) {
+                        v[i][j][g][e] = acc[i][j][4 * g + e];
+                    } else {
+                        const int q = ((i * 2 + j) * 16 + 4 * (g0 + g) + e) * 64 + lane;
+                        if constexpr (KQ == 2) v[i][j][g][e] = red[wn * RW + q] + red[(wn + WN) * RW + q];
+                        else v[i][j][g][e] = (red[q] + red[RW + q]) + (red[2 * RW + q] + red[3 * RW + q]);
+                    }
+                }
+            }
+        }
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int n = c0 + 32 * j + li;
+#pragma unroll
+            for (int g = 0; g < NG; g++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int m = 32 * (tm * MT + i) + 8 * (g0 + g) + 4 * lh + e;
+                    if (m < a.M && n < N) {
+                        const float r = v[i][j][g][e] * rs[i][g][e];
+                        y[m * a.ldy + n] = a.accumulate ? old[i][j][g][e] + r : r;  // one writer per output
+                    }
+                }
+        }
 }
 
 }  // namespace
@@ -832,19 +887,88 @@ static GemmWorkspace& gemm_workspace(int dev) {
     return *all[dev];
 }
 
+// 0: the GEMVs, one input or a few at a time; 1: the matrix cores; 2: the
+// matrix cores where a workspace can be had. K-quants with K a multiple of
+// 2048 from 16 rows on: below, the batched GEMVs read each weight row once
+// for up to eight inputs. Other depths and Q8_0, F16 and BF16 rows have one
+// GEMV launch per input, so the product pays from a few inputs on.
+static int rows_route(int32_t t, const GemvArgs& a) {
+    const bool kq = t == MIVI_GGML_Q4_K || t == MIVI_GGML_Q6_K;
+    const bool fmt = kq || t == MIVI_GGML_Q8_0 || t == MIVI_GGML_F16 || t == MIVI_GGML_BF16;
+    if (!fmt || a.K <= 0 || a.K % 256 || a.ncol > INT32_MAX - 64) return 0;
+    if (kq && a.K % 2048 == 0) {
+        auto a16 = [](const void* p) { return p == nullptr || (uintptr_t)p % 16 == 0; };
+        const bool aligned = a16(a.x) && a16(a.x2) && a16(a.norm_w) && a.xs % 4 == 0;
+        return a.ncol >= kMfmaMinBatch && aligned ? 1 : 0;
+    }
+    // From 1024 columns, the narrowest of the loader's configurations: models
+    // narrower than that (test sizes) keep the GEMVs, whose chunked prefill
+    // then equals the token path bit for bit, as the tests over Q8_0 caches
+    // expect. The GEMVs stage one input row in LDS: longer ones than 12288 are
+    // refused there.
+    return a.K >= 1024 && a.ncol >= (t == MIVI_GGML_Q8_0 ? kMfmaMinBatchQ8 : kMfmaMinBatchRows) && a.K <= 12288 ? 2 : 0;
+}
+
+// Workgroup shape of a product: WN column groups of 64 by KQ shares of the
+// depth, WN * KQ = 4 waves. Wider groups read the inputs fewer times; more
+// depth shares make more workgroups where the outputs alone would leave CUs
+// idle. Picks the least rounds(workgroups / CUs) * (fixed + super-blocks per
+// wave).
+struct RowsTile {
+    int wn, ntiles;
+};
+static RowsTile rows_tile(int32_t t, const GemvArgs& a, int mtiles) {
+    RowsTile best = {4, 0};
+    double least = 0;
+    static const int env_wn = env_knob("MIVI_ROWS_WN", 0);
+    const int wide = (t == MIVI_GGML_Q4_K || t == MIVI_GGML_Q6_K) && a.K % 2048 == 0 ? 4 : 1;
+    for (int wn = wide; wn >= 1; wn /= 2) {
+        if (env_wn && wn != env_wn && wide > 1) continue;
+        int nt = 0;
+        for (int i = 0; i < a.nseg; i++) nt += (a.seg[i].n + 64 * wn - 1) / (64 * wn);
+        const int kq = 4 / wn, nsb = (a.K / 256 + kq - 1) / kq;
+        const double rounds = (double)(((size_t)nt * mtiles + num_cus() - 1) / num_cus());
+        const double cost = rounds * (3.0 + nsb * (wn == 4 ? 1.7 : wn == 2 ? 1.9 : 2.2));
+        if (best.ntiles == 0 || cost < least) {
+            least = cost;
+            best = {wn, nt};
+        }
+    }
+    return best;
+}
+
+template <int FMT>
+static void launch_rows_kernel(const RowsArgs& r, int wn, int mt, hipStream_t s) {
+    const dim3 grid((unsigned)(r.ntiles * r.mtiles));
+#define LR(WN, MT, MID) hipLaunchKernelGGL((gemm_rows_kernel<FMT, WN, 4 / WN, MT, MID>), grid, dim3(256), 0, s, r)
+    if constexpr (FMT == RF_Q4P || FMT == RF_Q4 || FMT == RF_Q6) {
+        if (wn == 4) { if (mt == 1) LR(4, 1, false); else LR(4, 2, false); return; }
+        if (wn == 2) { if (mt == 1) LR(2, 1, false); else LR(2, 2, false); return; }
+        if (r.K % 2048 == 0) { if (mt == 1) LR(1, 1, false); else LR(1, 2, false); return; }
+    }
+    if (mt == 1) LR(1, 1, true); else LR(1, 2, true);
+#undef LR
+}
+
+// Most bytes of input planes one launch takes: longer batches run in slabs of
+// rows, so that the workspace stays bounded.
+constexpr size_t kRowsSlabBytes = 256u << 20;
+
 // Y_s[m * ys + n] (=|+=) sum_k W_s[n, k] * pro(X)[m, k] for the segments s
-// of a (Q4_K or Q6_K, K % 2048 == 0): one activation split, one GEMM per
-// segment.
+// of a (K % 256 == 0): one activation split, one product over all segments.
+// MIVI_ERR_UNSUPPORTED when the workspace cannot be had.
 static int32_t rows_mfma(int32_t t, int pro, const GemvArgs& a, hipStream_t s) {
-    const size_t batch = (size_t)a.ncol;
-    if (batch > (size_t)INT32_MAX - kTm) return err_overflow();
-    const size_t mp = (batch + kTm - 1) / kTm * kTm, K = (size_t)a.K;
-    const size_t bx = mp * K * 2, bs = mp * (K / 32) * 2, bytes = 2 * bx + 2 * bs + mp * 4 + 256;
+    const size_t K = (size_t)a.K, P = t == MIVI_GGML_BF16 ? 3 : 2;
+    const bool q4 = t == MIVI_GGML_Q4_K;
+    const size_t row_bytes = K * 2 * P + (q4 ? K / 8 : 0) + 4;
+    const size_t slab = std::max<size_t>(64, kRowsSlabBytes / row_bytes / 64 * 64);
+    const size_t mp0 = (std::min((size_t)a.ncol, slab) + 63) / 64 * 64;
+    const size_t bx = mp0 * K * 2 * P, bs = q4 ? mp0 * K / 8 : 0, bytes = bx + bs + mp0 * 4;
     int dev = 0;
     MIVI_HIP_CHECK(hipGetDevice(&dev));
     GemmWorkspace& ws = gemm_workspace(dev);
     std::lock_guard<std::mutex> lk(ws.mu);
-    if (!ws.done) MIVI_HIP_CHECK(hipEventCreateWithFlags(&ws.done, hipEventDisableTiming));
+    if (!ws.done) MIVI_HIP_CHECK(hipEventCreateWithFlags(&ws.done, hipEventDisableTiming | hipEventDisableSystemFence));
     else MIVI_HIP_CHECK(hipStreamWaitEvent(s, ws.done, 0));  // the previous user is done with it
     if (ws.bytes < bytes) {
         if (ws.ptr) {
@@ -853,32 +977,55 @@ static int32_t rows_mfma(int32_t t, int pro, const GemvArgs& a, hipStream_t s) {
             ws.ptr = nullptr;
             ws.bytes = 0;
         }
-        MIVI_HIP_CHECK(hipMalloc(&ws.ptr, bytes));
+        if (hipMalloc(&ws.ptr, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            ws.ptr = nullptr;
+            return set_error(MIVI_ERR_UNSUPPORTED, "no workspace of %zu bytes for the row products", bytes);
+        }
         ws.bytes = bytes;
     }
-    uint8_t* p = (uint8_t*)ws.ptr;
-    _Float16* xh = (_Float16*)p;
-    _Float16* xl = (_Float16*)(p + bx);
-    _Float16* sh = (_Float16*)(p + 2 * bx);
-    _Float16* sl = (_Float16*)(p + 2 * bx + bs);
-    float* rs = (float*)(p + 2 * bx + 2 * bs);
-    auto prep = K == 2048 ? gemm_prep_kernel<1> : K == 4096 ? gemm_prep_kernel<2> : K == 8192 ? gemm_prep_kernel<4>
-                                                                                             : gemm_prep_kernel<0>;
-    hipLaunchKernelGGL(prep, dim3((unsigned)mp), dim3(256), 0, s, a.x, a.x2, a.norm_w, a.eps, pro, a.xs,
-                       (int)batch, (int)K, xh, xl, sh, sl, rs);
-    for (int i = 0; i < a.nseg; i++) {
-        const int rows = a.seg[i].n;
-        if (rows == 0) continue;
-        dim3 grid((unsigned)((rows + kGN - 1) / kGN), (unsigned)(mp / kTm));
-        if (t == MIVI_GGML_Q6_K)
-            hipLaunchKernelGGL(gemm_q6k_kernel, grid, dim3(kGT), 0, s, a.seg[i].W, rows, (int)K, xh, xl, rs,
-                               a.seg[i].y, (int)batch, a.ys, a.accumulate);
-        else if (a.seg[i].wg && rows % 32 == 0)
-            hipLaunchKernelGGL(gemm_q4k_b16_kernel, grid, dim3(kGT), 0, s, a.seg[i].wg, rows, (int)K, xh, xl, sh, sl,
-                               rs, a.seg[i].y, (int)batch, a.ys, a.accumulate);
-        else
-            hipLaunchKernelGGL(gemm_q4k_kernel, grid, dim3(kGT), 0, s, a.seg[i].W, rows, (int)K, xh, xl, sh, sl, rs,
-                               a.seg[i].y, (int)batch, a.ys, a.accumulate);
+    auto a16 = [](const void* p) { return p == nullptr || (uintptr_t)p % 16 == 0; };
+    const int vec = a16(a.x) && a16(a.x2) && a16(a.norm_w) && a.xs % 4 == 0;
+    bool packed = q4;
+    for (int i = 0; i < a.nseg; i++) packed = packed && a.seg[i].wg && a.seg[i].n % 32 == 0;
+    for (size_t m0 = 0; m0 < (size_t)a.ncol; m0 += slab) {
+        const int M = (int)std::min(slab, (size_t)a.ncol - m0);
+        const int mt = M <= 32 ? 1 : 2, mtiles = (M + 32 * mt - 1) / (32 * mt);
+        RowsArgs r = {};
+        r.xa = (const uint8_t*)ws.ptr;
+        r.xs = q4 ? r.xa + bx : nullptr;
+        float* rs = (float*)((uint8_t*)ws.ptr + bx + bs);
+        r.rowscale = rs;
+        r.K = (int)K;
+        r.M = M;
+        r.mtiles = mtiles;
+        r.ldy = a.ys;
+        r.accumulate = a.accumulate;
+#define LP(R, PL)                                                                                                    \
+    hipLaunchKernelGGL((gemm_prep_kernel<R, PL>), dim3((unsigned)(mtiles * 32 * mt / kPrepRows)), dim3(512), 0, s, a.x + m0 * a.xs, \
+                       a.x2 ? a.x2 + m0 * a.xs : nullptr, a.norm_w, a.eps, pro, a.xs, M, (int)K, vec,                \
+                       (uint8_t*)ws.ptr, (uint8_t*)r.xs, rs)
+#define LPR(PL)                                                                                                      \
+    if (K <= 2048) LP(4, PL); else if (K <= 4096) LP(8, PL); else if (K <= 8192) LP(16, PL); \
+    else LP(0, PL)
+        if (P == 3) { LPR(3); } else { LPR(2); }
+#undef LPR
+#undef LP
+        const RowsTile tile = rows_tile(t, a, mtiles);
+        int t0 = 0;
+        for (int i = 0; i < a.nseg; i++) {
+            if (a.seg[i].n == 0) continue;  // (no tiles: left out of the table)
+            r.seg[r.nseg++] = {packed ? a.seg[i].wg : a.seg[i].W, a.seg[i].y + m0 * a.ys, a.seg[i].n, t0};
+            t0 += (a.seg[i].n + 64 * tile.wn - 1) / (64 * tile.wn);
+        }
+        r.ntiles = t0;
+        if (t0 == 0) break;
+        if (t == MIVI_GGML_Q6_K) launch_rows_kernel<RF_Q6>(r, tile.wn, mt, s);
+        else if (t == MIVI_GGML_Q8_0) launch_rows_kernel<RF_Q8>(r, tile.wn, mt, s);
+        else if (t == MIVI_GGML_F16) launch_rows_kernel<RF_F16>(r, tile.wn, mt, s);
+        else if (t == MIVI_GGML_BF16) launch_rows_kernel<RF_BF16>(r, tile.wn, mt, s);
+        else if (packed) launch_rows_kernel<RF_Q4P>(r, tile.wn, mt, s);
+        else launch_rows_kernel<RF_Q4>(r, tile.wn, mt, s);
     }
     MIVI_HIP_CHECK(hipGetLastError());
     MIVI_HIP_CHECK(hipEventRecord(ws.done, s));
@@ -900,11 +1047,20 @@ int32_t launch_pack_q4k_gemm(const uint8_t* src, uint8_t* dst, size_t rows, size
 int32_t launch_rows(int32_t t, int pro, const GemvArgs& a, hipStream_t s) {
     if (pro == PRO_CONV || a.epilogue != EPI_STORE)
         return set_error(MIVI_ERR_UNSUPPORTED, "row products take no conv prologue or fused epilogue");
-    // the activation split reads 16-byte vectors of every row
-    auto a16 = [](const void* p) { return p == nullptr || (uintptr_t)p % 16 == 0; };
-    const bool aligned = a16(a.x) && a16(a.x2) && a16(a.norm_w) && a.xs % 4 == 0;
-    if ((t == MIVI_GGML_Q4_K || t == MIVI_GGML_Q6_K) && a.ncol >= kMfmaMinBatch && a.K % 2048 == 0 && aligned)
-        return rows_mfma(t, pro, a, s);
+    const int route = rows_route(t, a);
+    if (route == 1) return rows_mfma(t, pro, a, s);
+    if (route == 2) {
+        // shapes whose GEMVs need no workspace: those still run them where
+        // none can be had (a capturing stream, no memory)
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
+            const int32_t rc = rows_mfma(t, pro, a, s);
+            if (rc != MIVI_ERR_UNSUPPORTED) return rc;
+            clear_error();
+        } else {
+            (void)hipGetLastError();
+        }
+    }
     return launch_gemv_ex(t, pro, a, s);
 }
 }  // namespace mivi
@@ -952,7 +1108,7 @@ extern "C" int32_t mivi_hip_quantized_matmul_rows_gemm_packed(float* out, size_t
     if (batch == 0 || rows == 0) return clear_error();
     if (!out || !w || !wg || !in) return set_error(MIVI_ERR_INVALID_ARGUMENT, "null buffer");
     if ((uintptr_t)wg % 16) return set_error(MIVI_ERR_INVALID_ARGUMENT, "packed copy must be 16-byte aligned");
-    if (rows > (size_t)INT32_MAX || cols > (size_t)INT32_MAX || batch > (size_t)INT32_MAX - kTm) return err_overflow();
+    if (rows > (size_t)INT32_MAX || cols > (size_t)INT32_MAX || batch > (size_t)INT32_MAX - 64) return err_overflow();
     clear_error();
     // batch >= kMfmaMinBatch: the matrix cores on the packed copy; fewer
     // rows: the GEMVs on the GGUF rows
@@ -980,7 +1136,7 @@ extern "C" int32_t mivi_hip_quantized_matmul_rows(float* out, size_t out_len, in
     if (!out || !w || !in) return set_error(MIVI_ERR_INVALID_ARGUMENT, "null buffer");
     clear_error();
     hipStream_t s = (hipStream_t)stream;
-    if (rows > (size_t)INT32_MAX || cols > (size_t)INT32_MAX || batch > (size_t)INT32_MAX - kTm) return err_overflow();
+    if (rows > (size_t)INT32_MAX || cols > (size_t)INT32_MAX || batch > (size_t)INT32_MAX - 64) return err_overflow();
     // Q4_K / Q6_K with batch >= kMfmaMinBatch and cols % 2048 == 0: the matrix cores;
     // otherwise one GEMV over the batch's input rows as columns: the streaming
     // kernel reads each weight row once per two inputs, with every input's

@@ -564,3 +564,96 @@ def test_packed_rejects_other_types_and_shapes(hip, torch_mod):
     with pytest.raises(hip.QuantError):
         hip.quantized_matmul_rows_packed(out, Q6_K, w6, x, 1, 4, 1024)
     assert hip.last_error().code == 116
+
+
+def _rows_case(hip, t, batch, rows, cols):
+    if t in (F16, BF16):
+        W = np.random.default_rng(7 * cols + rows).standard_normal((rows, cols)) * 0.02
+        W[0] *= 1e-5  # fp16 denormals: products must not flush them
+        w = dense_bytes(t, W)
+    else:
+        w = hip.synth_random_weights(t, 200 + cols + rows, rows, cols, 0.02)
+    X = hip.synth_normal(201 + batch, batch * cols).reshape(batch, cols).astype(np.float32)
+    X[0] *= np.float32(1e30)
+    X[1] = 0.0
+    X[2] *= np.float32(1e-30)
+    X[3, cols // 2] = np.float32(3e4)  # one dominant value
+    return w, X
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q6_K, Q8_0, F16, BF16])
+@pytest.mark.parametrize("batch,rows,cols", [(6, 1, 1024), (6, 63, 1280), (31, 65, 1024), (33, 200, 1792), (64, 129, 1536),
+                                             (65, 257, 4608), (8, 64, 10240), (97, 300, 2304), (32, 64, 12288)])
+def test_matmul_rows_matrix_cores_any_depth(hip, oracle, torch_mod, t, batch, rows, cols):
+    # the row products at depths with one GEMV launch per input (from 4 or 6
+    # inputs on): every weight format, tile edges in both directions, shares
+    # of the depth without a super-block, inputs from 1e-30 to 1e30; each
+    # output within a tenth of the bar of the f64 product of the stored
+    # weights (f32 sums and a 24-bit split of the inputs)
+    torch = torch_mod
+    w, X = _rows_case(hip, t, batch, rows, cols)
+    out = torch.full((batch * rows + 1,), 123.0, dtype=torch.float32, device="cuda")
+    hip.quantized_matmul_rows(out[:batch * rows], t, dev(torch, w), dev(torch, X.reshape(-1)), batch, rows, cols)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    assert got[-1] == 123.0
+    rc, deq, _ = oracle.dequantize_slice(t, w, rows * cols)
+    W = deq.reshape(rows, cols).astype(np.float64)
+    ref = X.astype(np.float64) @ W.T
+    bound = 1e-5 * np.linalg.norm(X.astype(np.float64), axis=1)[:, None] * np.linalg.norm(W, axis=1)[None, :]
+    err = np.abs(got[:-1].reshape(batch, rows).astype(np.float64) - ref)
+    assert np.all(err <= bound + 1e-44), float((err / np.maximum(bound, 1e-44)).max())
+
+
+@pytest.mark.parametrize("t", [Q8_0, F16, BF16])
+def test_matmul_rows_matrix_cores_infinite_inputs(hip, torch_mod, t):
+    # an infinite input gives the infinities and NaNs of its own matvec
+    torch = torch_mod
+    batch, rows, cols = 7, 70, 1280
+    w, X = _rows_case(hip, t, batch, rows, cols)
+    X[4, 17] = np.inf
+    X[5, 30], X[5, 31] = np.inf, -np.inf
+    X[6, 3] = np.nan
+    dw, dX = dev(torch, w), dev(torch, X)
+    out = torch.empty(batch, rows, dtype=torch.float32, device="cuda")
+    hip.quantized_matmul_rows(out, t, dw, dX, batch, rows, cols)
+    for b in range(4, 7):
+        one = torch.empty(rows, dtype=torch.float32, device="cuda")
+        hip.quantized_matvec(one, t, dw, dX[b].contiguous(), rows, cols)
+        torch.cuda.synchronize()
+        a, r = out[b].cpu().numpy(), one.cpu().numpy()
+        assert np.array_equal(np.isnan(a), np.isnan(r)) and not np.isfinite(a).any()
+        assert np.array_equal(a[~np.isnan(a)], r[~np.isnan(r)])
+
+
+def test_matmul_rows_any_depth_unaligned_and_captured(hip, torch_mod):
+    # inputs off a 16-byte boundary take the matrix cores too; under capture
+    # (no workspace there) the GEMVs run, replay for replay equal to the matvecs
+    torch = torch_mod
+    batch, rows, cols = 9, 130, 1024
+    w, X = _rows_case(hip, Q4_K, batch, rows, cols)
+    dw = dev(torch, w)
+    flat = torch.empty(batch * cols + 1, dtype=torch.float32, device="cuda")
+    dX = flat[1:]
+    dX.copy_(torch.from_numpy(X.reshape(-1)))
+    a = torch.empty(batch * rows, dtype=torch.float32, device="cuda")
+    b = torch.empty_like(a)
+    hip.quantized_matmul_rows(a, Q4_K, dw, dX, batch, rows, cols)
+    aligned = dX.clone()
+    hip.quantized_matmul_rows(b, Q4_K, dw, aligned, batch, rows, cols)
+    torch.cuda.synchronize()
+    assert torch.equal(a, b)
+    ones = torch.empty_like(a)
+    for i in range(batch):
+        hip.quantized_matvec(ones[i * rows:(i + 1) * rows], Q4_K, dw, aligned[i * cols:(i + 1) * cols], rows, cols)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        hip.quantized_matmul_rows(b, Q4_K, dw, aligned, batch, rows, cols)
+    for _ in range(3):
+        b.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(b, ones)
+        hip.quantized_matmul_rows(a, Q4_K, dw, aligned, batch, rows, cols)
+        torch.cuda.synchronize()
