@@ -1220,6 +1220,435 @@ __global__ void __launch_bounds__(64, 2) attn_f16_mfma_kernel(AttnArgs a) {
     }
 }
 
+// ------------------------------------------------ attention of a prefill tile
+//
+// Rows r0 .. of a tile (positions pos0 + r, their K/V already in the cache)
+// against the cache, head_dim 64, at most four query heads per kv head. A
+// workgroup's four waves take 32 rows of one query head each (the kv head's
+// heads, and 4 / hpk blocks of rows), sharing the kv head's K and V, staged in
+// LDS 64 tokens at a time, so a cache line is read once per workgroup instead
+// of once per row: 399 -> 27 us a launch at 512 rows and up to 2500 tokens.
+// v_mfma_f32_32x32x16 throughout, with the tokens as the rows of the scores:
+//  scores  S^T = K Q^T: lane = query, register = token, so the softmax of a
+//          query is a lane's own registers and one half swap;
+//  values  O^T = V^T P^T: the scores' registers are the B operand as they
+//          stand (the product's depth may be in any order while both operands
+//          agree: slot (half h, e) is token 8 (e / 4) + 4 h + e % 4 of 16), V
+//          transposed on its way out of LDS (ds_read_b64_tr_b16).
+// Precision: F16 caches: the query as fp16 hi + lo under a power-of-two scale
+// of its own, p as fp16 hi + lo, K and V as stored. Q8_0: K's and V's quants
+// are exact 16-bit integers; the scores' two blocks are scaled in f32, and p *
+// (V's block scale), whose range fp16 does not cover, enters as three bf16
+// parts. F32: every operand as three bf16 parts, the products up to 2^-24.
+// The softmax reference moves only when a maximum exceeds it by 2^8.
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+
+constexpr int kPfRows = 32;    // rows of a wave
+constexpr int kPfTokens = 64;  // tokens of an LDS tile
+constexpr int kPfVRow = 160;   // bytes of a V row in LDS: eight rows of 64 bytes cover every bank twice
+
+inline bool attn_prefill_ok(const mivi_model_info& c, bool packed) {
+    return c.head_dim == 64 && c.n_kv_heads > 0 && c.n_heads % c.n_kv_heads == 0 && c.n_heads / c.n_kv_heads <= 4 &&
+           (c.kv_precision != MIVI_KV_Q8_0 || packed);
+}
+// rows of a workgroup
+inline int attn_prefill_rows(int hpk) { return kPfRows * std::max(1, 4 / hpk); }
+
+// v into hi + mid + lo (an infinite v keeps its hi part only)
+__device__ __forceinline__ void split_bf16(float v, __bf16& b0, __bf16& b1, __bf16& b2) {
+    b0 = (__bf16)v;
+    const float r = fabsf((float)b0) <= 3.40282347e38f ? v - (float)b0 : 0.f;
+    b1 = (__bf16)r;
+    b2 = (__bf16)(r - (float)b1);
+}
+
+template <bool BF>
+__device__ __forceinline__ f32x16_t mfma32(const u32x4& a, const u32x4& b, const f32x16_t& c) {
+    if constexpr (BF)
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b), c, 0, 0, 0);
+}
+
+template <int KVP>
+__global__ void __launch_bounds__(256, 1) attn_prefill_kernel(AttnArgs a, int pos0, int rows, int nrb, int tsplit,
+                                                              float* out, int64_t out_s) {
+    constexpr bool F32C = KVP == MIVI_KV_F32, Q8 = KVP == MIVI_KV_Q8_0;
+    constexpr int KP = F32C ? 3 : 1;              // planes of K and of V in LDS
+    constexpr int QP = F32C ? 3 : 2;              // planes of the query
+    constexpr int PP = KVP == MIVI_KV_F16 ? 2 : 3;  // planes of p
+    constexpr bool SB = F32C, PB = KVP != MIVI_KV_F16;  // bf16 operands of the scores, of the values
+    constexpr int KB = kPfTokens * 128, VB = kPfTokens * kPfVRow;
+    constexpr int SCB = Q8 ? 2 * 2 * kPfTokens * 4 : 0;  // K's and V's block scales
+    constexpr int BUF = KP * (KB + VB) + SCB;
+    __shared__ __attribute__((aligned(16))) uint8_t smem[2 * BUF > 4 * kPfRows * 272 ? 2 * BUF : 4 * kPfRows * 272];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int li = lane & 31, lh = lane >> 5;
+    const int hpk = a.n_heads / a.n_kv_heads, nblk = max(1, 4 / hpk);
+    // workgroup -> kv head (id % n_kv: with eight of them one per XCD, whose L2
+    // then holds that head's K and V), split, row block (the longest first)
+    const int kvh = blockIdx.x % a.n_kv_heads, rest = blockIdx.x / a.n_kv_heads;
+    const int split = rest % a.nsplit, rb = nrb - 1 - rest / a.nsplit;
+    const int blk = wave / hpk;
+    const bool used = blk < nblk;  // (three heads: the fourth wave only loads)
+    const int head = kvh * hpk + wave % hpk;
+    const int row0 = (rb * nblk + (used ? blk : 0)) * kPfRows;  // the wave's first row
+    const int row = min(row0 + li, rows - 1);                    // the lane's query (past the end: not stored)
+    const int pos = pos0 + row;
+    // the workgroup's tokens: [t0, t1) of the split, no further than its last row
+    const int wg_last = min(rows, (rb + 1) * nblk * kPfRows) - 1;
+    const int t0 = split * tsplit, t1 = min(t0 + tsplit, pos0 + wg_last + 1);
+    const int tlast = pos0 + rows - 1;  // the cache holds tokens up to here
+
+    // K and V of a tile: global -> registers (a tile ahead) -> LDS
+    constexpr int LC = F32C ? 4 : KVP == MIVI_KV_F16 ? 2 : 1;
+    u32x4 rk[LC], rv[LC];
+    uint32_t rdk = 0, rdv = 0;
+    auto load_tile = [&](int t) {
+        if constexpr (Q8) {
+            const int g = min(t / 16 + (int)(threadIdx.x >> 6), tlast / 16);
+            const size_t o = ((size_t)g * a.n_kv_heads + kvh) * kQ8GroupBytes;
+            rk[0] = *(const u32x4*)(a.kc + o + 16 * lane);
+            rv[0] = *(const u32x4*)(a.vc + o + 16 * lane);
+            if (lane < 16) {
+                const bool in = 16 * g + lane <= tlast;
+                rdk = in ? *(const uint32_t*)(a.kc + o + q8g_d_off(lane, 0)) : 0u;
+                rdv = in ? *(const uint32_t*)(a.vc + o + q8g_d_off(lane, 0)) : 0u;
+            }
+        } else {
+            constexpr int EB = F32C ? 4 : 2, CPR = 64 * EB / 16;  // 16-byte chunks of a head's row
+#pragma unroll
+            for (int k = 0; k < LC; k++) {
+                const int ch = threadIdx.x + 256 * k, tok = min(t + ch / CPR, tlast);
+                const size_t o = (size_t)tok * a.row_bytes + (size_t)kvh * (64 * EB) + 16 * (ch % CPR);
+                rk[k] = *(const u32x4*)(a.kc + o);
+                rv[k] = *(const u32x4*)(a.vc + o);
+            }
+        }
+    };
+    // K row of a token: its 16-byte chunk c at c ^ (token % 8)
+    auto koff = [](int tok, int c) { return tok * 128 + ((c ^ (tok & 7)) * 16); };
+    auto store_tile = [&](uint8_t* b) {
+        uint8_t* kb = b;
+        uint8_t* vb = b + KP * KB;
+        if constexpr (KVP == MIVI_KV_F16) {
+#pragma unroll
+            for (int k = 0; k < LC; k++) {
+                const int ch = threadIdx.x + 256 * k, tok = ch / 8, c = ch % 8;
+                *(u32x4*)(kb + koff(tok, c)) = rk[k];
+                *(u32x4*)(vb + tok * kPfVRow + 16 * c) = rv[k];
+            }
+        } else if constexpr (Q8) {
+            // lane t + 16 c of group g: K quants 8c .. 8c+7 of both blocks, V dims 16c .. 16c+15 of token t
+            const int tok = 16 * (threadIdx.x >> 6) + (lane & 15), c = lane >> 4;
+            const uint32_t kw[4] = {rk[0].x, rk[0].y, rk[0].z, rk[0].w}, vw[4] = {rv[0].x, rv[0].y, rv[0].z, rv[0].w};
+            half8_t k0, k1;
+            bf16x8_t v0, v1;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                k0[e] = (_Float16)(short)(int8_t)(kw[e >> 2] >> (8 * (e & 3)));
+                k1[e] = (_Float16)(short)(int8_t)(kw[2 + (e >> 2)] >> (8 * (e & 3)));
+                v0[e] = (__bf16)sbyte_f32(vw[e >> 2], e & 3);
+                v1[e] = (__bf16)sbyte_f32(vw[2 + (e >> 2)], e & 3);
+            }
+            *(half8_t*)(kb + koff(tok, c)) = k0;
+            *(half8_t*)(kb + koff(tok, 4 + c)) = k1;
+            *(bf16x8_t*)(vb + tok * kPfVRow + 32 * c) = v0;
+            *(bf16x8_t*)(vb + tok * kPfVRow + 32 * c + 16) = v1;
+            if (lane < 16) {
+                float* sc = (float*)(vb + KP * VB);  // [K, V][block][token]
+                const int st = 16 * (threadIdx.x >> 6) + lane;
+                sc[st] = half_bits_to_f32(rdk);
+                sc[kPfTokens + st] = half_bits_to_f32(rdk >> 16);
+                sc[2 * kPfTokens + st] = half_bits_to_f32(rdv);
+                sc[3 * kPfTokens + st] = half_bits_to_f32(rdv >> 16);
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < LC; k++) {
+                const int ch = threadIdx.x + 256 * k, tok = ch / 16, c = ch % 16;  // dims 4c .. 4c+3
+                bf16x4_t kp[3], vp[3];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    __bf16 b0, b1, b2;
+                    split_bf16(__uint_as_float(rk[k][e]), b0, b1, b2);
+                    kp[0][e] = b0; kp[1][e] = b1; kp[2][e] = b2;
+                    split_bf16(__uint_as_float(rv[k][e]), b0, b1, b2);
+                    vp[0][e] = b0; vp[1][e] = b1; vp[2][e] = b2;
+                }
+#pragma unroll
+                for (int p = 0; p < 3; p++) {
+                    *(bf16x4_t*)(kb + p * KB + koff(tok, c / 2) + 8 * (c & 1)) = kp[p];
+                    *(bf16x4_t*)(vb + p * VB + tok * kPfVRow + 8 * c) = vp[p];
+                }
+            }
+        }
+    };
+    if (t0 < t1) load_tile(t0);
+
+    // the lane's query: dims 16 s + 8 lh .. + 7 of each k-step s, per-head
+    // RMSNorm (transformer.rs:81-96) and RoPE (rope.rs:452-473) as
+    // wave_prep_head, in log2 units, as the planes of the B operand
+    u32x4 qa[4][QP];
+    float qinv = 1.0f;
+    {
+        const float* qp = a.q + (int64_t)row * a.qkv_s + (size_t)head * 64;
+        const float* cs = a.rope_cos + (size_t)pos * 32;
+        const float* sn = a.rope_sin + (size_t)pos * 32;
+        float v[4][8];
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[s][e] = qp[16 * s + 8 * lh + e];
+        if (a.q_norm) {
+            float ss = 0.f;
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) ss = fmaf(v[s][e], v[s][e], ss);
+            float lo, hi;
+            swap32(ss, lo, hi);
+            const float sc = 1.0f / sqrtf((lo + hi) / 64.0f + a.eps);
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) v[s][e] = v[s][e] * sc * a.q_norm[16 * s + 8 * lh + e];
+        }
+        const float qscale = a.scale * 1.4426950408889634f;
+        float mx = 0.f;
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) {
+                const int i = 8 * s + 4 * lh + e / 2;
+                const float c = cs[i], n = sn[i], x0 = v[s][e], x1 = v[s][e + 1];
+                v[s][e] = (x0 * c - x1 * n) * qscale;
+                v[s][e + 1] = (x0 * n + x1 * c) * qscale;
+                mx = fmaxf(mx, fmaxf(fabsf(v[s][e]), fabsf(v[s][e + 1])));
+            }
+        if constexpr (!SB) {
+            // the largest value into [2^9, 2^10): lo parts clear of denormals,
+            // the sums of 64 products with fp16 keys within f32
+            float lo, hi;
+            swap32(mx, lo, hi);
+            mx = fmaxf(lo, hi);
+            int e = 0;
+            if (mx > 0.f && mx <= 3.40282347e38f) frexpf(mx, &e);
+            e = max(e - 10, -100);
+            const float f = ldexpf(1.0f, -e);
+            qinv = ldexpf(1.0f, e);
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                half8_t h, l;
+#pragma unroll
+                for (int k = 0; k < 8; k++) {
+                    const float y = v[s][k] * f;
+                    h[k] = (_Float16)y;
+                    l[k] = (_Float16)(y - (float)h[k]);
+                }
+                qa[s][0] = __builtin_bit_cast(u32x4, h);
+                qa[s][1] = __builtin_bit_cast(u32x4, l);
+            }
+        } else {
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                bf16x8_t b[3];
+#pragma unroll
+                for (int k = 0; k < 8; k++) {
+                    __bf16 b0, b1, b2;
+                    split_bf16(v[s][k], b0, b1, b2);
+                    b[0][k] = b0; b[1][k] = b1; b[2][k] = b2;
+                }
+#pragma unroll
+                for (int p = 0; p < 3; p++) qa[s][p] = __builtin_bit_cast(u32x4, b[p]);
+            }
+        }
+    }
+
+    float m_run = -INFINITY, l_run = 0.f;  // of the lane's query (l over the lane half's tokens)
+    f32x16_t o[2];                          // dims 32 d + 8 (r / 4) + 4 lh + r % 4 of the query
+    o[0] = f32x16_t{};
+    o[1] = f32x16_t{};
+    int buf = 0;
+    for (int t = t0; t < t1; t += kPfTokens) {
+        uint8_t* b = smem + buf * BUF;
+        store_tile(b);
+        if (t + kPfTokens < t1) load_tile(t + kPfTokens);
+        __syncthreads();  // (the buffer's readers of two tiles ago are past the last one)
+        buf ^= 1;
+        // rows below the tile have nothing in it (wave-uniform)
+        if (!used || t > pos0 + min(row0 + kPfRows, rows) - 1) continue;
+        const uint8_t* kb = b;
+        const uint8_t* vb = b + KP * KB;
+        const float* scl = (const float*)(vb + KP * VB);
+        // 1. scores of 2 x 32 tokens: register 16 u + r is token 32 u + 8 (r / 4) + 4 lh + r % 4
+        float s[32];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            f32x16_t c[Q8 ? 2 : 1];
+#pragma unroll
+            for (int k = 0; k < (Q8 ? 2 : 1); k++) c[k] = f32x16_t{};
+#pragma unroll
+            for (int st = 0; st < 4; st++) {
+                f32x16_t& cc = c[Q8 ? st / 2 : 0];
+#pragma unroll
+                for (int kp = KP - 1; kp >= 0; kp--) {
+                    const u32x4 kf = *(const u32x4*)(kb + kp * KB + koff(32 * u + li, 2 * st + lh));
+#pragma unroll
+                    for (int q = QP - 1; q >= 0; q--)
+                        if (KP == 1 || q + kp <= 2) cc = mfma32<SB>(kf, qa[st][q], cc);
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                if constexpr (Q8) {
+                    const int tk = 32 * u + 8 * (r / 4) + 4 * lh + r % 4;
+                    s[16 * u + r] = fmaf(scl[kPfTokens + tk], c[1][r], scl[tk] * c[0][r]);
+                } else {
+                    s[16 * u + r] = c[0][r];
+                }
+            }
+        }
+        // 2. mask (tiles on the diagonal), softmax
+        float mx = -INFINITY;
+        if (t + kPfTokens - 1 > pos0 + row0) {  // wave-uniform
+#pragma unroll
+            for (int k = 0; k < 32; k++) {
+                const int tk = t + 32 * (k / 16) + 8 * ((k % 16) / 4) + 4 * lh + k % 4;
+                s[k] = tk <= pos ? s[k] * qinv : -INFINITY;
+                mx = fmaxf(mx, s[k]);
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < 32; k++) {
+                s[k] *= qinv;
+                mx = fmaxf(mx, s[k]);
+            }
+        }
+        {
+            float lo, hi;
+            swap32(mx, lo, hi);
+            mx = fmaxf(lo, hi);
+        }
+        if (__builtin_amdgcn_ballot_w64(mx > m_run + 8.0f)) {
+            const float m_new = fmaxf(m_run, mx);
+            const float al = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_run - m_new);
+            m_run = m_new;
+            l_run *= al;
+            o[0] *= al;
+            o[1] *= al;
+        }
+        const float mr = m_run == -INFINITY ? 0.f : m_run;  // (a split may hold none of a row's tokens)
+#pragma unroll
+        for (int k = 0; k < 32; k++) {
+            s[k] = __builtin_amdgcn_exp2f(s[k] - mr);
+            l_run += s[k];
+        }
+        // 3. O^T += V^T P^T, 16 tokens at a time
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) {
+#pragma unroll
+            for (int d = 0; d < 2; d++) {
+                u32x4 pb[PP];
+                if constexpr (PB) {
+                    bf16x8_t x[3];
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        float w = s[8 * ks + e];
+                        if constexpr (Q8) w *= scl[(2 + d) * kPfTokens + 16 * ks + 8 * (e / 4) + 4 * lh + e % 4];
+                        __bf16 b0, b1, b2;
+                        split_bf16(w, b0, b1, b2);
+                        x[0][e] = b0; x[1][e] = b1; x[2][e] = b2;
+                    }
+#pragma unroll
+                    for (int p = 0; p < 3; p++) pb[p] = __builtin_bit_cast(u32x4, x[p]);
+                } else {
+                    half8_t h, l;
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        h[e] = (_Float16)s[8 * ks + e];
+                        l[e] = (_Float16)(s[8 * ks + e] - (float)h[e]);
+                    }
+                    pb[0] = __builtin_bit_cast(u32x4, h);
+                    pb[1] = __builtin_bit_cast(u32x4, l);
+                }
+#pragma unroll
+                for (int vp = KP - 1; vp >= 0; vp--) {
+                    // ds_read_b64_tr_b16: in each 16-lane group, lane 4 r + q
+                    // addresses four halves of token r and lane i receives dim
+                    // i of the four tokens (the fp16 decode kernel's read)
+                    typedef short s16x4 __attribute__((ext_vector_type(4)));
+                    const uint8_t* vr = vb + vp * VB + (16 * ks + 4 * lh + ((lane & 15) >> 2)) * kPfVRow +
+                                        2 * (32 * d + 16 * ((lane >> 4) & 1) + 4 * (lane & 3));
+                    const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)vr);
+                    const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                        (__attribute__((address_space(3))) s16x4*)(vr + 8 * kPfVRow));
+                    const u32x2 w0 = __builtin_bit_cast(u32x2, v0), w1 = __builtin_bit_cast(u32x2, v1);
+                    const u32x4 va = {w0.x, w0.y, w1.x, w1.y};
+#pragma unroll
+                    for (int p = PP - 1; p >= 0; p--)
+                        if (KP == 1 || p + vp <= 2) o[d] = mfma32<PB>(va, pb[p], o[d]);
+                }
+            }
+        }
+    }
+    // both halves' l; the wave's rows through LDS into whole lines
+    {
+        float lo, hi;
+        swap32(l_run, lo, hi);
+        l_run = lo + hi;
+    }
+    __syncthreads();
+    constexpr int OR = 68;  // floats of a row in LDS
+    float* ot = (float*)smem + wave * kPfRows * OR;
+    const bool whole = a.nsplit == 1;
+    const float f = whole ? (l_run > 0.f ? 1.0f / l_run : 0.f) : 1.0f;
+#pragma unroll
+    for (int d = 0; d < 2; d++)
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+            *(f32x4*)(ot + li * OR + 32 * d + 8 * g + 4 * lh) =
+                f32x4{o[d][4 * g] * f, o[d][4 * g + 1] * f, o[d][4 * g + 2] * f, o[d][4 * g + 3] * f};
+    __syncthreads();
+    if (!used) return;
+    const int r4 = lane >> 4, c4 = lane & 15;  // four rows of 16 chunks a pass
+#pragma unroll
+    for (int k = 0; k < kPfRows / 4; k++) {
+        const int r = 4 * k + r4;
+        if (row0 + r >= rows) continue;
+        const f32x4 v = *(const f32x4*)(ot + r * OR + 4 * c4);
+        if (whole) *(f32x4*)(out + (int64_t)(row0 + r) * out_s + (size_t)head * 64 + 4 * c4) = v;
+        else *(f32x4*)(a.part_acc + ((int64_t)(row0 + r) * a.part_s + (size_t)head * a.nsplit + split) * 64 + 4 * c4) = v;
+    }
+    if (!whole && lh == 0 && row0 + li < rows) {
+        const int64_t pi = (int64_t)(row0 + li) * a.part_s + (size_t)head * a.nsplit + split;
+        a.part_m[pi] = m_run;
+        a.part_l[pi] = l_run;
+    }
+}
+
+// Merges the splits of attn_prefill_kernel (m in log2 units; -inf where a
+// split holds none of the row's tokens): one wave per (head, row), lane = dim.
+__global__ void __launch_bounds__(64) attn_prefill_merge_kernel(const float* part_m, const float* part_l,
+                                                                const float* part_acc, float* out, int nsplit,
+                                                                int64_t part_s, int64_t out_s) {
+    const int h = blockIdx.x, lane = threadIdx.x;
+    const int64_t p0 = (int64_t)blockIdx.y * part_s + (int64_t)h * nsplit;
+    float M = -INFINITY;
+    for (int s = 0; s < nsplit; s++) M = fmaxf(M, part_m[p0 + s]);
+    float L = 0.f, v = 0.f;
+    for (int s = 0; s < nsplit; s++) {
+        const float m = part_m[p0 + s];
+        const float w = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - M);
+        L = fmaf(part_l[p0 + s], w, L);
+        v = fmaf(part_acc[(p0 + s) * 64 + lane], w, v);
+    }
+    out[(int64_t)blockIdx.y * out_s + h * 64 + lane] = L > 0.f ? v * (1.0f / L) : 0.f;
+}
+
 // Prefill tile: K/V of tile row blockIdx.x (position pos0 + row, k/v at
 // a.k/a.v + row * qkv_s) for kv head blockIdx.y into the cache, as the decode
 // step stores its current token. One wave per (row, kv head).
@@ -1925,6 +2354,32 @@ int32_t enqueue_batch_step(mivi_model* m, size_t batch, hipStream_t s) {
 }
 
 constexpr int kPrefillSplits = 16;  // attention splits per tile row, at most
+// Shorter tiles keep the per-row kernels of the decode: under 64 rows a row
+// reads little that another does not (and tests hold short tiles over Q8_0
+// caches to the token path's own bits).
+constexpr size_t kPfMinRows = 64;
+
+// Attention of a prefill tile's rows: splits of the cached tokens where the
+// row blocks alone would leave CUs idle (two workgroups per CU), at least 512
+// tokens each.
+void enqueue_attn_prefill(const mivi_model_info& c, AttnArgs a, int pos0, int rows, float* out, int64_t out_s,
+                          hipStream_t s) {
+    const int hpk = (int)(c.n_heads / c.n_kv_heads), wr = attn_prefill_rows(hpk);
+    const int nrb = (rows + wr - 1) / wr, total = pos0 + rows;
+    const int wgs = nrb * (int)c.n_kv_heads;
+    a.nsplit = std::max(1, std::min({kPrefillSplits, (2 * num_cus() + wgs - 1) / wgs, total / 512}));
+    const int tsplit = ((total + a.nsplit - 1) / a.nsplit + kPfTokens - 1) / kPfTokens * kPfTokens;
+    a.part_s = (int64_t)c.n_heads * a.nsplit;
+    const dim3 grid((unsigned)(wgs * a.nsplit));
+#define APF(KVP) hipLaunchKernelGGL((attn_prefill_kernel<KVP>), grid, dim3(256), 0, s, a, pos0, rows, nrb, tsplit, out, out_s)
+    if (c.kv_precision == MIVI_KV_F32) APF(MIVI_KV_F32);
+    else if (c.kv_precision == MIVI_KV_F16) APF(MIVI_KV_F16);
+    else APF(MIVI_KV_Q8_0);
+#undef APF
+    if (a.nsplit > 1)
+        hipLaunchKernelGGL(attn_prefill_merge_kernel, dim3((unsigned)c.n_heads, (unsigned)rows), dim3(64), 0, s, a.part_m,
+                           a.part_l, a.part_acc, out, a.nsplit, a.part_s, out_s);
+}
 
 // Tile buffers for `rows` rows (grow-only).
 int32_t prefill_buffers(mivi_model* m, size_t rows) {
@@ -2012,14 +2467,18 @@ int32_t enqueue_prefill_tile(mivi_model* m, size_t b, size_t p0, size_t rows, hi
             else KVS(MIVI_KV_Q8_0);
 #undef KVS
             // 2. attention of every row over the cache up to its position
-            const size_t tt = (size_t)attn_tile_tokens(c.head_dim);
-            const int nsplit = (int)std::max<size_t>(1, std::min<size_t>(kPrefillSplits, (p0 + rows + 8 * tt - 1) / (8 * tt)));
-            a.pos = m->pf_pos;
-            a.nsplit = nsplit;
-            a.part_m = m->pf_pm; a.part_l = m->pf_pl; a.part_acc = m->pf_pa;
-            a.part_s = (int64_t)c.n_heads * nsplit;
             a.keep_cache = 1;
-            enqueue_attention(c, a, (unsigned)R, m->pf_ao, (int64_t)D, s);
+            a.part_m = m->pf_pm; a.part_l = m->pf_pl; a.part_acc = m->pf_pa;
+            if (rows >= kPfMinRows && attn_prefill_ok(c, m->kv_packed)) {
+                enqueue_attn_prefill(c, a, (int)p0, R, m->pf_ao, (int64_t)D, s);
+            } else {
+                const size_t tt = (size_t)attn_tile_tokens(c.head_dim);
+                const int nsplit = (int)std::max<size_t>(1, std::min<size_t>(kPrefillSplits, (p0 + rows + 8 * tt - 1) / (8 * tt)));
+                a.pos = m->pf_pos;
+                a.nsplit = nsplit;
+                a.part_s = (int64_t)c.n_heads * nsplit;
+                enqueue_attention(c, a, (unsigned)R, m->pf_ao, (int64_t)D, s);
+            }
             g = {};
             g.seg[0] = {L.wo.w, m->pf_x, D, L.wo.gemm};
             g.nseg = 1; g.K = D; g.x = m->pf_ao; g.accumulate = 1;

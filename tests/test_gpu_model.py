@@ -599,3 +599,36 @@ def test_qk_norm_full_width_matches_oracle(hip, oracle, prec, oprec):
         else:
             lo = lo_own
         assert rel_err(m.forward(tok, n), lo) <= 1e-3, tile
+
+
+@pytest.mark.parametrize("n_heads,n_kv", [(12, 3), (12, 4), (12, 6), (12, 12)])
+@pytest.mark.parametrize("prec", [0, 2, 1])
+def test_prefill_tile_attention_matches_per_row_attention(hip, n_heads, n_kv, prec):
+    # tiles of 64 rows and more take the attention of a prefill tile (one to
+    # four query heads per kv head, ragged row blocks, splits of the cached
+    # tokens, later tiles over earlier ones), tiles of 32 the per-row kernels;
+    # every other product of this width is the same GEMV in both, so the
+    # caches and logits differ by the attention's f32 rounding alone (Q8_0
+    # caches: and by values on the edge of a code, the 1e-3 bar)
+    from mivi_hip.synthmodel import build_hybrid
+    img = build_hybrid(dim=768, hidden=768, n_layers=4, attn_layers=(0, 2, 3), n_heads=n_heads, n_kv=n_kv, vocab=512,
+                       ctx_len=2048, seed=31, qk_norm=n_kv == 4)
+    prompt = np.random.default_rng(32).integers(0, 512, 1334)
+    n = len(prompt) - 1
+    got = []
+    for tile in (32, 1100):
+        m = hip.Model(img, max_ctx=2048, kv_precision=prec)
+        m.set_prefill_strategy(tile)
+        m.prefill(prompt[:70], 0)
+        m.prefill(prompt[70:n], 70)
+        k, v, conv = m.export_state(n)
+        got.append((m.forward(int(prompt[-1]), n), k, v, conv))
+    (la, ka, va, ca), (lb, kb, vb, cb) = got
+    assert rel_err(lb, la) <= (1e-3 if prec == 1 else 2e-5)
+    if prec != 1:
+        dt = np.float32 if prec == 0 else np.float16
+        step = 2e-5 if prec == 0 else 1e-3  # one fp16 step
+        for x, y in ((ka, kb), (va, vb)):
+            x, y = x.view(dt).astype(np.float64), y.view(dt).astype(np.float64)
+            assert np.max(np.abs(x - y)) <= step * np.max(np.abs(x))
+        assert np.max(np.abs(ca - cb)) <= 1e-4 * np.max(np.abs(ca))
