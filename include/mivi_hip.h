@@ -103,8 +103,11 @@ int32_t mivi_hip_try_matvec_bf16(float* out, size_t out_len, const uint8_t* weig
 
 /* crates/mivi-quant/src/lib.rs:143-251 quantized_matmul_rows:
  * out[batch, rows] = inputs[batch, cols] * W[rows, cols]^T. batch == 1 is the
- * matvec path (lib.rs:173-182); Q4_K with batch >= 16 and cols a multiple of
- * 2048 runs on the matrix cores, other cases one GEMV per input row. */
+ * matvec path (lib.rs:173-182). On the matrix cores: Q4_K and Q6_K with batch
+ * >= 16 and cols a multiple of 2048; with cols another multiple of 256 from
+ * 1024 to 12288, Q4_K, Q6_K, F16 and BF16 with batch >= 4 and Q8_0 (2048 too)
+ * with batch >= 6, unless the stream is capturing. Other cases one GEMV per
+ * input row or per few. */
 int32_t mivi_hip_quantized_matmul_rows(float* out, size_t out_len, int32_t ggml_type,
                                        const uint8_t* weights, size_t weights_len,
                                        const float* inputs, size_t inputs_len, size_t batch,
@@ -262,7 +265,8 @@ int32_t mivi_hip_model_generate_greedy(mivi_model* m, size_t batch, const uint32
 /* Prompt prefill of one sequence (model.rs:499-606): with the default
  * PrefillStrategy::Token, forward_step(tokens[i], pos0 + i, false) per token;
  * after mivi_hip_model_set_prefill_tile(m, t > 1), PrefillStrategy::Chunked:
- * tiles of t tokens through every layer at once (model.rs:676-831,
+ * tiles of t tokens (from t = 64 on, as many as make up to 2048 tokens where
+ * every product runs on the matrix cores) through every layer at once (model.rs:676-831,
  * attention_forward_tile transformer.rs:356-559, ssm_forward_tile
  * ssm.rs:174-387): row-batch products (matrix cores for Q4_K), K/V and the
  * ShortConv state left as the token path leaves them. Synchronous. */

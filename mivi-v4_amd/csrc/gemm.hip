@@ -344,6 +344,7 @@ struct RowsArgs {
     const float* rowscale;
     int64_t ldy;
     int accumulate;            // y += result
+    int swiglu;                // seg[0] gate, seg[1] up, equal rows: seg[0].y = silu(gate) * up
 };
 
 // The 6-bit scale and min of sub-block j (compile time) from the 12 scale
@@ -427,9 +428,11 @@ __global__ void __launch_bounds__(256, 1) gemm_rows_kernel(const RowsArgs a) {
         tm = blockIdx.x / a.ntiles;
     }
     const int sg = a.nseg > 2 && tn >= a.seg[2].t0 ? 2 : a.nseg > 1 && tn >= a.seg[1].t0 ? 1 : 0;
-    const uint8_t* W = a.seg[sg].W;
     const int N = a.seg[sg].n;
-    const int c0 = ((tn - a.seg[sg].t0) * WN + wn) * 64;  // the wave's first column (weight row)
+    // the wave's two 32-column tiles: weight rows c0 + cj * j of Wj[j] (SwiGLU: the gate's rows and the up's)
+    const int cj = a.swiglu ? 0 : 32;
+    const int c0 = ((tn - a.seg[sg].t0) * WN + wn) * (32 + cj);
+    const uint8_t* const Wj[2] = {a.seg[sg].W, a.swiglu ? a.seg[1].W : a.seg[sg].W};
     const int K = a.K, KS = K / 16, NB = K / 256;
     const int nsb = (NB - kq + KQ - 1) / KQ;  // the wave's super-blocks kq, kq + KQ, ...
     const int nbt = SH ? (NB + KQ - 1) / KQ : nsb;
@@ -444,13 +447,13 @@ __global__ void __launch_bounds__(256, 1) gemm_rows_kernel(const RowsArgs a) {
 #pragma unroll
     for (int j = 0; j < 2; j++) {
         if constexpr (FMT == RF_Q4P) {
-            const int nt = min(c0 / 32 + j, N / 32 - 1);  // (past N: the last tile, computed and not stored)
-            Br[j] = buffer_of(W + (size_t)nt * KS * kStepBytes, (size_t)KS * kStepBytes);
-            Hr[j] = buffer_of(W + (size_t)N * K * 2 + (size_t)nt * NB * kGemmHBytes, (size_t)NB * kGemmHBytes);
+            const int nt = min((c0 + cj * j) / 32, N / 32 - 1);  // (past N: the last tile, computed and not stored)
+            Br[j] = buffer_of(Wj[j] + (size_t)nt * KS * kStepBytes, (size_t)KS * kStepBytes);
+            Hr[j] = buffer_of(Wj[j] + (size_t)N * K * 2 + (size_t)nt * NB * kGemmHBytes, (size_t)NB * kGemmHBytes);
         } else {
             const size_t rb = FMT == RF_Q4 ? (size_t)NB * 144 : FMT == RF_Q6 ? (size_t)NB * 210
                               : FMT == RF_Q8 ? (size_t)(K / 32) * 34 : (size_t)K * 2;
-            Bb[j] = W + (size_t)min(c0 + 32 * j + li, N - 1) * rb;
+            Bb[j] = Wj[j] + (size_t)min(c0 + cj * j + li, N - 1) * rb;
         }
     }
 
@@ -818,7 +821,7 @@ __global__ void __launch_bounds__(256, 1) gemm_rows_kernel(const RowsArgs a) {
             rs[i][g] = *(const f32x4*)(a.rowscale + m);
 #pragma unroll
             for (int j = 0; j < 2; j++) {
-                const int n = c0 + 32 * j + li;
+                const int n = c0 + cj * j + li;
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     old[i][j][g][e] = a.accumulate && m + e < a.M && n < N ? y[(m + e) * a.ldy + n] : 0.f;
@@ -836,14 +839,16 @@ __global__ void __launch_bounds__(256, 1) gemm_rows_kernel(const RowsArgs a) {
     for (int i = 0; i < MT; i++)
 #pragma unroll
         for (int j = 0; j < 2; j++) {
-            const int n = c0 + 32 * j + li;
+            if (a.swiglu && j == 1) continue;
+            const int n = c0 + cj * j + li;
 #pragma unroll
             for (int g = 0; g < NG; g++)
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     const int m = 32 * (tm * MT + i) + 8 * (g0 + g) + 4 * lh + e;
                     if (m < a.M && n < N) {
-                        const float r = v[i][j][g][e] * rs[i][g][e];
+                        float r = v[i][j][g][e] * rs[i][g][e];
+                        if (a.swiglu) r = silu_f(r) * (v[i][1][g][e] * rs[i][g][e]);  // ffn.rs:84-95
                         y[m * a.ldy + n] = a.accumulate ? old[i][j][g][e] + r : r;  // one writer per output
                     }
                 }
@@ -925,7 +930,9 @@ static RowsTile rows_tile(int32_t t, const GemvArgs& a, int mtiles) {
     for (int wn = wide; wn >= 1; wn /= 2) {
         if (env_wn && wn != env_wn && wide > 1) continue;
         int nt = 0;
-        for (int i = 0; i < a.nseg; i++) nt += (a.seg[i].n + 64 * wn - 1) / (64 * wn);
+        if (a.epilogue == EPI_SWIGLU) nt = (a.seg[0].n + 32 * wn - 1) / (32 * wn);
+        else
+            for (int i = 0; i < a.nseg; i++) nt += (a.seg[i].n + 64 * wn - 1) / (64 * wn);
         const int kq = 4 / wn, nsb = (a.K / 256 + kq - 1) / kq;
         const double rounds = (double)(((size_t)nt * mtiles + num_cus() - 1) / num_cus());
         const double cost = rounds * (3.0 + nsb * (wn == 4 ? 1.7 : wn == 2 ? 1.9 : 2.2));
@@ -954,20 +961,89 @@ static void launch_rows_kernel(const RowsArgs& r, int wn, int mt, hipStream_t s)
 // rows, so that the workspace stays bounded.
 constexpr size_t kRowsSlabBytes = 256u << 20;
 
+static size_t rows_slab(int32_t t, size_t K) {
+    const size_t P = t == MIVI_GGML_BF16 ? 3 : 2;
+    const size_t row_bytes = K * 2 * P + (t == MIVI_GGML_Q4_K ? K / 8 : 0) + 4;
+    return std::max<size_t>(64, kRowsSlabBytes / row_bytes / 64 * 64);
+}
+size_t mivi::launch_rows_workspace(int32_t t, size_t batch, size_t K) {
+    const size_t P = t == MIVI_GGML_BF16 ? 3 : 2;
+    const size_t mp = (std::min(batch, rows_slab(t, K)) + 63) / 64 * 64;
+    return mp * (K * 2 * P + (t == MIVI_GGML_Q4_K ? K / 8 : 0) + 4);
+}
+
+// The product with its workspace at hand.
+static int32_t rows_mfma_in(int32_t t, int pro, const GemvArgs& a, void* ws, hipStream_t s) {
+    const size_t K = (size_t)a.K, P = t == MIVI_GGML_BF16 ? 3 : 2;
+    const bool q4 = t == MIVI_GGML_Q4_K, swiglu = a.epilogue == EPI_SWIGLU;
+    const size_t slab = rows_slab(t, K);
+    const size_t mp0 = (std::min((size_t)a.ncol, slab) + 63) / 64 * 64;
+    const size_t bx = mp0 * K * 2 * P, bs = q4 ? mp0 * K / 8 : 0;
+    auto a16 = [](const void* p) { return p == nullptr || (uintptr_t)p % 16 == 0; };
+    const int vec = a16(a.x) && a16(a.x2) && a16(a.norm_w) && a.xs % 4 == 0;
+    bool packed = q4;
+    for (int i = 0; i < a.nseg; i++) packed = packed && a.seg[i].wg && a.seg[i].n % 32 == 0;
+    for (size_t m0 = 0; m0 < (size_t)a.ncol; m0 += slab) {
+        const int M = (int)std::min(slab, (size_t)a.ncol - m0);
+        const int mt = M <= 32 ? 1 : 2, mtiles = (M + 32 * mt - 1) / (32 * mt);
+        RowsArgs r = {};
+        r.xa = (const uint8_t*)ws;
+        r.xs = q4 ? r.xa + bx : nullptr;
+        float* rs = (float*)((uint8_t*)ws + bx + bs);
+        r.rowscale = rs;
+        r.K = (int)K;
+        r.M = M;
+        r.mtiles = mtiles;
+        r.ldy = a.ys;
+        r.accumulate = a.accumulate;
+        r.swiglu = swiglu;
+#define LP(R, PL)                                                                                                    \
+    hipLaunchKernelGGL((gemm_prep_kernel<R, PL>), dim3((unsigned)(mtiles * 32 * mt / kPrepRows)), dim3(512), 0, s, a.x + m0 * a.xs, \
+                       a.x2 ? a.x2 + m0 * a.xs : nullptr, a.norm_w, a.eps, pro, a.xs, M, (int)K, vec,                \
+                       (uint8_t*)ws, (uint8_t*)r.xs, rs)
+#define LPR(PL)                                                                                                      \
+    if (K <= 2048) LP(4, PL); else if (K <= 4096) LP(8, PL); else if (K <= 8192) LP(16, PL); \
+    else LP(0, PL)
+        if (P == 3) { LPR(3); } else { LPR(2); }
+#undef LPR
+#undef LP
+        const RowsTile tile = rows_tile(t, a, mtiles);
+        int t0 = 0;
+        for (int i = 0; i < a.nseg; i++) {
+            if (a.seg[i].n == 0) continue;  // (no tiles: left out of the table)
+            r.seg[r.nseg++] = {packed ? a.seg[i].wg : a.seg[i].W, a.seg[i].y + m0 * a.ys, a.seg[i].n, t0};
+            t0 += (a.seg[i].n + 64 * tile.wn - 1) / (64 * tile.wn);
+        }
+        if (swiglu) {
+            t0 = (a.seg[0].n + 32 * tile.wn - 1) / (32 * tile.wn);  // tiles of 32 gate|up pairs a wave
+            r.nseg = 1;  // (seg[1] stays in the table: the up rows)
+        }
+        r.ntiles = t0;
+        if (t0 == 0) break;
+        if (t == MIVI_GGML_Q6_K) launch_rows_kernel<RF_Q6>(r, tile.wn, mt, s);
+        else if (t == MIVI_GGML_Q8_0) launch_rows_kernel<RF_Q8>(r, tile.wn, mt, s);
+        else if (t == MIVI_GGML_F16) launch_rows_kernel<RF_F16>(r, tile.wn, mt, s);
+        else if (t == MIVI_GGML_BF16) launch_rows_kernel<RF_BF16>(r, tile.wn, mt, s);
+        else if (packed) launch_rows_kernel<RF_Q4P>(r, tile.wn, mt, s);
+        else launch_rows_kernel<RF_Q4>(r, tile.wn, mt, s);
+    }
+    MIVI_HIP_CHECK(hipGetLastError());
+    return MIVI_OK;
+}
+
 // Y_s[m * ys + n] (=|+=) sum_k W_s[n, k] * pro(X)[m, k] for the segments s
 // of a (K % 256 == 0): one activation split, one product over all segments.
 // MIVI_ERR_UNSUPPORTED when the workspace cannot be had.
 static int32_t rows_mfma(int32_t t, int pro, const GemvArgs& a, hipStream_t s) {
-    const size_t K = (size_t)a.K, P = t == MIVI_GGML_BF16 ? 3 : 2;
+    const size_t K = (size_t)a.K;
     const bool q4 = t == MIVI_GGML_Q4_K;
-    const size_t row_bytes = K * 2 * P + (q4 ? K / 8 : 0) + 4;
-    const size_t slab = std::max<size_t>(64, kRowsSlabBytes / row_bytes / 64 * 64);
-    const size_t mp0 = (std::min((size_t)a.ncol, slab) + 63) / 64 * 64;
-    const size_t bx = mp0 * K * 2 * P, bs = q4 ? mp0 * K / 8 : 0, bytes = bx + bs + mp0 * 4;
+    size_t bytes = launch_rows_workspace(t, (size_t)a.ncol, K);
+    if (a.ws && a.ws_bytes >= bytes) return rows_mfma_in(t, pro, a, a.ws, s);
     int dev = 0;
     MIVI_HIP_CHECK(hipGetDevice(&dev));
     GemmWorkspace& ws = gemm_workspace(dev);
     std::lock_guard<std::mutex> lk(ws.mu);
+    // (no system-scope release at the event: it orders work of this device, and the flush cost 6 us a call)
     if (!ws.done) MIVI_HIP_CHECK(hipEventCreateWithFlags(&ws.done, hipEventDisableTiming | hipEventDisableSystemFence));
     else MIVI_HIP_CHECK(hipStreamWaitEvent(s, ws.done, 0));  // the previous user is done with it
     if (ws.bytes < bytes) {
@@ -984,54 +1060,11 @@ static int32_t rows_mfma(int32_t t, int pro, const GemvArgs& a, hipStream_t s) {
         }
         ws.bytes = bytes;
     }
-    auto a16 = [](const void* p) { return p == nullptr || (uintptr_t)p % 16 == 0; };
-    const int vec = a16(a.x) && a16(a.x2) && a16(a.norm_w) && a.xs % 4 == 0;
-    bool packed = q4;
-    for (int i = 0; i < a.nseg; i++) packed = packed && a.seg[i].wg && a.seg[i].n % 32 == 0;
-    for (size_t m0 = 0; m0 < (size_t)a.ncol; m0 += slab) {
-        const int M = (int)std::min(slab, (size_t)a.ncol - m0);
-        const int mt = M <= 32 ? 1 : 2, mtiles = (M + 32 * mt - 1) / (32 * mt);
-        RowsArgs r = {};
-        r.xa = (const uint8_t*)ws.ptr;
-        r.xs = q4 ? r.xa + bx : nullptr;
-        float* rs = (float*)((uint8_t*)ws.ptr + bx + bs);
-        r.rowscale = rs;
-        r.K = (int)K;
-        r.M = M;
-        r.mtiles = mtiles;
-        r.ldy = a.ys;
-        r.accumulate = a.accumulate;
-#define LP(R, PL)                                                                                                    \
-    hipLaunchKernelGGL((gemm_prep_kernel<R, PL>), dim3((unsigned)(mtiles * 32 * mt / kPrepRows)), dim3(512), 0, s, a.x + m0 * a.xs, \
-                       a.x2 ? a.x2 + m0 * a.xs : nullptr, a.norm_w, a.eps, pro, a.xs, M, (int)K, vec,                \
-                       (uint8_t*)ws.ptr, (uint8_t*)r.xs, rs)
-#define LPR(PL)                                                                                                      \
-    if (K <= 2048) LP(4, PL); else if (K <= 4096) LP(8, PL); else if (K <= 8192) LP(16, PL); \
-    else LP(0, PL)
-        if (P == 3) { LPR(3); } else { LPR(2); }
-#undef LPR
-#undef LP
-        const RowsTile tile = rows_tile(t, a, mtiles);
-        int t0 = 0;
-        for (int i = 0; i < a.nseg; i++) {
-            if (a.seg[i].n == 0) continue;  // (no tiles: left out of the table)
-            r.seg[r.nseg++] = {packed ? a.seg[i].wg : a.seg[i].W, a.seg[i].y + m0 * a.ys, a.seg[i].n, t0};
-            t0 += (a.seg[i].n + 64 * tile.wn - 1) / (64 * tile.wn);
-        }
-        r.ntiles = t0;
-        if (t0 == 0) break;
-        if (t == MIVI_GGML_Q6_K) launch_rows_kernel<RF_Q6>(r, tile.wn, mt, s);
-        else if (t == MIVI_GGML_Q8_0) launch_rows_kernel<RF_Q8>(r, tile.wn, mt, s);
-        else if (t == MIVI_GGML_F16) launch_rows_kernel<RF_F16>(r, tile.wn, mt, s);
-        else if (t == MIVI_GGML_BF16) launch_rows_kernel<RF_BF16>(r, tile.wn, mt, s);
-        else if (packed) launch_rows_kernel<RF_Q4P>(r, tile.wn, mt, s);
-        else launch_rows_kernel<RF_Q4>(r, tile.wn, mt, s);
-    }
-    MIVI_HIP_CHECK(hipGetLastError());
+    const int32_t rc = rows_mfma_in(t, pro, a, ws.ptr, s);
+    if (rc) return rc;
     MIVI_HIP_CHECK(hipEventRecord(ws.done, s));
     return MIVI_OK;
 }
-
 namespace mivi {
 int32_t launch_pack_q4k_gemm(const uint8_t* src, uint8_t* dst, size_t rows, size_t cols, hipStream_t s) {
     if (rows % 32 || cols % 256 || rows > (size_t)INT32_MAX || cols > (size_t)INT32_MAX)
@@ -1045,9 +1078,16 @@ int32_t launch_pack_q4k_gemm(const uint8_t* src, uint8_t* dst, size_t rows, size
 }
 
 int32_t launch_rows(int32_t t, int pro, const GemvArgs& a, hipStream_t s) {
-    if (pro == PRO_CONV || a.epilogue != EPI_STORE)
-        return set_error(MIVI_ERR_UNSUPPORTED, "row products take no conv prologue or fused epilogue");
+    const bool swiglu = a.epilogue == EPI_SWIGLU;
+    if (pro == PRO_CONV || (a.epilogue != EPI_STORE && !swiglu))
+        return set_error(MIVI_ERR_UNSUPPORTED, "row products take no conv prologue and no such epilogue");
     const int route = rows_route(t, a);
+    if (swiglu) {
+        // (the models' prefill, with a workspace of its own and never under capture)
+        if (route == 0 || a.nseg != 2 || a.seg[1].n != a.seg[0].n || a.accumulate || !a.ws)
+            return set_error(MIVI_ERR_UNSUPPORTED, "no SwiGLU row product for this shape");
+        return rows_mfma(t, pro, a, s);
+    }
     if (route == 1) return rows_mfma(t, pro, a, s);
     if (route == 2) {
         // shapes whose GEMVs need no workspace: those still run them where

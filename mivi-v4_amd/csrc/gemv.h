@@ -58,6 +58,11 @@ struct GemvArgs {
     // Batched Q4_K columns (the column kernels): the launch's rows packed by
     // launch_pack_q4k_cols in the kernel's group order, else null (GGUF rows)
     const uint8_t* cw;
+    // Row products: the caller's workspace for the inputs' operand planes
+    // (launch_rows_workspace bytes, 16-byte aligned, used on the launch's
+    // stream only), else the device's shared one
+    void* ws;
+    size_t ws_bytes;
 };
 
 // Most columns one batched streaming launch takes (more are split into
@@ -93,11 +98,14 @@ int32_t launch_gemv_ex(int32_t ggml_type, int prologue, const GemvArgs& a, hipSt
 
 // Row-batch product: the a.ncol activation rows (row m at a.x + m * a.xs,
 // after the prologue) against each segment's weight rows, output row m of
-// segment s at a.seg[s].y + m * a.ys (=|+= with a.accumulate). Q4_K with at
-// least 16 rows and K % 2048 == 0 runs on the matrix cores (fp16 hi/lo
-// activations), anything else as a batched GEMV. No conv prologue, store
-// epilogue only.
+// segment s at a.seg[s].y + m * a.ys (=|+= with a.accumulate). On the matrix
+// cores where rows_route (gemm.hip) says so, else as batched GEMVs. No conv
+// prologue. Epilogues: store; EPI_SWIGLU (gate|up of equal rows, into
+// seg[0].y) on the matrix cores only (else MIVI_ERR_UNSUPPORTED, nothing
+// launched).
 int32_t launch_rows(int32_t ggml_type, int prologue, const GemvArgs& a, hipStream_t s);
+// Workspace of a product of `batch` rows of K columns (longer batches run in slabs).
+size_t launch_rows_workspace(int32_t ggml_type, size_t batch, size_t K);
 
 // rows x cols Q6_K (cols 2048/4096/8192) into the packed layout: row quads
 // when quad_layout(rows, cols), unit planes otherwise

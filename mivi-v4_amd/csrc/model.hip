@@ -2075,6 +2075,9 @@ struct mivi_model {
     float *pf_pm = nullptr, *pf_pl = nullptr, *pf_pa = nullptr;
     int* pf_pos = nullptr;
     uint32_t* pf_tok = nullptr;
+    uint8_t* pf_base = nullptr;  // the allocation that holds them
+    uint8_t* pf_ws = nullptr;    // the row products' workspace
+    size_t pf_ws_bytes = 0;
 
     ~mivi_model() {
         if (graph) hipGraphExecDestroy(graph);
@@ -2354,20 +2357,26 @@ int32_t enqueue_batch_step(mivi_model* m, size_t batch, hipStream_t s) {
 }
 
 constexpr int kPrefillSplits = 16;  // attention splits per tile row, at most
-// Shorter tiles keep the per-row kernels of the decode: under 64 rows a row
-// reads little that another does not (and tests hold short tiles over Q8_0
-// caches to the token path's own bits).
+// Shorter tiles keep the per-row kernels of the decode: the tests hold
+// chunked prefill in short tiles over Q8_0 caches, where one code's flip
+// shows, to the token path's own bits.
 constexpr size_t kPfMinRows = 64;
 
-// Attention of a prefill tile's rows: splits of the cached tokens where the
-// row blocks alone would leave CUs idle (two workgroups per CU), at least 512
-// tokens each.
+// Splits of the cached tokens where the row blocks of a tile alone would leave
+// CUs idle (two workgroups per CU).
+int attn_prefill_max_splits(const mivi_model_info& c, int rows) {
+    const int wr = attn_prefill_rows((int)(c.n_heads / c.n_kv_heads));
+    const int wgs = (rows + wr - 1) / wr * (int)c.n_kv_heads;
+    return std::max(1, std::min(kPrefillSplits, (2 * num_cus() + wgs - 1) / wgs));
+}
+
+// Attention of a prefill tile's rows, at least 512 tokens a split.
 void enqueue_attn_prefill(const mivi_model_info& c, AttnArgs a, int pos0, int rows, float* out, int64_t out_s,
                           hipStream_t s) {
     const int hpk = (int)(c.n_heads / c.n_kv_heads), wr = attn_prefill_rows(hpk);
     const int nrb = (rows + wr - 1) / wr, total = pos0 + rows;
     const int wgs = nrb * (int)c.n_kv_heads;
-    a.nsplit = std::max(1, std::min({kPrefillSplits, (2 * num_cus() + wgs - 1) / wgs, total / 512}));
+    a.nsplit = std::max(1, std::min(attn_prefill_max_splits(c, rows), total / 512));
     const int tsplit = ((total + a.nsplit - 1) / a.nsplit + kPfTokens - 1) / kPfTokens * kPfTokens;
     a.part_s = (int64_t)c.n_heads * a.nsplit;
     const dim3 grid((unsigned)(wgs * a.nsplit));
@@ -2381,20 +2390,67 @@ void enqueue_attn_prefill(const mivi_model_info& c, AttnArgs a, int pos0, int ro
                            a.part_l, a.part_acc, out, a.nsplit, a.part_s, out_s);
 }
 
-// Tile buffers for `rows` rows (grow-only).
+// Rows of a prefill pass through the layers: 2048 where every product runs on
+// the matrix cores, so that the 2048-row projections (32 x 8 tiles) fill 256
+// CUs; a tile of 512 leaves them 64 workgroups wide ones, or the narrow ones
+// that re-read the inputs 32 times (down projection: 185 us for 2048 rows
+// against 4 x 72). The tile the caller set stays the least a pass takes, and
+// all of it for other models.
+constexpr size_t kPassRows = 2048;
+size_t prefill_pass_rows(const mivi_model* m) {
+    const mivi_model_info& c = m->info;
+    const bool wide = c.dim >= 1024 && c.dim % 256 == 0 && c.hidden_dim % 256 == 0 && c.hidden_dim <= 12288 &&
+                      m->prefill_tile >= kPfMinRows && attn_prefill_ok(c, m->kv_packed);
+    return wide ? std::max(m->prefill_tile, kPassRows) : m->prefill_tile;
+}
+
+// Tile buffers for `rows` rows (grow-only), one allocation; a grown one takes
+// the old one's place.
 int32_t prefill_buffers(mivi_model* m, size_t rows) {
     if (m->pf_cap >= rows) return MIVI_OK;
     const mivi_model_info& c = m->info;
+    if (m->pf_base) {
+        // at least twice the rows, up to a whole pass: few regrowths
+        rows = std::max(rows, std::min(2 * m->pf_cap, prefill_pass_rows(m)));
+        MIVI_HIP_CHECK(hipStreamSynchronize(m->stream));
+        MIVI_HIP_CHECK(hipFree(m->pf_base));
+        m->allocs.erase(std::find(m->allocs.begin(), m->allocs.end(), (void*)m->pf_base));
+        m->pf_base = nullptr;
+        m->pf_cap = 0;
+    }
     const size_t D = c.dim, H = c.hidden_dim, KV = c.kv_dim;
     const size_t p1 = std::max({3 * D, D + 2 * KV, H});
-    const size_t parts = rows * c.n_heads * kPrefillSplits;
-    int32_t rc;
-    if ((rc = m->alloc(&m->pf_x, rows * D)) || (rc = m->alloc(&m->pf_p1, rows * p1)) ||
-        (rc = m->alloc(&m->pf_p2, rows * H)) || (rc = m->alloc(&m->pf_ao, rows * D)) ||
-        (rc = m->alloc(&m->pf_pm, parts)) || (rc = m->alloc(&m->pf_pl, parts)) ||
-        (rc = m->alloc(&m->pf_pa, parts * c.head_dim)) || (rc = m->alloc(&m->pf_pos, rows)) ||
-        (rc = m->alloc(&m->pf_tok, rows)))
-        return rc;
+    // attention partials: the per-row kernels' kPrefillSplits a row, or the
+    // prefill kernel's (two workgroups per CU in all; short tiles as above)
+    size_t parts = rows * kPrefillSplits;
+    if (attn_prefill_ok(c, m->kv_packed)) {
+        parts = std::min(rows, kPfMinRows) * kPrefillSplits;
+        for (size_t r = kPfMinRows; r <= rows; r++)
+            parts = std::max(parts, r * (size_t)attn_prefill_max_splits(c, (int)r));
+    }
+    parts *= c.n_heads;
+    size_t ws = 0;
+    for (const Layer& L : m->layers)
+        for (const Mat* x : {&L.wq, &L.wk, &L.wv, &L.wo, &L.in_proj, &L.out_proj, &L.gate, &L.up, &L.down})
+            if (x->w) ws = std::max(ws, launch_rows_workspace(x->type, rows, x->cols));
+    size_t off = 0;
+    auto take = [&](size_t bytes) {
+        const size_t o = off;
+        off += (bytes + 255) / 256 * 256;
+        return o;
+    };
+    const size_t o_x = take(rows * D * 4), o_p1 = take(rows * p1 * 4), o_p2 = take(rows * H * 4), o_ao = take(rows * D * 4);
+    const size_t o_pm = take(parts * 4), o_pl = take(parts * 4), o_pa = take(parts * c.head_dim * 4);
+    const size_t o_pos = take(rows * 4), o_tok = take(rows * 4), o_ws = take(ws);
+    uint8_t* base = nullptr;
+    int32_t rc = m->alloc(&base, off);
+    if (rc) return rc;
+    m->pf_base = base;
+    m->pf_x = (float*)(base + o_x); m->pf_p1 = (float*)(base + o_p1); m->pf_p2 = (float*)(base + o_p2);
+    m->pf_ao = (float*)(base + o_ao); m->pf_pm = (float*)(base + o_pm); m->pf_pl = (float*)(base + o_pl);
+    m->pf_pa = (float*)(base + o_pa); m->pf_pos = (int*)(base + o_pos); m->pf_tok = (uint32_t*)(base + o_tok);
+    m->pf_ws = base + o_ws;
+    m->pf_ws_bytes = ws;
     m->pf_cap = rows;
     return MIVI_OK;
 }
@@ -2420,6 +2476,8 @@ int32_t enqueue_prefill_tile(mivi_model* m, size_t b, size_t p0, size_t rows, hi
     for (size_t l = 0; l < c.n_layers; l++) {
         const Layer& L = m->layers[l];
         GemvArgs g = {};
+        g.ws = m->pf_ws; g.ws_bytes = m->pf_ws_bytes;
+        const GemvArgs g0 = g;
         if (!L.attn) {
             if (c.ssm_conv_kernel == 0) continue;  // ssm.rs:60-62
             g.seg[0] = {L.in_proj.w, m->pf_p1, 3 * D, L.in_proj.gemm};
@@ -2433,7 +2491,7 @@ int32_t enqueue_prefill_tile(mivi_model* m, size_t b, size_t p0, size_t rows, hi
                                dim3(256), 0, s, m->pf_p1,
                                m->pf_ao, R, D, (int)ks, L.conv, mode, st.conv_a + l * (size_t)D * ks,
                                st.conv_b + l * (size_t)D * ks, &m->ctrl->phase[b]);
-            g = {};
+            g = g0;
             g.seg[0] = {L.out_proj.w, m->pf_x, D, L.out_proj.gemm};
             g.nseg = 1; g.K = D; g.x = m->pf_ao; g.accumulate = 1;
             g.ncol = R; g.xs = D; g.ys = D;
@@ -2479,19 +2537,29 @@ int32_t enqueue_prefill_tile(mivi_model* m, size_t b, size_t p0, size_t rows, hi
                 a.part_s = (int64_t)c.n_heads * nsplit;
                 enqueue_attention(c, a, (unsigned)R, m->pf_ao, (int64_t)D, s);
             }
-            g = {};
+            g = g0;
             g.seg[0] = {L.wo.w, m->pf_x, D, L.wo.gemm};
             g.nseg = 1; g.K = D; g.x = m->pf_ao; g.accumulate = 1;
             g.ncol = R; g.xs = D; g.ys = D;
             if ((rc = launch_rows(L.wo.type, PRO_NONE, g, s))) return rc;
         }
         // ffn.rs:56-108 on the rows
-        g = {};
+        g = g0;
         g.seg[0] = {L.gate.w, m->pf_p1, H, L.gate.gemm};
         g.seg[1] = {L.up.w, m->pf_p2, H, L.up.gemm};
         g.nseg = 2; g.K = D; g.x = m->pf_x; g.norm_w = L.ffn_norm; g.eps = c.rms_norm_eps;
         g.ncol = R; g.xs = D; g.ys = H;
+        bool fused = false;
         if (L.gate.type == L.up.type) {
+            // silu(gate) * up in the product's store, where it runs on the matrix cores
+            g.epilogue = EPI_SWIGLU;
+            rc = launch_rows(L.gate.type, PRO_RMSNORM, g, s);
+            fused = rc == MIVI_OK;
+            if (rc && rc != MIVI_ERR_UNSUPPORTED) return rc;
+            g.epilogue = EPI_STORE;
+        }
+        if (fused) {
+        } else if (L.gate.type == L.up.type) {
             if ((rc = launch_rows(L.gate.type, PRO_RMSNORM, g, s))) return rc;
         } else {
             GemvArgs g1 = g;
@@ -2500,11 +2568,11 @@ int32_t enqueue_prefill_tile(mivi_model* m, size_t b, size_t p0, size_t rows, hi
             g1.seg[0] = g.seg[1];
             if ((rc = launch_rows(L.up.type, PRO_RMSNORM, g1, s))) return rc;
         }
-        g = {};
+        g = g0;
         g.seg[0] = {L.down.w, m->pf_x, D, L.down.gemm};
         g.nseg = 1; g.K = H; g.x = m->pf_p1; g.x2 = m->pf_p2; g.accumulate = 1;
         g.ncol = R; g.xs = H; g.ys = D;
-        if ((rc = launch_rows(L.down.type, PRO_SWIGLU, g, s))) return rc;
+        if ((rc = launch_rows(L.down.type, fused ? PRO_NONE : PRO_SWIGLU, g, s))) return rc;
     }
     MIVI_HIP_CHECK(hipGetLastError());
     return MIVI_OK;
@@ -3071,9 +3139,15 @@ extern "C" int32_t mivi_hip_model_prefill(mivi_model* m, size_t seq, const uint3
         if (rc) return rc;
     }
     if (m->prefill_tile > 1 && n > 1) {
-        // chunked: tiles of prefill_tile rows (model.rs:676-831)
-        const size_t tile = std::min(m->prefill_tile, n);
+        // chunked: tiles of prefill_tile rows (model.rs:676-831), several of
+        // them a pass where that fills the device
+        size_t tile = std::min(prefill_pass_rows(m), n);
         int32_t rc = prefill_buffers(m, tile);
+        if (rc && tile > m->prefill_tile) {  // no memory for the long pass: the caller's tiles
+            (void)hipGetLastError();
+            tile = std::min(m->prefill_tile, n);
+            rc = prefill_buffers(m, tile);
+        }
         if (rc) return rc;
         for (size_t c0 = 0; c0 < n; c0 += tile) {
             const size_t rows = std::min(tile, n - c0);
