@@ -105,9 +105,10 @@ int32_t mivi_hip_try_matvec_bf16(float* out, size_t out_len, const uint8_t* weig
  * out[batch, rows] = inputs[batch, cols] * W[rows, cols]^T. batch == 1 is the
  * matvec path (lib.rs:173-182). On the matrix cores: Q4_K and Q6_K with batch
  * >= 16 and cols a multiple of 2048; with cols another multiple of 256 from
- * 1024 to 12288, Q4_K, Q6_K, F16 and BF16 with batch >= 4 and Q8_0 (2048 too)
- * with batch >= 6, unless the stream is capturing. Other cases one GEMV per
- * input row or per few. */
+ * 1024 to 12288 Q4_K and Q6_K with batch >= 4; with any of these cols Q8_0, F16
+ * and BF16 from the batch on where that is faster (about 4 to 12); the last
+ * two unless the stream is capturing. Other cases one GEMV per input row or
+ * per few. */
 int32_t mivi_hip_quantized_matmul_rows(float* out, size_t out_len, int32_t ggml_type,
                                        const uint8_t* weights, size_t weights_len,
                                        const float* inputs, size_t inputs_len, size_t batch,

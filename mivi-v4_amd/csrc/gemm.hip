@@ -35,7 +35,6 @@ namespace {
 
 constexpr int kMfmaMinBatch = 16;     // K-quants at the depths of the batched GEMVs
 constexpr int kMfmaMinBatchRows = 4;  // shapes with one GEMV launch per input
-constexpr int kMfmaMinBatchQ8 = 6;    // the same, Q8_0
 constexpr int kTk = 64;  // k-tile of the packed copy: one Q4_K group (a sub-block pair)
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
@@ -911,7 +910,17 @@ static int rows_route(int32_t t, const GemvArgs& a) {
     // then equals the token path bit for bit, as the tests over Q8_0 caches
     // expect. The GEMVs stage one input row in LDS: longer ones than 12288 are
     // refused there.
-    return a.K >= 1024 && a.ncol >= (t == MIVI_GGML_Q8_0 ? kMfmaMinBatchQ8 : kMfmaMinBatchRows) && a.K <= 12288 ? 2 : 0;
+    if (a.K < 1024 || a.K > 12288 || a.ncol < kMfmaMinBatchRows) return 0;
+    if (kq) return 2;  // (4 inputs: 14-32 us against 24-46)
+    // Q8_0, F16, BF16: a GEMV is near its bytes' time, so few inputs stay
+    // with it. Fitted to both sides at 1024 to 8192 rows of 1024 to 4608
+    // columns (f16 2048 x 2048: 4 inputs 18 us against 22, 6 inputs 26 against
+    // 23; Q8_0 1024 x 4608: 8 inputs 34 against 52, 12 inputs 50 against 52).
+    double bytes = 0;
+    for (int i = 0; i < a.nseg; i++) bytes += (double)a.seg[i].n * a.K * (t == MIVI_GGML_Q8_0 ? 34.0 / 32 : 2.0);
+    const double gemvs = a.ncol * (3.2 + bytes / 4.2e6);
+    const double product = 10.0 + a.K * (t == MIVI_GGML_Q8_0 ? 0.0095 : 0.0072) + bytes / 5e6;
+    return product < gemvs ? 2 : 0;
 }
 
 // Workgroup shape of a product: WN column groups of 64 by KQ shares of the
@@ -1034,11 +1043,11 @@ static int32_t rows_mfma_in(int32_t t, int pro, const GemvArgs& a, void* ws, hip
 // Y_s[m * ys + n] (=|+=) sum_k W_s[n, k] * pro(X)[m, k] for the segments s
 // of a (K % 256 == 0): one activation split, one product over all segments.
 // MIVI_ERR_UNSUPPORTED when the workspace cannot be had.
-static int32_t rows_mfma(int32_t t, int pro, const GemvArgs& a, hipStream_t s) {
+static int32_t rows_mfma(int32_t t, int pro, const GemvArgs& a, hipStream_t s, const RowsWorkspace& own) {
     const size_t K = (size_t)a.K;
     const bool q4 = t == MIVI_GGML_Q4_K;
     size_t bytes = launch_rows_workspace(t, (size_t)a.ncol, K);
-    if (a.ws && a.ws_bytes >= bytes) return rows_mfma_in(t, pro, a, a.ws, s);
+    if (own.p && own.bytes >= bytes) return rows_mfma_in(t, pro, a, own.p, s);
     int dev = 0;
     MIVI_HIP_CHECK(hipGetDevice(&dev));
     GemmWorkspace& ws = gemm_workspace(dev);
@@ -1077,24 +1086,24 @@ int32_t launch_pack_q4k_gemm(const uint8_t* src, uint8_t* dst, size_t rows, size
     return MIVI_OK;
 }
 
-int32_t launch_rows(int32_t t, int pro, const GemvArgs& a, hipStream_t s) {
+int32_t launch_rows(int32_t t, int pro, const GemvArgs& a, hipStream_t s, const RowsWorkspace& ws) {
     const bool swiglu = a.epilogue == EPI_SWIGLU;
     if (pro == PRO_CONV || (a.epilogue != EPI_STORE && !swiglu))
         return set_error(MIVI_ERR_UNSUPPORTED, "row products take no conv prologue and no such epilogue");
     const int route = rows_route(t, a);
     if (swiglu) {
         // (the models' prefill, with a workspace of its own and never under capture)
-        if (route == 0 || a.nseg != 2 || a.seg[1].n != a.seg[0].n || a.accumulate || !a.ws)
+        if (route == 0 || a.nseg != 2 || a.seg[1].n != a.seg[0].n || a.accumulate || !ws.p)
             return set_error(MIVI_ERR_UNSUPPORTED, "no SwiGLU row product for this shape");
-        return rows_mfma(t, pro, a, s);
+        return rows_mfma(t, pro, a, s, ws);
     }
-    if (route == 1) return rows_mfma(t, pro, a, s);
+    if (route == 1) return rows_mfma(t, pro, a, s, ws);
     if (route == 2) {
         // shapes whose GEMVs need no workspace: those still run them where
         // none can be had (a capturing stream, no memory)
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
-            const int32_t rc = rows_mfma(t, pro, a, s);
+            const int32_t rc = rows_mfma(t, pro, a, s, ws);
             if (rc != MIVI_ERR_UNSUPPORTED) return rc;
             clear_error();
         } else {

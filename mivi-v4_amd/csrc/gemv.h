@@ -58,11 +58,14 @@ struct GemvArgs {
     // Batched Q4_K columns (the column kernels): the launch's rows packed by
     // launch_pack_q4k_cols in the kernel's group order, else null (GGUF rows)
     const uint8_t* cw;
-    // Row products: the caller's workspace for the inputs' operand planes
-    // (launch_rows_workspace bytes, 16-byte aligned, used on the launch's
-    // stream only), else the device's shared one
-    void* ws;
-    size_t ws_bytes;
+};
+
+// Row products: a caller's workspace for the inputs' operand planes
+// (launch_rows_workspace bytes, 16-byte aligned, used on the launches' stream
+// only); none: the device's shared one.
+struct RowsWorkspace {
+    void* p = nullptr;
+    size_t bytes = 0;
 };
 
 // Most columns one batched streaming launch takes (more are split into
@@ -103,7 +106,7 @@ int32_t launch_gemv_ex(int32_t ggml_type, int prologue, const GemvArgs& a, hipSt
 // prologue. Epilogues: store; EPI_SWIGLU (gate|up of equal rows, into
 // seg[0].y) on the matrix cores only (else MIVI_ERR_UNSUPPORTED, nothing
 // launched).
-int32_t launch_rows(int32_t ggml_type, int prologue, const GemvArgs& a, hipStream_t s);
+int32_t launch_rows(int32_t ggml_type, int prologue, const GemvArgs& a, hipStream_t s, const RowsWorkspace& ws = {});
 // Workspace of a product of `batch` rows of K columns (longer batches run in slabs).
 size_t launch_rows_workspace(int32_t ggml_type, size_t batch, size_t K);
 

@@ -2467,6 +2467,7 @@ int32_t enqueue_prefill_tile(mivi_model* m, size_t b, size_t p0, size_t rows, hi
     SeqState& st = m->seqs[b];
     const int D = (int)c.dim, H = (int)c.hidden_dim, KV = (int)c.kv_dim, R = (int)rows;
     const size_t ldq = (size_t)D + 2 * KV;
+    const RowsWorkspace ws = {m->pf_ws, m->pf_ws_bytes};
     int32_t rc;
     size_t bs, ts;
     format_sizes(m->embd.type, &bs, &ts);
@@ -2476,14 +2477,12 @@ int32_t enqueue_prefill_tile(mivi_model* m, size_t b, size_t p0, size_t rows, hi
     for (size_t l = 0; l < c.n_layers; l++) {
         const Layer& L = m->layers[l];
         GemvArgs g = {};
-        g.ws = m->pf_ws; g.ws_bytes = m->pf_ws_bytes;
-        const GemvArgs g0 = g;
         if (!L.attn) {
             if (c.ssm_conv_kernel == 0) continue;  // ssm.rs:60-62
             g.seg[0] = {L.in_proj.w, m->pf_p1, 3 * D, L.in_proj.gemm};
             g.nseg = 1; g.K = D; g.x = m->pf_x; g.norm_w = L.norm; g.eps = c.rms_norm_eps;
             g.ncol = R; g.xs = D; g.ys = 3 * D;
-            if ((rc = launch_rows(L.in_proj.type, PRO_RMSNORM, g, s))) return rc;
+            if ((rc = launch_rows(L.in_proj.type, PRO_RMSNORM, g, s, ws))) return rc;
             const size_t ks = c.ssm_conv_kernel;
             const int mode = (L.conv && L.conv_len >= (size_t)D * ks) ? 0 : (L.conv && L.conv_len >= ks) ? 1 : 2;
             hipLaunchKernelGGL(conv_rows_kernel,
@@ -2491,11 +2490,11 @@ int32_t enqueue_prefill_tile(mivi_model* m, size_t b, size_t p0, size_t rows, hi
                                dim3(256), 0, s, m->pf_p1,
                                m->pf_ao, R, D, (int)ks, L.conv, mode, st.conv_a + l * (size_t)D * ks,
                                st.conv_b + l * (size_t)D * ks, &m->ctrl->phase[b]);
-            g = g0;
+            g = {};
             g.seg[0] = {L.out_proj.w, m->pf_x, D, L.out_proj.gemm};
             g.nseg = 1; g.K = D; g.x = m->pf_ao; g.accumulate = 1;
             g.ncol = R; g.xs = D; g.ys = D;
-            if ((rc = launch_rows(L.out_proj.type, PRO_NONE, g, s))) return rc;
+            if ((rc = launch_rows(L.out_proj.type, PRO_NONE, g, s, ws))) return rc;
         } else {
             g.seg[0] = {L.wq.w, m->pf_p1, D, L.wq.gemm};
             g.seg[1] = {L.wk.w, m->pf_p1 + D, KV, L.wk.gemm};
@@ -2503,7 +2502,7 @@ int32_t enqueue_prefill_tile(mivi_model* m, size_t b, size_t p0, size_t rows, hi
             g.nseg = 3; g.K = D; g.x = m->pf_x; g.norm_w = L.norm; g.eps = c.rms_norm_eps;
             g.ncol = R; g.xs = D; g.ys = (int64_t)ldq;
             rc = by_type_runs(g, {&L.wq, &L.wk, &L.wv}, [&](int32_t t, const GemvArgs& gr, const Mat* const*, int) {
-                return launch_rows(t, PRO_RMSNORM, gr, s);
+                return launch_rows(t, PRO_RMSNORM, gr, s, ws);
             });
             if (rc) return rc;
             AttnArgs a = {};
@@ -2537,14 +2536,14 @@ int32_t enqueue_prefill_tile(mivi_model* m, size_t b, size_t p0, size_t rows, hi
                 a.part_s = (int64_t)c.n_heads * nsplit;
                 enqueue_attention(c, a, (unsigned)R, m->pf_ao, (int64_t)D, s);
             }
-            g = g0;
+            g = {};
             g.seg[0] = {L.wo.w, m->pf_x, D, L.wo.gemm};
             g.nseg = 1; g.K = D; g.x = m->pf_ao; g.accumulate = 1;
             g.ncol = R; g.xs = D; g.ys = D;
-            if ((rc = launch_rows(L.wo.type, PRO_NONE, g, s))) return rc;
+            if ((rc = launch_rows(L.wo.type, PRO_NONE, g, s, ws))) return rc;
         }
         // ffn.rs:56-108 on the rows
-        g = g0;
+        g = {};
         g.seg[0] = {L.gate.w, m->pf_p1, H, L.gate.gemm};
         g.seg[1] = {L.up.w, m->pf_p2, H, L.up.gemm};
         g.nseg = 2; g.K = D; g.x = m->pf_x; g.norm_w = L.ffn_norm; g.eps = c.rms_norm_eps;
@@ -2553,26 +2552,26 @@ int32_t enqueue_prefill_tile(mivi_model* m, size_t b, size_t p0, size_t rows, hi
         if (L.gate.type == L.up.type) {
             // silu(gate) * up in the product's store, where it runs on the matrix cores
             g.epilogue = EPI_SWIGLU;
-            rc = launch_rows(L.gate.type, PRO_RMSNORM, g, s);
+            rc = launch_rows(L.gate.type, PRO_RMSNORM, g, s, ws);
             fused = rc == MIVI_OK;
             if (rc && rc != MIVI_ERR_UNSUPPORTED) return rc;
             g.epilogue = EPI_STORE;
         }
         if (fused) {
         } else if (L.gate.type == L.up.type) {
-            if ((rc = launch_rows(L.gate.type, PRO_RMSNORM, g, s))) return rc;
+            if ((rc = launch_rows(L.gate.type, PRO_RMSNORM, g, s, ws))) return rc;
         } else {
             GemvArgs g1 = g;
             g1.nseg = 1;
-            if ((rc = launch_rows(L.gate.type, PRO_RMSNORM, g1, s))) return rc;
+            if ((rc = launch_rows(L.gate.type, PRO_RMSNORM, g1, s, ws))) return rc;
             g1.seg[0] = g.seg[1];
-            if ((rc = launch_rows(L.up.type, PRO_RMSNORM, g1, s))) return rc;
+            if ((rc = launch_rows(L.up.type, PRO_RMSNORM, g1, s, ws))) return rc;
         }
-        g = g0;
+        g = {};
         g.seg[0] = {L.down.w, m->pf_x, D, L.down.gemm};
         g.nseg = 1; g.K = H; g.x = m->pf_p1; g.x2 = m->pf_p2; g.accumulate = 1;
         g.ncol = R; g.xs = H; g.ys = D;
-        if ((rc = launch_rows(L.down.type, fused ? PRO_NONE : PRO_SWIGLU, g, s))) return rc;
+        if ((rc = launch_rows(L.down.type, fused ? PRO_NONE : PRO_SWIGLU, g, s, ws))) return rc;
     }
     MIVI_HIP_CHECK(hipGetLastError());
     return MIVI_OK;

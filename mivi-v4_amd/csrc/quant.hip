@@ -432,8 +432,224 @@ __global__ void __launch_bounds__(kWG) gemv_q6k_kernel(const mivi::GemvArgs a) {
     }
 }
 
+// --------------------------------------------- F16, BF16 and F32 rows, any K
+
+enum RowKind : int { RK_F16 = 0, RK_BF16 = 1, RK_F32 = 2 };
+typedef uint32_t u32x4_a1 __attribute__((ext_vector_type(4), aligned(1)));
+
+// A wave takes groups of R rows (group, group + waves, ...), its 64 lanes
+// consecutive 16-byte chunks of a row, NJ chunks a lane and row per batch, so
+// that R * NJ loads of a batch are in flight while the batch before is
+// multiplied: memory-bound, where one 2-byte load a lane at a time was bound by
+// latency (bf16 65536 x 1024: 67 -> 25 us, f16 8192 x 2048: 20 -> 9.6, f16 2048
+// x 8192: 54 -> 14; the first one's bytes take 22 us at 6 TB/s). Rows of one
+// batch (K <= 64 * NJ chunks) keep their inputs in registers. ODD: K not a
+// whole number of chunks; rows then start on any 2-byte boundary, where a
+// 16-byte load splits (three times the time), so the 16-bit kinds load aligned
+// dwords and shift, and the last K % CW values come one to a lane. Four sums a
+// lane and row keep the f32 chains short.
+template <int KIND, int R, int NJ, bool ODD, int PRO>
+__global__ void __launch_bounds__(kWG) gemv_rows_kernel(const mivi::GemvArgs a) {
+    extern __shared__ float lds[];
+    stage_input<PRO, 0>(lds, a);
+    constexpr int CW = KIND == RK_F32 ? 4 : 8, EB = KIND == RK_F32 ? 4 : 2;  // values of a chunk, bytes of a value
+    const int K = a.K, KF = K / CW * CW, rem = K - KF;  // whole chunks, the values after them
+    const Segs sg(a, (size_t)K * EB);
+    const int n = sg.n;
+    const int lane = threadIdx.x & 63;
+    const int nwaves = gridDim.x * (kWG / 64);
+    const int ng = (n + R - 1) / R, nj = (KF + 64 * CW - 1) / (64 * CW), nb = max(1, (nj + NJ - 1) / NJ);
+
+    struct Batch {
+        u32x4 w[R][NJ];
+        uint32_t t[ODD ? R : 1];  // ODD: the lane's value of the remainder (last batch)
+    };
+    auto load = [&](Batch& B, int g, int bt) {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const uint8_t* row = sg.row(min(g * R + r, n - 1));
+            if (!ODD || KF > 0) {
+#pragma unroll
+                for (int j = 0; j < NJ; j++) {
+                    const int k = CW * (lane + 64 * (bt * NJ + j));
+                    const bool in = k < KF;
+                    const uint8_t* p = row + (size_t)(in ? k : 0) * EB;
+                    u32x4 v;
+                    if constexpr (ODD && EB == 2) v = ld16_a2(p);
+                    else v = *(const u32x4_a1*)p;
+                    B.w[r][j] = in ? v : u32x4{0u, 0u, 0u, 0u};
+                }
+            }
+            if constexpr (ODD) {
+                const uint8_t* p = row + (size_t)(KF + (lane < rem ? lane : 0)) * EB;
+                uint32_t v = p[0] | (p[1] << 8);
+                if constexpr (EB == 4) v |= (p[2] << 16) | ((uint32_t)p[3] << 24);
+                B.t[r] = lane < rem ? v : 0u;
+            }
+        }
+    };
+    auto inputs = [&](float (&x)[CW], int j) {  // the lane's inputs of chunk j (0 past the end)
+        const int k = CW * (lane + 64 * j);
+        const bool in = k < KF;
+#pragma unroll
+        for (int q = 0; q < CW / 4; q++) {
+            const f32x4 v = *(const f32x4*)(lds + (in ? k : 0) + 4 * q);
+            x[4 * q] = in ? v.x : 0.f; x[4 * q + 1] = in ? v.y : 0.f;
+            x[4 * q + 2] = in ? v.z : 0.f; x[4 * q + 3] = in ? v.w : 0.f;
+        }
+    };
+    auto weight = [&](const u32x4& w, int e) -> float {  // value e of a chunk
+        if constexpr (KIND == RK_F32) return __uint_as_float(w[e]);
+        else if constexpr (KIND == RK_F16) return half_bits_to_f32(w[e >> 1] >> (16 * (e & 1)));
+        else return __uint_as_float(e & 1 ? w[e >> 1] & 0xFFFF0000u : w[e >> 1] << 16);
+    };
+
+    constexpr bool XR = NJ * CW <= 32;  // one batch a row: inputs in registers
+    float xr[XR ? NJ : 1][CW];
+    if constexpr (XR)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) inputs(xr[j], j);
+    const float xt = ODD && lane < rem ? lds[KF + lane] : 0.f;
+    float acc[R][4];
+    auto clear = [&]() {
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[r][i] = 0.f;
+    };
+    auto multiply = [&](const Batch& B, int bt) {
+        if (!ODD || KF > 0) {
+#pragma unroll
+            for (int j = 0; j < NJ; j++) {
+                float x[CW];
+                if (XR && nb == 1) {
+#pragma unroll
+                    for (int e = 0; e < CW; e++) x[e] = xr[XR ? j : 0][e];
+                } else {
+                    inputs(x, bt * NJ + j);
+                }
+#pragma unroll
+                for (int r = 0; r < R; r++)
+#pragma unroll
+                    for (int e = 0; e < CW; e++) acc[r][e & 3] = fmaf(weight(B.w[r][j], e), x[e], acc[r][e & 3]);
+            }
+        }
+    };
+    Batch ring[2];
+    int g = blockIdx.x * (kWG / 64) + (threadIdx.x >> 6), bt = 0;
+    if (g >= ng) return;
+    load(ring[0], g, 0);
+    clear();
+    auto step = [&](const Batch& cur, Batch& nxt) {  // returns with (g, bt) moved on
+        int gn = g, bn = bt + 1;
+        if (bn == nb) { bn = 0; gn = g + nwaves; }
+        load(nxt, gn < ng ? gn : g, gn < ng ? bn : bt);  // (past the end: a re-read)
+        multiply(cur, bt);
+        if (bt + 1 == nb) {
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                if constexpr (ODD) acc[r][0] = fmaf(weight(u32x4{cur.t[r], 0u, 0u, 0u}, 0), xt, acc[r][0]);
+                const float v = xsum_all64((acc[r][0] + acc[r][1]) + (acc[r][2] + acc[r][3]));
+                if (lane == 0 && g * R + r < n) store_out(sg, a.accumulate, g * R + r, v);
+            }
+            clear();
+        }
+        g = gn;
+        bt = bn;
+    };
+    while (true) {
+        step(ring[0], ring[1]);
+        if (g >= ng) break;
+        step(ring[1], ring[0]);
+        if (g >= ng) break;
+    }
+}
+
 // ------------------------------------------------------------------- Q8_0
 
+// Q8_0 rows of block pairs (K % 64 == 0, 4-byte aligned): a lane takes whole
+// pairs, 68 bytes as 17 aligned dwords (a block alone starts on a 2-byte
+// boundary, where wide loads split), LPR lanes to a row of up to LPR * NC
+// pairs, the pairs' inputs in registers for the whole launch, two steps of
+// rows in flight.
+template <int LPR, int NC, int PRO>
+__global__ void __launch_bounds__(kWG) gemv_q80_pairs_kernel(const mivi::GemvArgs a) {
+    extern __shared__ float lds[];
+    stage_input<PRO, 0>(lds, a);
+    constexpr int RPW = 64 / LPR;  // rows of a wave step
+    const int np = a.K / 64;
+    // the inputs again, 68 floats a pair: the lanes' 64-float slices, read at
+    // one stride, then fall in distinct banks (512 x 2048: 9.3 us without)
+    float* xp = lds + a.K;
+    for (int q = threadIdx.x; q < a.K / 4; q += kWG) *(f32x4*)(xp + 4 * q + 4 * (q / 16)) = *(const f32x4*)(lds + 4 * q);
+    __syncthreads();
+    const Segs sg(a, (size_t)np * 68);
+    const int n = sg.n;
+    const int lane = threadIdx.x & 63, lr = lane % LPR, sub = lane / LPR;
+    const int nwaves = gridDim.x * (kWG / 64), nsteps = (n + RPW - 1) / RPW;
+    float x[NC][64];
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+        const bool in = lr + LPR * c < np;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const f32x4 v = *(const f32x4*)(xp + (in ? 68 * (lr + LPR * c) : 0) + 4 * i);
+            x[c][4 * i] = v.x; x[c][4 * i + 1] = v.y; x[c][4 * i + 2] = v.z; x[c][4 * i + 3] = v.w;
+        }
+    }
+    struct Step {
+        u32x4 w[NC][4];
+        uint32_t t[NC];
+    };
+    auto load = [&](Step& S, int st) {
+        const uint8_t* row = sg.row(min(st * RPW + sub, n - 1));
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            const uint8_t* p = row + (size_t)min(lr + LPR * c, np - 1) * 68;
+#pragma unroll
+            for (int i = 0; i < 4; i++) S.w[c][i] = *(const u32x4_a4*)(p + 16 * i);
+            S.t[c] = *(const uint32_t*)(p + 64);
+        }
+    };
+    Step ring[2];
+    int st = blockIdx.x * (kWG / 64) + (threadIdx.x >> 6);
+    if (st >= nsteps) return;
+    load(ring[0], st);
+    auto step = [&](const Step& S, Step& N) {
+        const int sn = st + nwaves;
+        load(N, sn < nsteps ? sn : st);  // (past the end: a re-read)
+        float acc = 0.f;
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            uint32_t d[17];
+#pragma unroll
+            for (int i = 0; i < 16; i++) d[i] = S.w[c][i >> 2][i & 3];
+            d[16] = S.t[c];
+            // block 0: d0 | quants from byte 2; block 1: its scale at byte 34, quants from byte 36
+            float s0[4] = {0.f, 0.f, 0.f, 0.f}, s1[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int e = 0; e < 32; e++) {
+                s0[e & 3] = fmaf(sbyte_f32(d[(2 + e) >> 2], (2 + e) & 3), x[c][e], s0[e & 3]);
+                s1[e & 3] = fmaf(sbyte_f32(d[9 + (e >> 2)], e & 3), x[c][32 + e], s1[e & 3]);
+            }
+            const float p = fmaf(half_bits_to_f32(d[0]), (s0[0] + s0[1]) + (s0[2] + s0[3]),
+                                 half_bits_to_f32(d[8] >> 16) * ((s1[0] + s1[1]) + (s1[2] + s1[3])));
+            acc += lr + LPR * c < np ? p : 0.f;
+        }
+        acc = group_sum<LPR>(acc);
+        const int r = st * RPW + sub;
+        if (lr == 0 && r < n) store_out(sg, a.accumulate, r, acc);
+        st = sn;
+    };
+    while (true) {
+        step(ring[0], ring[1]);
+        if (st >= nsteps) break;
+        step(ring[1], ring[0]);
+        if (st >= nsteps) break;
+    }
+}
+
+// Any K (a multiple of 32) and alignment: one block a lane.
 template <int LPR, int U, int PRO>
 __global__ void __launch_bounds__(kWG) gemv_q80_kernel(const mivi::GemvArgs a) {
     extern __shared__ float lds[];
@@ -485,39 +701,6 @@ __global__ void __launch_bounds__(kWG) gemv_q80_kernel(const mivi::GemvArgs a) {
             int r = tile * RPT + k * RPG + sub;
             if (lr == 0 && r < n) store_out(sg, a.accumulate, r, s);
         }
-    }
-}
-
-// -------------------------------------------------- F16 / BF16 / F32 rows
-
-// KIND 0 f16, 1 bf16, 2 f32. One wave per row; rows of any alignment.
-template <int KIND, int PRO>
-__global__ void __launch_bounds__(kWG) gemv_dense_kernel(const mivi::GemvArgs a) {
-    extern __shared__ float lds[];
-    stage_input<PRO, 0>(lds, a);
-    const int d = a.K;
-    const size_t row_bytes = (size_t)d * (KIND == 2 ? 4 : 2);
-    const Segs sg(a, row_bytes);
-    const int n = sg.n;
-    const int lane = threadIdx.x & 63;
-    const int nwaves = gridDim.x * (kWG / 64);
-    for (int r = blockIdx.x * (kWG / 64) + (threadIdx.x >> 6); r < n; r += nwaves) {
-        const uint8_t* row = sg.row(r, row_bytes);
-        float acc = 0.f;
-        for (int k = lane; k < d; k += 64) {
-            float w;
-            if (KIND == 2) {
-                const uint8_t* p = row + 4 * (size_t)k;
-                w = ((uintptr_t)p & 3) ? __uint_as_float(p[0] | (p[1] << 8) | (p[2] << 16) | ((uint32_t)p[3] << 24))
-                                       : *(const float*)p;
-            } else {
-                uint32_t bits = ld_u16(row + 2 * (size_t)k);
-                w = KIND == 0 ? half_bits_to_f32(bits) : bf16_bits_to_f32(bits);
-            }
-            acc = fmaf(w, lds[k], acc);
-        }
-        acc = wave_sum(acc);
-        if (lane == 0) store_out(sg, a.accumulate, r, acc);
     }
 }
 
@@ -3462,8 +3645,24 @@ int32_t launch_pro(int32_t t, const mivi::GemvArgs& a, int n, hipStream_t s) {
     }
     case MIVI_GGML_Q8_0: {
         const int nb = K / 32;
+        size_t lds = (size_t)K * 4;
+        bool pairs = K % 64 == 0 && K <= 8192;
+        for (int i = 0; i < a.nseg; i++) pairs = pairs && (uintptr_t)a.seg[i].W % 4 == 0;
+        if (pairs) {
+            lds += (size_t)K / 64 * 272;
+            const int np = K / 64, lpr = std::max(8, std::min(64, pow2_ceil(np)));
+            static const int per_cu = env_int("MIVI_GEMV_Q80_WG_PER_CU", 2);
+            const int grid = std::max(1, std::min((n + 4 * (64 / lpr) - 1) / (4 * (64 / lpr)), mivi::num_cus() * per_cu));
+#define LQ(LPR, NC) hipLaunchKernelGGL((gemv_q80_pairs_kernel<LPR, NC, PRO>), dim3(grid), dim3(kWG), lds, s, a)
+            if (np > 64) LQ(64, 2);
+            else if (lpr == 64) LQ(64, 1);
+            else if (lpr == 32) LQ(32, 1);
+            else if (lpr == 16) LQ(16, 1);
+            else LQ(8, 1);
+#undef LQ
+            break;
+        }
         const int lpr = std::min(64, pow2_ceil(nb));
-        const size_t lds = (size_t)K * 4;
         const int grid = grid_for((n + (64 / lpr) * U - 1) / ((64 / lpr) * U));
         BY_LPR(gemv_q80_kernel)
         break;
@@ -3471,11 +3670,24 @@ int32_t launch_pro(int32_t t, const mivi::GemvArgs& a, int n, hipStream_t s) {
     case MIVI_GGML_F16:
     case MIVI_GGML_BF16:
     case MIVI_GGML_F32: {
-        const size_t lds = (size_t)K * 4;
-        const int grid = grid_for(n);
-        if (t == MIVI_GGML_F16) hipLaunchKernelGGL((gemv_dense_kernel<0, PRO>), dim3(grid), dim3(kWG), lds, s, a);
-        else if (t == MIVI_GGML_BF16) hipLaunchKernelGGL((gemv_dense_kernel<1, PRO>), dim3(grid), dim3(kWG), lds, s, a);
-        else hipLaunchKernelGGL((gemv_dense_kernel<2, PRO>), dim3(grid), dim3(kWG), lds, s, a);
+        const int cw = t == MIVI_GGML_F32 ? 4 : 8;
+        const int nj = (K + 64 * cw - 1) / (64 * cw);
+        const bool odd = K % cw != 0;
+        // rows of up to two chunks a lane in groups of four, up to four
+        // chunks in pairs, longer ones alone: eight loads a batch each way
+        const int R = nj <= 2 ? 4 : nj <= 4 ? 2 : 1;
+        const size_t lds = (size_t)(K + 3) / 4 * 16;
+        // two workgroups per CU: 25.2 us for bf16 65536 x 1024 (26.8 at four, 27.1 at eight)
+        static const int per_cu = env_int("MIVI_GEMV_ROWS_WG_PER_CU", 2);
+        const int grid = std::max(1, std::min(((n + R - 1) / R + 3) / 4, mivi::num_cus() * per_cu));
+#define LR(KIND, R, NJ, ODD) hipLaunchKernelGGL((gemv_rows_kernel<KIND, R, NJ, ODD, PRO>), dim3(grid), dim3(kWG), lds, s, a)
+#define LRS(KIND, ODD) \
+    if (R == 4) LR(KIND, 4, 2, ODD); else if (R == 2) LR(KIND, 2, 4, ODD); else LR(KIND, 1, 8, ODD)
+        if (t == MIVI_GGML_F16) { if (odd) { LRS(RK_F16, true); } else { LRS(RK_F16, false); } }
+        else if (t == MIVI_GGML_BF16) { if (odd) { LRS(RK_BF16, true); } else { LRS(RK_BF16, false); } }
+        else { if (odd) { LRS(RK_F32, true); } else { LRS(RK_F32, false); } }
+#undef LRS
+#undef LR
         break;
     }
     default: return mivi::err_unsupported(t);

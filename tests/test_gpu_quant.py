@@ -585,7 +585,7 @@ def _rows_case(hip, t, batch, rows, cols):
 @pytest.mark.parametrize("batch,rows,cols", [(6, 1, 1024), (6, 63, 1280), (31, 65, 1024), (33, 200, 1792), (64, 129, 1536),
                                              (65, 257, 4608), (8, 64, 10240), (97, 300, 2304), (32, 64, 12288)])
 def test_matmul_rows_matrix_cores_any_depth(hip, oracle, torch_mod, t, batch, rows, cols):
-    # the row products at depths with one GEMV launch per input (from 4 or 6
+    # the row products at depths with one GEMV launch per input (from a few
     # inputs on): every weight format, tile edges in both directions, shares
     # of the depth without a super-block, inputs from 1e-30 to 1e30; each
     # output within a tenth of the bar of the f64 product of the stored
@@ -609,7 +609,7 @@ def test_matmul_rows_matrix_cores_any_depth(hip, oracle, torch_mod, t, batch, ro
 def test_matmul_rows_matrix_cores_infinite_inputs(hip, torch_mod, t):
     # an infinite input gives the infinities and NaNs of its own matvec
     torch = torch_mod
-    batch, rows, cols = 7, 70, 1280
+    batch, rows, cols = 16, 70, 1280
     w, X = _rows_case(hip, t, batch, rows, cols)
     X[4, 17] = np.inf
     X[5, 30], X[5, 31] = np.inf, -np.inf
@@ -657,3 +657,32 @@ def test_matmul_rows_any_depth_unaligned_and_captured(hip, torch_mod):
         assert torch.equal(b, ones)
         hip.quantized_matmul_rows(a, Q4_K, dw, aligned, batch, rows, cols)
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("t", [Q8_0, F16, BF16, F32])
+@pytest.mark.parametrize("rows,cols", [(1, 64), (7, 96), (65, 320), (130, 512), (257, 1024), (9, 1088), (33, 2048),
+                                       (300, 4096), (5, 4160), (66, 8192), (3, 8256), (17, 12288)])
+def test_gemv_rows_any_depth(hip, oracle, torch_mod, t, rows, cols):
+    # the streaming GEMVs of Q8_0 (block pairs, 8 to 64 lanes a row, one or
+    # two pairs a lane; single blocks past 8192 columns or off 4 bytes) and of
+    # F16 / BF16 / F32 rows (one to many 16-byte chunks a lane, odd widths and
+    # rows off every alignment), with guard values around the weights, against
+    # the f64 product: f32 sums of at most K / 64 + 10 steps a lane
+    torch = torch_mod
+    shifts = [0] if t == F32 else [0, 2]
+    for d in ([cols] if t == Q8_0 else [cols, cols - 1, min(cols + 3, 12288)]):
+        w = hip.synth_random_weights(t, 300 + d, rows, d, 0.02) if t == Q8_0 else weights(t, rows, d, 300 + d)
+        x = hip.synth_normal(301, d)
+        rc, deq, _ = oracle.dequantize_slice(t, w, rows * d)
+        W = deq.reshape(rows, d).astype(np.float64)
+        ref = W @ x.astype(np.float64)
+        bound = (d / 64 + 10) * 2.0 ** -23 * (np.abs(W) @ np.abs(x.astype(np.float64)))
+        for sh in shifts:
+            buf = torch.full((w.nbytes + 64,), 0xFF, dtype=torch.uint8, device="cuda")  # NaN values around the rows
+            buf[32 + sh:32 + sh + w.nbytes].copy_(torch.from_numpy(w))
+            out = torch.full((rows + 1,), 7.0, dtype=torch.float32, device="cuda")
+            hip.quantized_matvec(out[:rows], t, buf[32 + sh:32 + sh + w.nbytes], dev(torch, x), rows, d)
+            torch.cuda.synchronize()
+            y = out.cpu().numpy()
+            assert y[-1] == 7.0
+            assert np.all(np.abs(y[:rows].astype(np.float64) - ref) <= bound + 1e-40), (d, sh)
