@@ -686,3 +686,25 @@ def test_gemv_rows_any_depth(hip, oracle, torch_mod, t, rows, cols):
             y = out.cpu().numpy()
             assert y[-1] == 7.0
             assert np.all(np.abs(y[:rows].astype(np.float64) - ref) <= bound + 1e-40), (d, sh)
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q6_K, Q8_0, F16, BF16, F32])
+@pytest.mark.parametrize("n", [1, 3, 5, 37, 33000])
+def test_dequantize_runs_of_four_at_any_alignment(hip, oracle, torch_mod, t, n):
+    # n blocks or values: the last run of dense values is short, the output
+    # starts off a 16-byte boundary, the bytes on an even one; 33000 K-quant
+    # blocks are stored past the caches
+    torch = torch_mod
+    bs, ts = (BS[t], TS[t])
+    w = weights(t, n, bs, 400 + n) if bs > 1 else weights(t, 1, n, 400 + n)
+    buf = torch.zeros(w.nbytes + 8, dtype=torch.uint8, device="cuda")
+    raw = buf[2:2 + w.nbytes]
+    raw.copy_(torch.from_numpy(w))
+    out = torch.full((n * bs + 4,), 7.5, dtype=torch.float32, device="cuda")
+    hip.dequantize_slice(t, raw, out[1:1 + n * bs])
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    rc, ref, _ = oracle.dequantize_slice(t, w, n * bs)
+    assert rc == 0
+    assert np.array_equal(got[1:1 + n * bs].view(np.uint32), ref.view(np.uint32))
+    assert got[0] == 7.5 and np.all(got[1 + n * bs:] == 7.5)
