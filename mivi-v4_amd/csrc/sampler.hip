@@ -16,7 +16,8 @@
 //   whole-row steps from the transformed row instead.
 //
 // Order statistics run as radix searches over order-preserving 32-bit keys of
-// the floats (four 8-bit passes, 256-bin histograms in LDS). Probability
+// the floats (four 8-bit passes, 256-bin histograms in LDS); a top-k of at most
+// 64 by counting ranks first (select_kth). Probability
 // masses are accumulated as 2^-40 fixed-point integers, so every bin sum and
 // prefix is exact and the result does not depend on thread timing. The draw r
 // is bit-exact with the reference; the cumulative sums it is compared against
@@ -48,6 +49,7 @@ constexpr int kKMax = 128;                // largest top_k the split path select
 constexpr int kCandVPT = 8;               // candidates per thread of the pick workgroup
 constexpr int kCapB = kST * kCandVPT;     // candidates a row may hold
 constexpr int kMaxChunks = kST;           // chunks the pick workgroup indexes
+constexpr int kSelMax = 256;              // elements the rank selection counts (select_kth)
 
 enum { kModeRow = 0, kModeGreedy = 1, kModeTopK = 2, kModeCat = 3 };
 
@@ -85,7 +87,6 @@ struct Shared {
     int wi[kSW];
     uint32_t bin;
     unsigned long long above;
-    float r;
     int found;
     float sp[64];
     int sid[64];
@@ -145,6 +146,86 @@ __device__ __forceinline__ void select_bin(const T* hist, T above, T target, uin
     }
 }
 
+// The k-th largest active key of a workgroup of NT threads, VPT keys each
+// (1 <= k <= 64, at least k active elements, active keys > 0), in four
+// barriers where the radix search takes twelve: the 64 maxima over the threads
+// t, t + 64, ... are distinct elements, so the k-th largest of them, T, bounds
+// the answer from below; the keys >= T (about 64 ln(64 / (64 - k)) of them
+// when the order is random) are gathered in LDS and ranked by counting. The
+// answer is the least key with fewer than k larger ones. False (in every
+// thread; K unset) where more than kSelMax keys reach T: ties, or the active
+// elements in fewer than k of the groups. Bound by its chain of barriers and
+// LDS round trips: eight rows of 65536 logits, default sampling (with the
+// logits' copies) 46.2 us on the radix searches, 40.4 with this in both
+// kernels and the row's zeros and generator state off the pick's chain. Called
+// at most once per kernel on one SelectShared.
+template <int NT>
+struct SelectShared {
+    __align__(16) uint32_t ck[kSelMax];
+    uint32_t tm[NT];
+    unsigned cnt;
+    uint32_t T, K;
+};
+
+__device__ __forceinline__ uint32_t wave_min(uint32_t v) {
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) v = min(v, (uint32_t)__shfl_xor(v, o, 64));
+    return v;
+}
+
+template <int NT, int VPT>
+__device__ __forceinline__ bool select_kth(const uint32_t (&key)[VPT], const bool (&act)[VPT], unsigned k,
+                                           SelectShared<NT>& s, uint32_t* K) {
+    const int t = threadIdx.x, lane = t & 63;
+    uint32_t m = 0;
+#pragma unroll
+    for (int j = 0; j < VPT; j++)
+        if (act[j]) m = max(m, key[j]);
+    s.tm[t] = m;
+    if (t < kSelMax) s.ck[t] = 0;
+    if (t == 0) { s.cnt = 0; s.K = 0xFFFFFFFFu; }
+    __syncthreads();
+    if (t < 64) {
+        uint32_t g = 0;
+#pragma unroll
+        for (int w = 0; w < NT / 64; w++) g = max(g, s.tm[t + 64 * w]);
+        unsigned larger = 0;
+#pragma unroll
+        for (int i = 0; i < 64; i++) larger += (uint32_t)__builtin_amdgcn_readlane((int)g, i) > g;
+        g = wave_min(larger < k ? g : 0xFFFFFFFFu);
+        if (t == 0) s.T = g;
+    }
+    __syncthreads();
+    const uint32_t T = s.T;
+#pragma unroll
+    for (int j = 0; j < VPT; j++) {
+        const bool in = act[j] && key[j] >= T;
+        const unsigned long long b = __ballot(in);
+        if (!b) continue;
+        const int lead = __builtin_ctzll(b);
+        unsigned at = 0;
+        if (lane == lead) at = atomicAdd(&s.cnt, (unsigned)__popcll(b));
+        at = __shfl(at, lead, 64) + (unsigned)__popcll(b & ((1ull << lane) - 1));
+        if (in && at < (unsigned)kSelMax) s.ck[at] = key[j];
+    }
+    __syncthreads();
+    const unsigned c = s.cnt;
+    if (c > (unsigned)kSelMax) return false;
+    if ((unsigned)(t & ~63) < c) {  // ck[c ..] are zero: larger than nothing
+        const uint32_t mine = s.ck[t];
+        unsigned larger = 0;
+        for (unsigned i = 0; i < c; i += 4) {
+            const uint4 v = *(const uint4*)(s.ck + i);
+            larger += (v.x > mine) + (v.y > mine) + (v.z > mine) + (v.w > mine);
+        }
+        const uint32_t lo = wave_min((unsigned)t < c && larger < k ? mine : 0xFFFFFFFFu);
+        if (lane == 0) atomicMin(&s.K, lo);
+    }
+    __syncthreads();
+    *K = s.K;
+    return true;
+}
+
 // A row as the passes see it: read and written in memory on each pass
 // (MemRow, element threadIdx.x + kST j in step j; the row stays in L2), or
 // the candidates of the split path (CandRow). each(f) calls f(i, x) for every
@@ -154,8 +235,8 @@ struct MemRow {
     float* L;
     int n;
     __device__ __forceinline__ void load(float* L_, int n_) { L = L_; n = n_; }
-    __device__ __forceinline__ void store(float*) const {}
     __device__ __forceinline__ int size() const { return n; }
+    __device__ __forceinline__ bool kth(unsigned, uint32_t*) const { return false; }
     template <class F>
     __device__ __forceinline__ void each(F f) {
         for (int i = threadIdx.x; i < n; i += kST) {
@@ -177,18 +258,19 @@ struct MemRow {
 };
 
 // The candidates of one row (list position threadIdx.x + kST j in slot j),
-// with their indices in the row; store() writes the whole row: zero outside
-// the candidates (whose probability is zero on every path through here).
+// with their indices in the row. The row in memory ends as zeros outside the
+// candidates (whose probability is zero on every path through here): clear()
+// writes the zeros, once the candidates' loads are issued, so that they drain
+// behind the selection; store(), barriers later, the candidates.
 struct CandRow {
     float v[kCandVPT];
     int id[kCandVPT];
-    int m, n;
-    bool write;
-    __device__ __forceinline__ void load(const float* cval, const int* cidx, size_t base, const int* off, int nch, int M, int n_,
-                         bool write_) {
+    int m;
+    SelectShared<kST>* sel;
+    __device__ __forceinline__ void load(const float* cval, const int* cidx, size_t base, const int* off, int nch, int M,
+                                         SelectShared<kST>* sel_) {
         m = M;
-        n = n_;
-        write = write_;
+        sel = sel_;
 #pragma unroll
         for (int j = 0; j < kCandVPT; j++) {
             const int p = (int)threadIdx.x + kST * j;
@@ -207,8 +289,7 @@ struct CandRow {
             }
         }
     }
-    __device__ __forceinline__ void store(float* L) const {
-        if (!write) return;
+    __device__ __forceinline__ void clear(float* L, int n) const {
         for (int i = 4 * threadIdx.x; i < n; i += 4 * kST) {
             if (i + 3 < n && ((uintptr_t)L & 15) == 0) {
                 *(f32x4*)(L + i) = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -216,10 +297,23 @@ struct CandRow {
                 for (int e = 0; e < 4 && i + e < n; e++) L[i + e] = 0.0f;
             }
         }
-        __syncthreads();
+    }
+    __device__ __forceinline__ void store(float* L) const {
 #pragma unroll
         for (int j = 0; j < kCandVPT; j++)
             if ((int)threadIdx.x + kST * j < m) L[id[j]] = v[j];
+    }
+    // the key of the k-th largest candidate, where the rank selection can tell
+    __device__ __forceinline__ bool kth(unsigned k, uint32_t* K) const {
+        if (k > 64) return false;
+        uint32_t key[kCandVPT];
+        bool act[kCandVPT];
+#pragma unroll
+        for (int j = 0; j < kCandVPT; j++) {
+            act[j] = (int)threadIdx.x + kST * j < m;
+            key[j] = fkey(v[j]);
+        }
+        return select_kth<kST>(key, act, k, *sel, K);
     }
     __device__ __forceinline__ int size() const { return m; }
     template <class F>
@@ -350,21 +444,23 @@ __device__ __forceinline__ uint32_t radix_search(Row& row, F f, unsigned long lo
     return prefix;
 }
 
-// sampler.rs:70-77 (thread 0), broadcast
-__device__ __forceinline__ float draw(unsigned long long* rng, Shared& sh) {
-    if (threadIdx.x == 0) {
-        unsigned long long s = *rng;
-        s ^= s >> 12;
-        s ^= s << 25;
-        s ^= s >> 27;
-        *rng = s;
-        const unsigned long long r = (s * 0x2545F4914F6CDD1DULL) >> 32;
-        sh.r = (float)(r >> 8) / 16777216.0f;
-    }
-    __syncthreads();
-    const float r = sh.r;
-    __syncthreads();
-    return r;
+// A row's generator: the state every thread loaded before the kernel's first
+// barrier (a load at the draw itself is a memory round trip in the middle of
+// the chain), and where thread 0 stores the next one.
+struct Rng {
+    unsigned long long s;
+    unsigned long long* p;
+};
+
+// sampler.rs:70-77; at least one barrier after the state's load
+__device__ __forceinline__ float draw(const Rng& rng) {
+    unsigned long long s = rng.s;
+    s ^= s >> 12;
+    s ^= s << 25;
+    s ^= s >> 27;
+    if (threadIdx.x == 0) *rng.p = s;
+    const unsigned long long r = (s * 0x2545F4914F6CDD1DULL) >> 32;
+    return (float)(r >> 8) / 16777216.0f;
 }
 
 // Wave 0 finishes a draw over s <= 64 elements (probability sp[l], index
@@ -435,10 +531,10 @@ __device__ __forceinline__ void compact_small(Row& row, M match, int pos, Shared
 }
 
 // Steps 4-7 of Sampler::sample over a row already penalised and divided by
-// the temperature: min-p, top-k, softmax (the probabilities written back to
-// L), then top-p or categorical. n is the length of the whole row.
+// the temperature: min-p, top-k, softmax (the row ends holding the
+// probabilities), then top-p or categorical. n is the length of the whole row.
 template <class Row>
-__device__ __forceinline__ int sample_tail(Row& row, float* L, int n, const SampleArgs& c, unsigned long long* rng, Shared& sh) {
+__device__ __forceinline__ int sample_tail(Row& row, int n, const SampleArgs& c, const Rng& rng, Shared& sh) {
     // 4. min-p (sampler.rs:260-276); ln(min_p) comes from the host's libm
     if (c.min_p > 0.0f && c.min_p < 1.0f) {
         const float mx = bmax_finite(row, sh);
@@ -453,10 +549,13 @@ __device__ __forceinline__ int sample_tail(Row& row, float* L, int n, const Samp
     // Over candidates holding fewer than k elements every finite logit is a
     // candidate and the cutoff is -inf: nothing to mask.
     if (c.top_k > 0 && c.top_k < n && c.top_k <= row.size()) {
-        unsigned long long above;
-        const uint32_t K = radix_search(
-            row, [&](int, float x, uint32_t& k, unsigned long long& w) { k = fkey(x); w = 1; return true; },
-            (unsigned long long)c.top_k, &above, sh);
+        uint32_t K;
+        if (!row.kth((unsigned)c.top_k, &K)) {
+            unsigned long long above;
+            K = radix_search(
+                row, [&](int, float x, uint32_t& k, unsigned long long& w) { k = fkey(x); w = 1; return true; },
+                (unsigned long long)c.top_k, &above, sh);
+        }
         const float cutoff = funkey(K);
         row.each([&](int, float& x) {
             if (x < cutoff) x = -INFINITY;
@@ -488,8 +587,6 @@ __device__ __forceinline__ int sample_tail(Row& row, float* L, int n, const Samp
             }
         }
     }
-    row.store(L);
-    __syncthreads();
     if (c.top_p < 1.0f) {
         // 7a. top-p (sampler.rs:150-215)
         const float cutoff = n > 1 ? (1.0f - c.top_p) / ((float)n - 1.0f) : 0.0f;
@@ -512,7 +609,8 @@ __device__ __forceinline__ int sample_tail(Row& row, float* L, int n, const Samp
         if (nh <= 64) {
             // few candidates carry mass (top-k left few): one wave finishes
             compact_small(row, heavy, (int)ph, sh);
-            const float r = draw(rng, sh);
+            __syncthreads();
+            const float r = draw(rng);
             if (threadIdx.x < 64) {
                 const int t = wave_pick(sh, (int)nh, true, c.top_p, r, n);
                 if (threadIdx.x == 0) sh.found = t;
@@ -542,7 +640,7 @@ __device__ __forceinline__ int sample_tail(Row& row, float* L, int n, const Samp
             nmass = above + t * ws;
         }
         const float mass = (float)((double)nmass / kFix);
-        const float r = draw(rng, sh) * mass;
+        const float r = draw(rng) * mass;
         unsigned long long tr = (unsigned long long)ceil((double)r * kFix);
         tr = tr ? tr : 1;
         tr = tr < nmass ? tr : nmass;
@@ -579,7 +677,8 @@ __device__ __forceinline__ int sample_tail(Row& row, float* L, int n, const Samp
         unsigned long long nh;
         const unsigned long long ph = bscan_excl<kSW, unsigned long long>(hv, &nh, sh.wsum);
         if (nh <= 64) compact_small(row, heavy, (int)ph, sh);
-        const float r = draw(rng, sh);
+        __syncthreads();
+        const float r = draw(rng);
         const unsigned long long tr = (unsigned long long)ceil((double)r * kFix);
         if (tr == 0 || n == 0) return 0;
         if (tot < tr) return n - 1;
@@ -612,7 +711,7 @@ __device__ __forceinline__ int sample_tail(Row& row, float* L, int n, const Samp
 // kernel did it). The passes run over `row` (Row::load takes L), which ends
 // holding the probabilities, written back to L as the reference leaves them.
 template <class Row, bool PRE, class R>
-__device__ __forceinline__ int sample_body(float* L, int n, const R& recent, const SampleArgs& c, unsigned long long* rng,
+__device__ __forceinline__ int sample_body(float* L, int n, const R& recent, const SampleArgs& c, const Rng& rng,
                            Shared& sh) {
     const int tid = threadIdx.x;
     const int nr = recent.n;
@@ -642,12 +741,12 @@ __device__ __forceinline__ int sample_body(float* L, int n, const R& recent, con
         const float inv_t = 1.0f / c.temperature;
         row.each([&](int, float& x) { x *= inv_t; });
     }
-    return sample_tail(row, L, n, c, rng, sh);
+    return sample_tail(row, n, c, rng, sh);
 }
 
 template <bool PRE, class R>
 __device__ __forceinline__ int sample_row(float* L, int n, const R& recent, const SampleArgs& c,
-                                          unsigned long long* rng, Shared& sh) {
+                                          const Rng& rng, Shared& sh) {
     return sample_body<MemRow, PRE>(L, n, recent, c, rng, sh);
 }
 
@@ -695,6 +794,7 @@ struct ChunkShared {
     int wi[kCW];
     uint32_t bin;
     unsigned above;
+    SelectShared<kCT> sel;
 };
 
 // The split path's chunk kernel: chunk blockIdx.x (kCC logits) of row
@@ -819,7 +919,7 @@ __global__ void __launch_bounds__(kCT) sample_chunk_kernel(float* logits, int64_
     unsigned nfin;
     bscan_excl<kCW>(nf, &nfin, sh.wtot);
     uint32_t K = 0;
-    if (nfin > k) {
+    if (nfin > k && !(k <= 64 && select_kth<kCT>(key, ok, k, sh.sel, &K))) {
         uint32_t prefix = 0, pmask = 0;
         unsigned above = 0;
         for (int pass = 0; pass < 4; pass++) {
@@ -957,18 +1057,20 @@ __global__ void __launch_bounds__(kST) sample_pick_kernel(float* logits, int64_t
                                                           const int* ccount, unsigned long long* rng, TokOut out,
                                                           int write) {
     __shared__ Shared sh;
+    __shared__ SelectShared<kST> sel;
     const int t = threadIdx.x, b = blockIdx.x;
     float* L = logits + (int64_t)b * lstride;
+    const Rng rs{rng[b], rng + b};
     if (mode == kModeCat) {
         // 7b. categorical (sampler.rs:137-148) over the probabilities the
         // chunk kernels left: the chunk where the fixed-point mass reaches
         // r, then the index inside it
-        const float r = draw(rng + b, sh);
-        const unsigned long long tr = (unsigned long long)ceil((double)r * kFix);
         const unsigned long long cm =
             t < nch ? *(const unsigned long long*)(cidx + ((size_t)b * nch + t) * kCapC) : 0ull;
         unsigned long long tot;
         const unsigned long long ex = bscan_excl<kSW, unsigned long long>(cm, &tot, sh.wsum);
+        const float r = draw(rs);
+        const unsigned long long tr = (unsigned long long)ceil((double)r * kFix);
         if (t == 0) sh.bin = 0;
         __syncthreads();
         if (t < nch && cm && ex < tr && tr <= ex + cm) {
@@ -1015,11 +1117,17 @@ __global__ void __launch_bounds__(kST) sample_pick_kernel(float* logits, int64_t
     }
     int tok;
     if (!fast) {
-        tok = sample_row<true>(L, n, NoRecent{}, c, rng + b, sh);
+        tok = sample_row<true>(L, n, NoRecent{}, c, rs, sh);
     } else {
         CandRow row;
-        row.load(cval, cidx, (size_t)b * nch * kCapC, sh.off, nch, M, n, write != 0);
-        tok = mode == kModeGreedy ? bargmax(row, sh) : sample_tail(row, L, n, c, rng + b, sh);
+        row.load(cval, cidx, (size_t)b * nch * kCapC, sh.off, nch, M, &sel);
+        if (mode == kModeGreedy) {
+            tok = bargmax(row, sh);
+        } else {
+            if (write) row.clear(L, n);
+            tok = sample_tail(row, n, c, rs, sh);
+            if (write) row.store(L);
+        }
     }
     if (t == 0) {
         out.tok[b] = (uint32_t)tok;

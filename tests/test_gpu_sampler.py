@@ -208,6 +208,20 @@ def test_rows_ties(hip, oracle, torch_mod, scale):
     run_pair(hip, oracle, torch_mod, logits, [], cfg, 17, 16, "rows")
 
 
+@pytest.mark.parametrize("top_k", [1, 2, 40, 64, 65])
+@pytest.mark.parametrize("n,groups", [(66, 64), (1025, 64), (70001, 64), (65536, 32), (9000, 1)])
+def test_rank_selection_edges(hip, oracle, torch_mod, n, groups, top_k):
+    """The rank selection of the top-k cutoff at the smallest k, its largest
+    (64; 65 takes the radix search), and with finite logits in 32 or one of the
+    64 thread groups its lower bound comes from (fewer groups than top_k: the
+    bound falls to zero and, with 32, more keys reach it than are ranked)."""
+    rng = np.random.default_rng(n + top_k)
+    logits = (rng.standard_normal(n) * 3).astype(np.float32)
+    logits[(np.arange(n) // 4) % 64 >= groups] = -np.inf
+    cfg = dict(temperature=0.8, top_p=0.95, top_k=top_k)
+    run_pair(hip, oracle, torch_mod, logits, [], cfg, 31 + top_k, 8, "rows")
+
+
 @pytest.mark.parametrize("name", ["default", "categorical", "greedy_penalised", "min_p_top_k"])
 def test_rows_batch_independent(hip, oracle, torch_mod, name):
     """Three rows at once, each with its own logits, window and state, against
