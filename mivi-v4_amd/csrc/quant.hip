@@ -497,9 +497,10 @@ typedef uint32_t u32x4_a1 __attribute__((ext_vector_type(4), aligned(1)));
 // batch (K <= 64 * NJ chunks) keep their inputs in registers. ODD: K not a
 // whole number of chunks; rows then start on any 2-byte boundary, where a
 // 16-byte load splits (three times the time), so the 16-bit kinds load aligned
-// dwords and shift, and the last K % CW values come one to a lane. Four sums a
-// lane and row keep the f32 chains short.
-template <int KIND, int R, int NJ, bool ODD, int PRO>
+// dwords and shift (ODD 2, weights on an odd byte: the split loads), and the
+// last K % CW values come one to a lane. Four sums a lane and row keep the f32
+// chains short.
+template <int KIND, int R, int NJ, int ODD, int PRO>
 __global__ void __launch_bounds__(kWG) gemv_rows_kernel(const mivi::GemvArgs a) {
     extern __shared__ float lds[];
     stage_input<PRO, 0>(lds, a);
@@ -526,7 +527,7 @@ __global__ void __launch_bounds__(kWG) gemv_rows_kernel(const mivi::GemvArgs a) 
                     const bool in = k < KF;
                     const uint8_t* p = row + (size_t)(in ? k : 0) * EB;
                     u32x4 v;
-                    if constexpr (ODD && EB == 2) v = ld16_a2(p);
+                    if constexpr (ODD == 1 && EB == 2) v = ld16_a2(p);
                     else v = *(const u32x4_a1*)p;
                     B.w[r][j] = in ? v : u32x4{0u, 0u, 0u, 0u};
                 }
@@ -3724,6 +3725,8 @@ int32_t launch_pro(int32_t t, const mivi::GemvArgs& a, int n, hipStream_t s) {
         const int cw = t == MIVI_GGML_F32 ? 4 : 8;
         const int nj = (K + 64 * cw - 1) / (64 * cw);
         const bool odd = K % cw != 0;
+        bool even = true;  // (rows on odd bytes: ld16_a2 needs even ones)
+        for (int i = 0; i < a.nseg; i++) even = even && (uintptr_t)a.seg[i].W % 2 == 0;
         // rows of up to two chunks a lane in groups of four, up to four
         // chunks in pairs, longer ones alone: eight loads a batch each way
         const int R = nj <= 2 ? 4 : nj <= 4 ? 2 : 1;
@@ -3734,9 +3737,13 @@ int32_t launch_pro(int32_t t, const mivi::GemvArgs& a, int n, hipStream_t s) {
 #define LR(KIND, R, NJ, ODD) hipLaunchKernelGGL((gemv_rows_kernel<KIND, R, NJ, ODD, PRO>), dim3(grid), dim3(kWG), lds, s, a)
 #define LRS(KIND, ODD) \
     if (R == 4) LR(KIND, 4, 2, ODD); else if (R == 2) LR(KIND, 2, 4, ODD); else LR(KIND, 1, 8, ODD)
-        if (t == MIVI_GGML_F16) { if (odd) { LRS(RK_F16, true); } else { LRS(RK_F16, false); } }
-        else if (t == MIVI_GGML_BF16) { if (odd) { LRS(RK_BF16, true); } else { LRS(RK_BF16, false); } }
-        else { if (odd) { LRS(RK_F32, true); } else { LRS(RK_F32, false); } }
+#define LRK(KIND) \
+    if (!odd) { LRS(KIND, 0); } else if (even) { LRS(KIND, 1); } else { LRS(KIND, 2); }
+        if (t == MIVI_GGML_F16) { LRK(RK_F16) }
+        else if (t == MIVI_GGML_BF16) { LRK(RK_BF16) }
+        else if (odd) { LRS(RK_F32, 1); }
+        else { LRS(RK_F32, 0); }
+#undef LRK
 #undef LRS
 #undef LR
         break;

@@ -124,6 +124,22 @@ def test_gemv_unaligned_f32_rows(hip, oracle, torch_mod):
     check_bound(oracle, F32, W.view(np.uint8).reshape(-1), x, out.cpu().numpy(), rows, cols)
 
 
+@pytest.mark.parametrize("t", [F16, BF16])
+@pytest.mark.parametrize("cols", [51, 1003, 2055, 4099])
+def test_gemv_rows_on_odd_bytes(hip, oracle, torch_mod, t, cols):
+    # 16-bit rows of odd widths that start on an odd byte
+    torch = torch_mod
+    rows = 9
+    w = weights(t, rows, cols, 8)
+    buf = torch.zeros(w.nbytes + 33, dtype=torch.uint8, device="cuda")
+    buf[17:17 + w.nbytes].copy_(torch.from_numpy(w))
+    x = np.random.default_rng(2).standard_normal(cols).astype(np.float32)
+    out = torch.empty(rows, dtype=torch.float32, device="cuda")
+    hip.quantized_matvec(out, t, buf[17:17 + w.nbytes], dev(torch, x), rows, cols)
+    torch.cuda.synchronize()
+    check_bound(oracle, t, w, x, out.cpu().numpy(), rows, cols)
+
+
 @pytest.mark.parametrize("fn,t", [("try_matvec_q4_k_m", Q4_K), ("try_matvec_q6_k", Q6_K), ("try_matvec_q8_0", Q8_0),
                                   ("try_matvec_f16", F16), ("try_matvec_bf16", BF16)])
 def test_typed_entry_points(hip, oracle, torch_mod, fn, t):
