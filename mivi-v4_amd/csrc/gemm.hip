@@ -934,10 +934,8 @@ struct RowsTile {
 static RowsTile rows_tile(int32_t t, const GemvArgs& a, int mtiles) {
     RowsTile best = {4, 0};
     double least = 0;
-    static const int env_wn = env_knob("MIVI_ROWS_WN", 0);
     const int wide = (t == MIVI_GGML_Q4_K || t == MIVI_GGML_Q6_K) && a.K % 2048 == 0 ? 4 : 1;
     for (int wn = wide; wn >= 1; wn /= 2) {
-        if (env_wn && wn != env_wn && wide > 1) continue;
         int nt = 0;
         if (a.epilogue == EPI_SWIGLU) nt = (a.seg[0].n + 32 * wn - 1) / (32 * wn);
         else
