@@ -599,11 +599,13 @@ def _rows_case(hip, t, batch, rows, cols):
 
 @pytest.mark.parametrize("t", [Q4_K, Q6_K, Q8_0, F16, BF16])
 @pytest.mark.parametrize("batch,rows,cols", [(6, 1, 1024), (6, 63, 1280), (31, 65, 1024), (33, 200, 1792), (64, 129, 1536),
-                                             (65, 257, 4608), (8, 64, 10240), (97, 300, 2304), (32, 64, 12288)])
+                                             (65, 257, 4608), (8, 64, 10240), (97, 300, 2304), (32, 64, 12288),
+                                             (97, 4160, 1024)])
 def test_matmul_rows_matrix_cores_any_depth(hip, oracle, torch_mod, t, batch, rows, cols):
     # the row products at depths with one GEMV launch per input (from a few
     # inputs on): every weight format, tile edges in both directions, shares
-    # of the depth without a super-block, inputs from 1e-30 to 1e30; each
+    # of the depth without a super-block, tiles of 64 inputs (the last shape:
+    # they fill half of the CUs) and of 32, inputs from 1e-30 to 1e30; each
     # output within a tenth of the bar of the f64 product of the stored
     # weights (f32 sums and a 24-bit split of the inputs)
     torch = torch_mod
