@@ -7,7 +7,7 @@ projection through one type dispatch (crates/mivi-quant/src/lib.rs:89-131,
 143-357), and so does this build: here the one-column decode GEMVs stream
 the Q6_K projections packed (row quads at 2048 columns, unit planes at
 8192), q|k and the Q6_K v run as two launches, and the chunked prefill runs
-the Q6_K products on the matrix cores (gemm_q6k_kernel). The model below
+the Q6_K products on the matrix cores (gemm_rows_kernel). The model below
 has dim 2048 and hidden 8192, so every one of those paths is the one the
 1.2B shape takes.
 
