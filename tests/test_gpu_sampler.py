@@ -222,6 +222,18 @@ def test_rank_selection_edges(hip, oracle, torch_mod, n, groups, top_k):
     run_pair(hip, oracle, torch_mod, logits, [], cfg, 31 + top_k, 8, "rows")
 
 
+@pytest.mark.parametrize("name", ["greedy_penalised", "min_p_top_k"])
+@pytest.mark.parametrize("window", [255, 257, 1100])
+def test_long_penalty_windows(hip, oracle, torch_mod, name, window):
+    # windows around and past a chunk workgroup's threads, ids repeated and
+    # beyond the row, over a partial last chunk
+    n = 2051
+    rng = np.random.default_rng(window)
+    logits = (rng.standard_normal(n) * 3).astype(np.float32)
+    recent = np.minimum(rng.integers(0, n + 50, window), rng.integers(0, n + 50, window)).tolist()
+    run_pair(hip, oracle, torch_mod, logits, recent, CONFIGS[name], 77, 4, "rows")
+
+
 @pytest.mark.parametrize("name", ["default", "categorical", "greedy_penalised", "min_p_top_k"])
 def test_rows_batch_independent(hip, oracle, torch_mod, name):
     """Three rows at once, each with its own logits, window and state, against
