@@ -1241,6 +1241,10 @@ __global__ void __launch_bounds__(64, 2) attn_f16_mfma_kernel(AttnArgs a) {
 // (V's block scale), whose range fp16 does not cover, enters as three bf16
 // parts. F32: every operand as three bf16 parts, the products up to 2^-24.
 // The softmax reference moves only when a maximum exceeds it by 2^8.
+// A product of parts cannot carry an infinity or NaN (0 * inf, and a masked
+// token's p = 0 against its V): tiles that hold one in K or V (or, with F32
+// caches, whose query does) form their scores and values in f32, token by
+// token, only over the tokens each row sees.
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
@@ -1265,6 +1269,13 @@ __device__ __forceinline__ void split_bf16(float v, __bf16& b0, __bf16& b1, __bf
     b2 = (__bf16)(r - (float)b1);
 }
 
+// value e of eight 16-bit ones
+template <bool BF>
+__device__ __forceinline__ float part_f32(const u32x4& w, int e) {
+    const uint32_t b = w[e >> 1] >> (16 * (e & 1));
+    return BF ? __uint_as_float(b << 16) : half_bits_to_f32(b);
+}
+
 template <bool BF>
 __device__ __forceinline__ f32x16_t mfma32(const u32x4& a, const u32x4& b, const f32x16_t& c) {
     if constexpr (BF)
@@ -1274,7 +1285,7 @@ __device__ __forceinline__ f32x16_t mfma32(const u32x4& a, const u32x4& b, const
 }
 
 template <int KVP>
-__global__ void __launch_bounds__(256, 1) attn_prefill_kernel(AttnArgs a, int pos0, int rows, int nrb, int tsplit,
+__global__ void __launch_bounds__(256, KVP == MIVI_KV_F32 ? 1 : 2) attn_prefill_kernel(AttnArgs a, int pos0, int rows, int nrb, int tsplit,
                                                               float* out, int64_t out_s) {
     constexpr bool F32C = KVP == MIVI_KV_F32, Q8 = KVP == MIVI_KV_Q8_0;
     constexpr int KP = F32C ? 3 : 1;              // planes of K and of V in LDS
@@ -1285,6 +1296,7 @@ __global__ void __launch_bounds__(256, 1) attn_prefill_kernel(AttnArgs a, int po
     constexpr int SCB = Q8 ? 2 * 2 * kPfTokens * 4 : 0;  // K's and V's block scales
     constexpr int BUF = KP * (KB + VB) + SCB;
     __shared__ __attribute__((aligned(16))) uint8_t smem[2 * BUF > 4 * kPfRows * 272 ? 2 * BUF : 4 * kPfRows * 272];
+    __shared__ __attribute__((aligned(16))) uint32_t odd[2][4];  // per LDS tile and loading wave: an infinity or NaN in it
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int li = lane & 31, lh = lane >> 5;
     const int hpk = a.n_heads / a.n_kv_heads, nblk = max(1, 4 / hpk);
@@ -1387,6 +1399,21 @@ __global__ void __launch_bounds__(256, 1) attn_prefill_kernel(AttnArgs a, int po
             }
         }
     };
+    // whether the thread's part of the loaded tile holds an infinity or NaN
+    // (an exponent of all ones), Q8_0: in V's block scales (K's are f32 factors)
+    auto nonfinite = [&]() -> bool {
+        constexpr uint32_t E = F32C ? 0x7F800000u : 0x7C007C00u, ONE = F32C ? 0x00800000u : 0x04000400u;
+        uint32_t any = 0;
+        if constexpr (Q8) {
+            any = (rdv & E) + ONE;
+        } else {
+#pragma unroll
+            for (int k = 0; k < LC; k++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) any |= ((rk[k][i] & E) + ONE) | ((rv[k][i] & E) + ONE);
+        }
+        return any & (F32C ? 0x80000000u : 0x80008000u);
+    };
     if (t0 < t1) load_tile(t0);
 
     // the lane's query: dims 16 s + 8 lh .. + 7 of each k-step s, per-head
@@ -1394,6 +1421,7 @@ __global__ void __launch_bounds__(256, 1) attn_prefill_kernel(AttnArgs a, int po
     // wave_prep_head, in log2 units, as the planes of the B operand
     u32x4 qa[4][QP];
     float qinv = 1.0f;
+    bool qodd = false;  // F32: an infinity or NaN in a query of the wave
     {
         const float* qp = a.q + (int64_t)row * a.qkv_s + (size_t)head * 64;
         const float* cs = a.rope_cos + (size_t)pos * 32;
@@ -1429,6 +1457,14 @@ __global__ void __launch_bounds__(256, 1) attn_prefill_kernel(AttnArgs a, int po
                 v[s][e + 1] = (x0 * n + x1 * c) * qscale;
                 mx = fmaxf(mx, fmaxf(fabsf(v[s][e]), fabsf(v[s][e + 1])));
             }
+        if constexpr (F32C) {
+            float z = 0.f;  // 0 * x summed: 0 unless an x is infinite or NaN
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) z = fmaf(v[s][e], 0.f, z);
+            qodd = __builtin_amdgcn_ballot_w64(z != 0.f) != 0;
+        }
         if constexpr (!SB) {
             // the largest value into [2^9, 2^10): lo parts clear of denormals,
             // the sums of 64 products with fp16 keys within f32
@@ -1447,7 +1483,7 @@ __global__ void __launch_bounds__(256, 1) attn_prefill_kernel(AttnArgs a, int po
                 for (int k = 0; k < 8; k++) {
                     const float y = v[s][k] * f;
                     h[k] = (_Float16)y;
-                    l[k] = (_Float16)(y - (float)h[k]);
+                    l[k] = fabsf(y) <= 3.40282347e38f ? (_Float16)(y - (float)h[k]) : (_Float16)0.0f;
                 }
                 qa[s][0] = __builtin_bit_cast(u32x4, h);
                 qa[s][1] = __builtin_bit_cast(u32x4, l);
@@ -1476,8 +1512,12 @@ __global__ void __launch_bounds__(256, 1) attn_prefill_kernel(AttnArgs a, int po
     for (int t = t0; t < t1; t += kPfTokens) {
         uint8_t* b = smem + buf * BUF;
         store_tile(b);
+        const uint64_t mine = __builtin_amdgcn_ballot_w64(nonfinite());
+        if (lane == 0) odd[buf][wave] = mine != 0;
         if (t + kPfTokens < t1) load_tile(t + kPfTokens);
         __syncthreads();  // (the buffer's readers of two tiles ago are past the last one)
+        const u32x4 ow = *(const u32x4*)odd[buf];
+        const bool kvodd = __builtin_amdgcn_readfirstlane(ow.x | ow.y | ow.z | ow.w) != 0;
         buf ^= 1;
         // rows below the tile have nothing in it (wave-uniform)
         if (!used || t > pos0 + min(row0 + kPfRows, rows) - 1) continue;
@@ -1509,6 +1549,37 @@ __global__ void __launch_bounds__(256, 1) attn_prefill_kernel(AttnArgs a, int po
                     s[16 * u + r] = fmaf(scl[kPfTokens + tk], c[1][r], scl[tk] * c[0][r]);
                 } else {
                     s[16 * u + r] = c[0][r];
+                }
+            }
+        }
+        if constexpr (!Q8) {
+            if (kvodd || qodd) {  // (wave-uniform)
+                // the score of token tk: the lane half's 32 dims, then both
+                // halves; into its register in the half that holds it
+#pragma unroll 1
+                for (int tk = 0; tk < kPfTokens; tk++) {
+                    float part = 0.f;
+#pragma unroll
+                    for (int st = 0; st < 4; st++) {
+                        u32x4 kp[KP];
+#pragma unroll
+                        for (int p = 0; p < KP; p++) kp[p] = *(const u32x4*)(kb + p * KB + koff(tk, 2 * st + lh));
+#pragma unroll
+                        for (int e = 0; e < 8; e++) {
+                            float q = 0.f, k = 0.f;
+#pragma unroll
+                            for (int p = QP - 1; p >= 0; p--) q += part_f32<SB>(qa[st][p], e);
+#pragma unroll
+                            for (int p = KP - 1; p >= 0; p--) k += part_f32<SB>(kp[p], e);
+                            part = fmaf(q, k, part);
+                        }
+                    }
+                    float lo, hi;
+                    swap32(part, lo, hi);
+                    const float sum = lo + hi;
+                    const int at = ((tk >> 2) & 1) == lh ? 16 * (tk >> 5) + 4 * ((tk >> 3) & 3) + (tk & 3) : -1;
+#pragma unroll
+                    for (int k = 0; k < 32; k++) s[k] = k == at ? sum : s[k];
                 }
             }
         }
@@ -1546,6 +1617,38 @@ __global__ void __launch_bounds__(256, 1) attn_prefill_kernel(AttnArgs a, int po
         for (int k = 0; k < 32; k++) {
             s[k] = __builtin_amdgcn_exp2f(s[k] - mr);
             l_run += s[k];
+        }
+        if (kvodd) {
+            // 3'. token by token, as far as the row sees
+#pragma unroll 1
+            for (int tk = 0; tk < kPfTokens; tk++) {
+                const int at = 16 * (tk >> 5) + 4 * ((tk >> 3) & 3) + (tk & 3);
+                float w = 0.f;
+#pragma unroll
+                for (int k = 0; k < 32; k++) w = k == at ? s[k] : w;
+                float lo, hi;
+                swap32(w, lo, hi);
+                w = (tk >> 2) & 1 ? hi : lo;
+                const bool seen = t + tk <= pos;
+#pragma unroll
+                for (int d = 0; d < 2; d++)
+#pragma unroll
+                    for (int g = 0; g < 4; g++) {
+                        u32x2 vp[KP];
+#pragma unroll
+                        for (int p = 0; p < KP; p++)
+                            vp[p] = *(const u32x2*)(vb + p * VB + tk * kPfVRow + 2 * (32 * d + 8 * g + 4 * lh));
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            float v = 0.f;
+#pragma unroll
+                            for (int p = KP - 1; p >= 0; p--) v += part_f32<PB>(u32x4{vp[p].x, vp[p].y, 0u, 0u}, e);
+                            if constexpr (Q8) v *= scl[(2 + d) * kPfTokens + tk];
+                            o[d][4 * g + e] = seen ? fmaf(w, v, o[d][4 * g + e]) : o[d][4 * g + e];
+                        }
+                    }
+            }
+            continue;
         }
         // 3. O^T += V^T P^T, 16 tokens at a time
 #pragma unroll
@@ -1605,13 +1708,15 @@ __global__ void __launch_bounds__(256, 1) attn_prefill_kernel(AttnArgs a, int po
     constexpr int OR = 68;  // floats of a row in LDS
     float* ot = (float*)smem + wave * kPfRows * OR;
     const bool whole = a.nsplit == 1;
-    const float f = whole ? (l_run > 0.f ? 1.0f / l_run : 0.f) : 1.0f;
+    const float f = whole ? 1.0f / l_run : 1.0f;
+    const bool none = whole && !(l_run > 0.f);  // (no weight, or NaN: zeros, as the decode's merge gives)
 #pragma unroll
     for (int d = 0; d < 2; d++)
 #pragma unroll
-        for (int g = 0; g < 4; g++)
-            *(f32x4*)(ot + li * OR + 32 * d + 8 * g + 4 * lh) =
-                f32x4{o[d][4 * g] * f, o[d][4 * g + 1] * f, o[d][4 * g + 2] * f, o[d][4 * g + 3] * f};
+        for (int g = 0; g < 4; g++) {
+            const f32x4 v = {o[d][4 * g] * f, o[d][4 * g + 1] * f, o[d][4 * g + 2] * f, o[d][4 * g + 3] * f};
+            *(f32x4*)(ot + li * OR + 32 * d + 8 * g + 4 * lh) = none ? f32x4{0.f, 0.f, 0.f, 0.f} : v;
+        }
     __syncthreads();
     if (!used) return;
     const int r4 = lane >> 4, c4 = lane & 15;  // four rows of 16 chunks a pass

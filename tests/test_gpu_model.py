@@ -632,3 +632,77 @@ def test_prefill_tile_attention_matches_per_row_attention(hip, n_heads, n_kv, pr
             x, y = x.view(dt).astype(np.float64), y.view(dt).astype(np.float64)
             assert np.max(np.abs(x - y)) <= step * np.max(np.abs(x))
         assert np.max(np.abs(ca - cb)) <= 1e-4 * np.max(np.abs(ca))
+
+
+def _patch_f32(img, name, f):
+    """img with the F32 matrix `name` ([rows, cols]) changed in place by f."""
+    from mivi_hip.gguf import read_tensor_index
+    t, dims, off, n = read_tensor_index(img)[name]
+    m = np.frombuffer(img[off:off + n].tobytes(), np.float32).reshape(dims[1], dims[0]).copy()
+    f(m)
+    img[off:off + n] = np.frombuffer(m.tobytes(), np.uint8)
+
+
+@pytest.mark.parametrize("prec,part,big,small", [(2, "v", 3600.0, 1e-4), (0, "v", 1.6e37, 1e-36), (1, "v", 4e5, 1e-6),
+                                                 (0, "k", 1.6e37, 1.0)])
+def test_prefill_tile_attention_infinite_keys_and_values(hip, prec, part, big, small):
+    # one prompt token whose V (K) overflows the cache's precision in one dim
+    # of one kv head: the rows before it never see it (a masked token's p = 0
+    # times an infinity must not reach them), the rows from it on give what the
+    # per-row kernels (tiles of 32) give: infinities that end as NaN behind the
+    # next norm, or, for an infinite key, scores of -inf (no weight) or +inf
+    from mivi_hip import GgmlType
+    from mivi_hip.synthmodel import build_hybrid
+    dim, n_heads, n_kv, at, n = 768, 12, 4, 70, 100
+    img = build_hybrid(dim=dim, hidden=512, n_layers=3, attn_layers=(0, 2), n_heads=n_heads, n_kv=n_kv, vocab=256,
+                       ctx_len=512, seed=51, weight_type=GgmlType.F32, embd_type=GgmlType.F32)
+    rng = np.random.default_rng(52)
+    sign = np.where(rng.random(dim) < 0.5, -1.0, 1.0).astype(np.float32)
+
+    def embd(m):
+        m[7] = 0.02 * sign
+
+    def proj(m):  # row 5 of kv head 1, along token 7's embedding
+        m[64 + 5] = np.float32(big / np.sqrt(dim)) * sign
+
+    def wo(m):  # the overflowing dim's share of the other tokens back to their size
+        for h in range(3, 6):
+            m[:, 64 * h + 5] *= np.float32(small)
+
+    _patch_f32(img, "token_embd.weight", embd)
+    _patch_f32(img, f"blk.0.attn_{part}.weight", proj)
+    if part == "v":
+        _patch_f32(img, "blk.0.attn_output.weight", wo)
+    prompt = rng.integers(8, 256, n)
+    other = prompt.copy()
+    prompt[at] = 7
+
+    def run(tokens, tile):
+        m = hip.Model(img, max_ctx=512, kv_precision=prec)
+        m.set_prefill_strategy(tile)
+        m.prefill(tokens, 0)
+        k, v, _ = m.export_state(n)
+        row = m.kv_row_bytes()
+        return [x.reshape(2, n, row) for x in (k, v)]
+
+    a, ref, b = run(prompt, 128), run(prompt, 32), run(other, 128)
+    dt = {0: np.float32, 2: np.float16}.get(prec)
+    first = (a[1] if part == "v" else a[0])[0, at]
+    if dt:
+        assert np.isinf(first.view(dt)).any()
+    else:
+        assert np.isinf(first.reshape(-1, 34)[:, :2].copy().view(np.float16)).any()
+    for x, r, y in zip(a, ref, b):
+        assert np.array_equal(x[1, :64], y[1, :64])
+        if dt is None:
+            assert q8_rows_close(x[1, 64:at].reshape(-1), y[1, 64:at].reshape(-1), at - 64, 1, x.shape[2])
+            continue
+        xf, rf, yf = (z[1].copy().view(dt).astype(np.float64) for z in (x, r, y))
+        tol = 2e-5 if prec == 0 else 1e-3  # f32 rounding; one fp16 step
+        assert np.max(np.abs(xf[:at] - yf[:at])) <= tol * np.max(np.abs(yf[:at]))
+        assert np.array_equal(np.isnan(xf[at:]), np.isnan(rf[at:]))
+        fin = np.isfinite(rf[at:])
+        assert np.array_equal(fin, np.isfinite(xf[at:]))
+        if part == "k":
+            assert fin.all()
+            assert np.max(np.abs(xf[at:] - rf[at:])) <= tol * np.max(np.abs(rf[at:]))
