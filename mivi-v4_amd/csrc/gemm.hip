@@ -396,6 +396,13 @@ __device__ __forceinline__ f32x16 mfma16(const u32x4& a, const u32x4& b, const f
         return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0, 0);
 }
 
+// value e of eight fp16 or bf16 ones
+template <bool BF>
+__device__ __forceinline__ float part16_f32(const u32x4& w, int e) {
+    const uint32_t b = w[e >> 1] >> (16 * (e & 1));
+    return BF ? bf16_bits_to_f32(b) : half_bits_to_f32(b);
+}
+
 typedef uint32_t u32x4_a2g __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t u32x2_a2g __attribute__((ext_vector_type(2), aligned(2)));
 
@@ -835,6 +842,52 @@ __global__ void __launch_bounds__(256, 1) gemm_rows_kernel(const RowsArgs a) {
                 }
             }
         }
+    if constexpr (FMT == RF_F16 || BF) {
+        // An infinite weight times a lo part (0, or of the other sign) is NaN
+        // where the value itself gives an infinity: outputs that came out
+        // infinite or NaN are summed again in f32 from whole weights and
+        // inputs, one per lane at a time (ordinary data: none; the test costs
+        // 0.2 us of 20).
+        static_assert(KQ == 4, "four outputs per column tile and 32 rows");
+        float z[4] = {0.f, 0.f, 0.f, 0.f};  // 0 * v summed: 0 unless a v is infinite or NaN
+#pragma unroll
+        for (int q = 0; q < MT * 8; q++) z[q % 4] = fmaf(v[q / 8][(q / 4) % 2][0][q % 4], 0.f, z[q % 4]);
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64((z[0] + z[1]) + (z[2] + z[3]) != 0.f) != 0, 0)) {
+            uint32_t again = 0;
+#pragma unroll
+            for (int q = 0; q < MT * 8; q++) {
+                const int i = q / 8, j = (q / 4) % 2, e = q % 4;
+                const bool in = 32 * (tm * MT + i) + 8 * g0 + 4 * lh + e < a.M && c0 + cj * j + li < N;
+                if (in && !(fabsf(v[i][j][0][e]) <= 3.40282347e38f)) again |= 1u << q;
+            }
+            while (__builtin_amdgcn_ballot_w64(again != 0)) {
+                const int q = again ? __builtin_ctz(again) : 0;
+                const int m = 32 * (tm * MT + q / 8) + 8 * g0 + 4 * lh + q % 4;
+                const uint8_t* const w = (q / 4) % 2 ? Bb[1] : Bb[0];
+                const uint8_t* const x = a.xa + (size_t)(m >> 5) * a_mt + 16 * (m & 31);
+                float sum = 0.f;
+#pragma unroll 1
+                for (int k = 0; k < K / 8; k++) {
+                    const u32x4 wk = *(const u32x4_a2g*)(w + (size_t)16 * k);
+                    u32x4 xk[P];
+#pragma unroll
+                    for (int p = 0; p < P; p++)
+                        xk[p] = *(const u32x4*)(x + (size_t)((k >> 1) * P + p) * kStepBytes + 512 * (k & 1));
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        float xv = 0.f;
+#pragma unroll
+                        for (int p = P - 1; p >= 0; p--) xv += part16_f32<BF>(xk[p], e);
+                        sum = fmaf(part16_f32<BF>(wk, e), xv, sum);
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < MT * 8; k++)
+                    if (again && k == q) v[k / 8][(k / 4) % 2][0][k % 4] = sum;
+                again &= again - 1;  // (0 stays 0)
+            }
+        }
+    }
 #pragma unroll
     for (int i = 0; i < MT; i++)
 #pragma unroll

@@ -644,6 +644,41 @@ def test_matmul_rows_matrix_cores_infinite_inputs(hip, torch_mod, t):
         assert np.array_equal(a[~np.isnan(a)], r[~np.isnan(r)])
 
 
+@pytest.mark.parametrize("t", [F16, BF16])
+@pytest.mark.parametrize("batch,rows,cols", [(16, 70, 1280), (40, 129, 1792), (200, 4200, 1024)])
+def test_matmul_rows_matrix_cores_infinite_weights(hip, torch_mod, t, batch, rows, cols):
+    # an infinite or NaN weight gives the infinities and NaNs of the inputs'
+    # own matvecs (a split input's small parts, zero or of the other sign, must
+    # not turn infinities into NaN), alone, in pairs of either sign, against
+    # zero and infinite inputs; the other rows stay finite
+    torch = torch_mod
+    w, X = _rows_case(hip, t, batch, rows, cols)
+    inf = {F16: 0x7C00, BF16: 0x7F80}[t]
+    W = w.view(np.uint16).reshape(rows, cols).copy()
+    W[3, 40] = inf
+    W[5, cols - 1] = inf | 0x8000
+    W[9, 100] = inf | 1
+    W[11, 3], W[11, cols - 3] = inf, inf
+    W[12, 3], W[12, cols - 3] = inf, inf | 0x8000
+    W[rows - 1, 0] = inf
+    X[4, 17] = np.inf
+    X[5, 40] = np.inf
+    X[6, 40] = 0.0
+    dw, dX = dev(torch, W.view(np.uint8).reshape(-1)), dev(torch, X)
+    out = torch.empty(batch, rows, dtype=torch.float32, device="cuda")
+    hip.quantized_matmul_rows(out, t, dw, dX, batch, rows, cols)
+    for b in list(range(8)) + [batch - 1]:
+        one = torch.empty(rows, dtype=torch.float32, device="cuda")
+        hip.quantized_matvec(one, t, dw, dX[b].contiguous(), rows, cols)
+        torch.cuda.synchronize()
+        a, r = out[b].cpu().numpy(), one.cpu().numpy()
+        assert np.array_equal(np.isnan(a), np.isnan(r)), b
+        assert np.array_equal(np.isposinf(a), np.isposinf(r)) and np.array_equal(np.isneginf(a), np.isneginf(r)), b
+    g = out[7].cpu().numpy()
+    odd = [3, 5, 9, 11, 12, rows - 1]
+    assert not np.isfinite(g[odd]).any() and np.isfinite(np.delete(g, odd)).all()
+
+
 def test_matmul_rows_any_depth_unaligned_and_captured(hip, torch_mod):
     # inputs off a 16-byte boundary take the matrix cores too; under capture
     # (no workspace there) the GEMVs run, replay for replay equal to the matvecs
