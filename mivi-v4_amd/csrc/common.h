@@ -65,6 +65,20 @@ __device__ __forceinline__ float bf16_bits_to_f32(uint32_t bits) {
     return __uint_as_float((bits & 0xFFFFu) << 16);
 }
 
+// v = b0 + b1 + b2, each the nearest bf16 to what the parts before leave
+// (24 bits in all). An infinite or NaN v is b0 alone; a finite one past the
+// largest bf16, whose nearest is infinite, takes b0 toward zero (LARGE false:
+// the caller's values are infinite, NaN or smaller than that).
+template <bool LARGE = true>
+__device__ __forceinline__ void split_bf16(float v, __bf16& b0, __bf16& b1, __bf16& b2) {
+    float hi = (float)(__bf16)v;
+    if (LARGE && fabsf(hi) == __builtin_inff()) hi = __uint_as_float(__float_as_uint(v) & 0xFFFF0000u);
+    const float r = fabsf(hi) <= 3.40282347e38f ? v - hi : 0.f;
+    b0 = (__bf16)hi;
+    b1 = (__bf16)r;
+    b2 = (__bf16)(r - (float)b1);
+}
+
 __device__ __forceinline__ uint32_t f32_to_half_bits(float f) {
     // round to nearest even (v_cvt_f16_f32 under the default rounding mode)
     return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)f);

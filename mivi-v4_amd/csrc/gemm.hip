@@ -201,11 +201,9 @@ __global__ void __launch_bounds__(512) gemm_prep_kernel(const float* __restrict_
             bf16x8 b[3];
 #pragma unroll
             for (int q = 0; q < 8; q++) {
-                b[0][q] = (__bf16)o[q];
-                const bool fin = fabsf((float)b[0][q]) <= 3.40282347e38f;
-                const float r1 = fin ? o[q] - (float)b[0][q] : 0.f;
-                b[1][q] = (__bf16)r1;
-                b[2][q] = (__bf16)(r1 - (float)b[1][q]);
+                __bf16 b0, b1, b2;
+                split_bf16(o[q], b0, b1, b2);
+                b[0][q] = b0; b[1][q] = b1; b[2][q] = b2;
             }
 #pragma unroll
             for (int p = 0; p < 3; p++) *(bf16x8*)(dst + p * PS) = b[p];

@@ -1261,14 +1261,6 @@ inline bool attn_prefill_ok(const mivi_model_info& c, bool packed) {
 // rows of a workgroup
 inline int attn_prefill_rows(int hpk) { return kPfRows * std::max(1, 4 / hpk); }
 
-// v into hi + mid + lo (an infinite v keeps its hi part only)
-__device__ __forceinline__ void split_bf16(float v, __bf16& b0, __bf16& b1, __bf16& b2) {
-    b0 = (__bf16)v;
-    const float r = fabsf((float)b0) <= 3.40282347e38f ? v - (float)b0 : 0.f;
-    b1 = (__bf16)r;
-    b2 = (__bf16)(r - (float)b1);
-}
-
 // value e of eight 16-bit ones
 template <bool BF>
 __device__ __forceinline__ float part_f32(const u32x4& w, int e) {
@@ -1663,7 +1655,7 @@ __global__ void __launch_bounds__(256, KVP == MIVI_KV_F32 ? 1 : 2) attn_prefill_
                         float w = s[8 * ks + e];
                         if constexpr (Q8) w *= scl[(2 + d) * kPfTokens + 16 * ks + 8 * (e / 4) + 4 * lh + e % 4];
                         __bf16 b0, b1, b2;
-                        split_bf16(w, b0, b1, b2);
+                        split_bf16<false>(w, b0, b1, b2);  // (p <= 256, times a block scale)
                         x[0][e] = b0; x[1][e] = b1; x[2][e] = b2;
                     }
 #pragma unroll

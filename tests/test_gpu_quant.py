@@ -644,6 +644,26 @@ def test_matmul_rows_matrix_cores_infinite_inputs(hip, torch_mod, t):
         assert np.array_equal(a[~np.isnan(a)], r[~np.isnan(r)])
 
 
+@pytest.mark.parametrize("value", [3.4028235e38, 3.3961776e38])
+def test_matmul_rows_bf16_inputs_past_the_largest_bf16(hip, torch_mod, value):
+    # finite inputs whose nearest bf16 is infinite (the largest float; the
+    # tie above the largest bf16, 3.3895e38) keep finite products; f32 sums
+    # and a 24-bit split, as test_matmul_rows_matrix_cores_any_depth
+    torch = torch_mod
+    batch, rows, cols = 16, 70, 1280
+    w, X = _rows_case(hip, BF16, batch, rows, cols)
+    X[4, 17] = value
+    X[5, 3], X[5, 4] = value, -value
+    W = (w.view(np.uint16).reshape(rows, cols).astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    out = torch.empty(batch, rows, dtype=torch.float32, device="cuda")
+    hip.quantized_matmul_rows(out, BF16, dev(torch, w), dev(torch, X), batch, rows, cols)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy().astype(np.float64)
+    ref = X.astype(np.float64) @ W.T
+    bound = 1e-5 * np.linalg.norm(X.astype(np.float64), axis=1)[:, None] * np.linalg.norm(W, axis=1)[None, :]
+    assert np.all(np.abs(got - ref) <= bound + 1e-44)
+
+
 @pytest.mark.parametrize("t", [F16, BF16])
 @pytest.mark.parametrize("batch,rows,cols", [(16, 70, 1280), (40, 129, 1792), (200, 4200, 1024)])
 def test_matmul_rows_matrix_cores_infinite_weights(hip, torch_mod, t, batch, rows, cols):
