@@ -337,6 +337,7 @@ struct RowsArgs {
     RowsSeg seg[3];
     int nseg, ntiles, mtiles;  // column tiles (all segments), row tiles
     int K, M;
+    size_t rb;                 // bytes from a weight row to the next (the rows' own, also where K is a piece of them)
     const uint8_t* xa;         // gemm_prep_kernel's operands of the rows
     const uint8_t* xs;
     const float* rowscale;
@@ -456,9 +457,7 @@ __global__ void __launch_bounds__(256, 1) gemm_rows_kernel(const RowsArgs a) {
             Br[j] = buffer_of(Wj[j] + (size_t)nt * KS * kStepBytes, (size_t)KS * kStepBytes);
             Hr[j] = buffer_of(Wj[j] + (size_t)N * K * 2 + (size_t)nt * NB * kGemmHBytes, (size_t)NB * kGemmHBytes);
         } else {
-            const size_t rb = FMT == RF_Q4 ? (size_t)NB * 144 : FMT == RF_Q6 ? (size_t)NB * 210
-                              : FMT == RF_Q8 ? (size_t)(K / 32) * 34 : (size_t)K * 2;
-            Bb[j] = Wj[j] + (size_t)min(c0 + cj * j + li, N - 1) * rb;
+            Bb[j] = Wj[j] + (size_t)min(c0 + cj * j + li, N - 1) * a.rb;
         }
     }
 
@@ -1020,6 +1019,16 @@ static void launch_rows_kernel(const RowsArgs& r, int wn, int mt, hipStream_t s)
 // rows, so that the workspace stays bounded.
 constexpr size_t kRowsSlabBytes = 256u << 20;
 
+// Deepest product of one launch: the kernel addresses the inputs of a tile
+// (256 bytes a column) in 32 bits. Deeper rows run in pieces, summed in y.
+constexpr size_t kRowsMaxDepth = 1u << 22;
+
+static size_t row_bytes(int32_t t, size_t K) {
+    size_t bs, ts;
+    format_sizes(t, &bs, &ts);
+    return K / bs * ts;
+}
+
 static size_t rows_slab(int32_t t, size_t K) {
     const size_t P = t == MIVI_GGML_BF16 ? 3 : 2;
     const size_t row_bytes = K * 2 * P + (t == MIVI_GGML_Q4_K ? K / 8 : 0) + 4;
@@ -1031,8 +1040,9 @@ size_t mivi::launch_rows_workspace(int32_t t, size_t batch, size_t K) {
     return mp * (K * 2 * P + (t == MIVI_GGML_Q4_K ? K / 8 : 0) + 4);
 }
 
-// The product with its workspace at hand.
-static int32_t rows_mfma_in(int32_t t, int pro, const GemvArgs& a, void* ws, hipStream_t s) {
+// The product with its workspace at hand; weight rows of Kw columns (Kw > K:
+// a piece of them).
+static int32_t rows_mfma_in(int32_t t, int pro, const GemvArgs& a, size_t Kw, void* ws, hipStream_t s) {
     const size_t K = (size_t)a.K, P = t == MIVI_GGML_BF16 ? 3 : 2;
     const bool q4 = t == MIVI_GGML_Q4_K, swiglu = a.epilogue == EPI_SWIGLU;
     const size_t slab = rows_slab(t, K);
@@ -1051,6 +1061,7 @@ static int32_t rows_mfma_in(int32_t t, int pro, const GemvArgs& a, void* ws, hip
         float* rs = (float*)((uint8_t*)ws + bx + bs);
         r.rowscale = rs;
         r.K = (int)K;
+        r.rb = row_bytes(t, Kw);
         r.M = M;
         r.ldy = a.ys;
         r.accumulate = a.accumulate;
@@ -1100,11 +1111,29 @@ static int32_t rows_mfma_in(int32_t t, int pro, const GemvArgs& a, void* ws, hip
 // Y_s[m * ys + n] (=|+=) sum_k W_s[n, k] * pro(X)[m, k] for the segments s
 // of a (K % 256 == 0): one activation split, one product over all segments.
 // MIVI_ERR_UNSUPPORTED when the workspace cannot be had.
-static int32_t rows_mfma(int32_t t, int pro, const GemvArgs& a, hipStream_t s, const RowsWorkspace& own) {
+static int32_t rows_mfma(int32_t t, int pro, const GemvArgs& a, hipStream_t s, const RowsWorkspace& own,
+                         size_t Kw = 0) {
     const size_t K = (size_t)a.K;
-    const bool q4 = t == MIVI_GGML_Q4_K;
+    if (!Kw) Kw = K;
+    if (K > kRowsMaxDepth) {
+        if (pro == PRO_RMSNORM || a.epilogue != EPI_STORE)  // (they need whole rows)
+            return set_error(MIVI_ERR_UNSUPPORTED, "no row product of %d columns with a norm or SwiGLU", a.K);
+        for (size_t k0 = 0; k0 < K; k0 += kRowsMaxDepth) {
+            GemvArgs p = a;
+            p.K = (int)std::min(kRowsMaxDepth, K - k0);
+            p.x += k0;
+            if (p.x2) p.x2 += k0;
+            for (int i = 0; i < a.nseg; i++) {
+                p.seg[i].W += row_bytes(t, k0);
+                p.seg[i].wg = nullptr;
+            }
+            p.accumulate = a.accumulate || k0 > 0;
+            if (int32_t rc = rows_mfma(t, pro, p, s, own, Kw)) return rc;
+        }
+        return MIVI_OK;
+    }
     size_t bytes = launch_rows_workspace(t, (size_t)a.ncol, K);
-    if (own.p && own.bytes >= bytes) return rows_mfma_in(t, pro, a, own.p, s);
+    if (own.p && own.bytes >= bytes) return rows_mfma_in(t, pro, a, Kw, own.p, s);
     int dev = 0;
     MIVI_HIP_CHECK(hipGetDevice(&dev));
     GemmWorkspace& ws = gemm_workspace(dev);
@@ -1126,7 +1155,7 @@ static int32_t rows_mfma(int32_t t, int pro, const GemvArgs& a, hipStream_t s, c
         }
         ws.bytes = bytes;
     }
-    const int32_t rc = rows_mfma_in(t, pro, a, ws.ptr, s);
+    const int32_t rc = rows_mfma_in(t, pro, a, Kw, ws.ptr, s);
     if (rc) return rc;
     MIVI_HIP_CHECK(hipEventRecord(ws.done, s));
     return MIVI_OK;

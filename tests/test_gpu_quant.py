@@ -297,6 +297,32 @@ def test_matmul_rows_mfma_ragged_and_scaled_rows(hip, oracle, torch_mod, t, batc
     _matmul_check(hip, oracle, torch, t, w, X, rows, cols)
 
 
+@pytest.mark.parametrize("t", [Q4_K, Q6_K])
+def test_matmul_rows_past_32_bit_operand_offsets(hip, oracle, torch_mod, t):
+    # 16.8 M columns: the split inputs of 64 rows pass 4 GB, so the product
+    # runs in pieces of the depth; the weights of each fifth repeat a stretch
+    # of 2048 columns of their own
+    torch = torch_mod
+    batch, rows, reps = 17, 3, 1639
+    cols = 5 * reps * 2048
+    per = [hip.synth_random_weights(t, 60 + i, rows, 2048, 0.02) for i in range(5)]
+    w = np.concatenate([np.tile(p.reshape(rows, -1), (1, reps)) for p in per], axis=1).reshape(-1)
+    X = torch.randn(batch, cols, generator=torch.Generator(device="cuda").manual_seed(61), device="cuda")
+    out = torch.full((batch * rows + 1,), 5.0, dtype=torch.float32, device="cuda")
+    hip.quantized_matmul_rows(out[:-1], t, dev(torch, w), X.reshape(-1), batch, rows, cols)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    assert got[-1] == 5.0
+    ref, norm = np.zeros((batch, rows)), np.zeros(rows)
+    for i, p in enumerate(per):
+        W = oracle.dequantize_slice(t, p, rows * 2048)[1].reshape(rows, 2048).astype(np.float64)
+        x = X[:, i * reps * 2048:(i + 1) * reps * 2048].reshape(batch, reps, 2048).sum(1, dtype=torch.float64)
+        ref += x.cpu().numpy() @ W.T
+        norm += reps * (W * W).sum(1)
+    bound = 1e-5 * X.norm(dim=1).cpu().numpy()[:, None] * np.sqrt(norm)[None, :]
+    assert np.all(np.abs(got[:-1].reshape(batch, rows) - ref) <= bound)
+
+
 def test_matmul_rows_q6k_ffn_down_prefill_shape(hip, oracle, torch_mod):
     # a Q4_K_M file's Q6_K ffn_down [2048 x 8192] on a prefill tile of 512
     # rows (the matrix-core GEMM with the per-sub-block scale)
