@@ -962,7 +962,18 @@ static int rows_route(int32_t t, const GemvArgs& a) {
     // expect. The GEMVs stage one input row in LDS: longer ones than 12288 are
     // refused there.
     if (a.K < 1024 || a.K > 12288 || a.ncol < kMfmaMinBatchRows) return 0;
-    if (kq) return 2;  // (4 inputs: 14-32 us against 24-46)
+    if (t == MIVI_GGML_Q4_K) return 2;  // (4 inputs: 14-32 us against 24-46)
+    if (t == MIVI_GGML_Q6_K) {
+        // Below 4096 rows a GEMV takes about 1.5 us and 5 for each 4096
+        // columns begun, the product 6.5 and 7.6 for each 1024 begun: at four
+        // inputs of 512 rows 16 us against 23 at 1024 columns and 41 against
+        // 48 at 4608, but 61 against 47.5 at 6400 and 96 against 77 at 12032;
+        // from six inputs on the product. More rows fill the GEMVs' CUs (8192
+        // x 6400: 61 against 130).
+        int64_t n = 0;
+        for (int i = 0; i < a.nseg; i++) n += a.seg[i].n;
+        return n >= 4096 || a.ncol * (1.5 + 5.0 * ((a.K + 4095) / 4096)) > 6.5 + 7.6 * ((a.K + 1023) / 1024) ? 2 : 0;
+    }
     // Q8_0, F16, BF16: a GEMV is near its bytes' time, so few inputs stay
     // with it. Fitted to both sides at 1024 to 8192 rows of 1024 to 4608
     // columns (f16 2048 x 2048: 4 inputs 18 us against 22, 6 inputs 26 against

@@ -608,6 +608,22 @@ def test_packed_rejects_other_types_and_shapes(hip, torch_mod):
     assert hip.last_error().code == 116
 
 
+@pytest.mark.parametrize("batch,rows,cols", [(4, 512, 6400), (5, 100, 6400), (4, 2048, 12032), (4, 65, 2304)])
+def test_matmul_rows_q6k_few_inputs_run_as_matvecs(hip, torch_mod, batch, rows, cols):
+    # few inputs over few deep Q6_K rows, where the GEMVs are faster: each
+    # input's outputs are its own matvec's bit for bit
+    torch = torch_mod
+    w = dev(torch, hip.synth_random_weights(Q6_K, 63, rows, cols, 0.02))
+    X = dev(torch, hip.synth_normal(64, batch * cols))
+    out = torch.empty(batch, rows, dtype=torch.float32, device="cuda")
+    hip.quantized_matmul_rows(out, Q6_K, w, X, batch, rows, cols)
+    one = torch.empty_like(out)
+    for b in range(batch):
+        hip.quantized_matvec(one[b], Q6_K, w, X[b * cols:(b + 1) * cols], rows, cols)
+    torch.cuda.synchronize()
+    assert torch.equal(out, one)
+
+
 def _rows_case(hip, t, batch, rows, cols):
     if t in (F16, BF16):
         W = np.random.default_rng(7 * cols + rows).standard_normal((rows, cols)) * 0.02
