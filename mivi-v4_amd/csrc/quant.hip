@@ -3901,9 +3901,11 @@ int32_t launch_dequant(int32_t t, const uint8_t* src, float* out, size_t count, 
     if (count == 0) return MIVI_OK;
     size_t threads;
     const size_t per = t == MIVI_GGML_Q4_K || t == MIVI_GGML_Q6_K ? 256 : t == MIVI_GGML_Q8_0 ? 32 : 1;
-    // Past the L2s (32 MB): around them. Two instances, since a choice at run
-    // time compiles to the cached stores.
-    const bool nt = count * per * 4 > (32u << 20);
+    // Past the L2s (32 MB): around them, where whole lines leave a wave at once
+    // (16-byte aligned outputs; off them the stores split, and Q6_K, 98304
+    // blocks, took 38.9 us around the caches against 19.5). Two instances,
+    // since a choice at run time compiles to the cached stores.
+    const bool nt = count * per * 4 > (32u << 20) && (uintptr_t)out % 16 == 0;
 #define LD(KER, ...) \
     if (nt) hipLaunchKernelGGL(KER<true>, __VA_ARGS__); else hipLaunchKernelGGL(KER<false>, __VA_ARGS__)
     switch (t) {
