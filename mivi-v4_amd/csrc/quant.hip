@@ -617,6 +617,39 @@ __global__ void __launch_bounds__(kWG) gemv_rows_kernel(const mivi::GemvArgs a) 
     }
 }
 
+// Short rows and odd widths (dense_rows_wide): one wave a row at a time, a
+// value a lane. Bound by latency; more waves than above, each with less to set
+// up: 60000 rows of 64 bf16 values 8.3 us against 14.2 above, 512 rows of 64
+// 2.5 against 3.5, of 769 (odd) 3.8 against 5.3.
+template <int KIND, int PRO>
+__global__ void __launch_bounds__(kWG) gemv_short_rows_kernel(const mivi::GemvArgs a) {
+    extern __shared__ float lds[];
+    stage_input<PRO, 0>(lds, a);
+    const int d = a.K;
+    const Segs sg(a, (size_t)d * (KIND == RK_F32 ? 4 : 2));
+    const int n = sg.n;
+    const int lane = threadIdx.x & 63;
+    const int nwaves = gridDim.x * (kWG / 64);
+    for (int r = blockIdx.x * (kWG / 64) + (threadIdx.x >> 6); r < n; r += nwaves) {
+        const uint8_t* row = sg.row(r);
+        float acc = 0.f;
+        for (int k = lane; k < d; k += 64) {
+            float w;
+            if (KIND == RK_F32) {
+                const uint8_t* p = row + 4 * (size_t)k;
+                w = ((uintptr_t)p & 3) ? __uint_as_float(p[0] | (p[1] << 8) | (p[2] << 16) | ((uint32_t)p[3] << 24))
+                                       : *(const float*)p;
+            } else {
+                const uint32_t bits = ld_u16(row + 2 * (size_t)k);
+                w = KIND == RK_F16 ? half_bits_to_f32(bits) : bf16_bits_to_f32(bits);
+            }
+            acc = fmaf(w, lds[k], acc);
+        }
+        acc = wave_sum(acc);
+        if (lane == 0) store_out(sg, a.accumulate, r, acc);
+    }
+}
+
 // ------------------------------------------------------------------- Q8_0
 
 // Q8_0 rows of block pairs (K % 64 == 0, 4-byte aligned): a lane takes whole
@@ -3359,6 +3392,30 @@ int grid_for(int waves) {
     return std::max(1, std::min(wgs, cap));
 }
 
+// Whether n F16, BF16 (eb 2) or F32 (eb 4) rows of K values stream in 16-byte
+// chunks (gemv_rows_kernel) rather than value by value (gemv_short_rows_kernel):
+// where that is the faster one, from both timed at 4 to 12288 columns and 512
+// to 60000 rows. w: the row's length in 16-bit values.
+//  Whole chunks: long rows (n 512, bf16: 768 columns 3.7 us against 3.5, 1280
+//  4.1 against 4.7), shorter ones with the rows to make up for the setup (n
+//  4096: 520 columns 3.7 against 3.8, f32 260 columns 3.4 against 3.3; n 60000: 256 columns 14.5 against 13.9,
+//  264 14.8 against 16.1, f32 192 columns 13.5 against 12.9, 224 14.2 against
+//  15.3).
+//  Odd widths, whose loads are shifted together: long rows of few (n 512: 2049
+//  columns 5.8 against 6.1; n 4096: 2563 11.8 against 13.1), or many bytes
+//  where the last batch of eight chunks a lane is not half empty (n 60000:
+//  387 columns 26.1 against 22.0, 769 27.9 against 37.1; n 16000: 1795 17.7
+//  against 23.8, 2049 31.2 against 26.4, 4105 54.5 against 48.7).
+inline bool dense_rows_wide(int eb, int K, int n, bool odd) {
+    const int w = K * (eb / 2);
+    const bool f32 = eb == 4;
+    if (!odd)
+        return w >= (f32 ? 1032 : 1024) || (n >= 4096 && w >= (f32 ? 520 : 512)) || (n >= 32768 && w > (f32 ? 384 : 256));
+    if ((n <= 2048 && w > 2048) || (n <= 4096 && w > 2560)) return true;
+    if ((int64_t)n * w < 12000000) return false;
+    return (!f32 && w > 512 && w <= 2048) || (w > 3072 && w < 4104) || w > (f32 ? 5120 : 4608);
+}
+
 template <int PRO>
 int32_t launch_pro(int32_t t, const mivi::GemvArgs& a, int n, hipStream_t s) {
     const int K = a.K;
@@ -3703,8 +3760,7 @@ int32_t launch_pro(int32_t t, const mivi::GemvArgs& a, int n, hipStream_t s) {
         if (pairs) {
             lds += (size_t)K / 64 * 272;
             const int np = K / 64, lpr = std::max(8, std::min(64, pow2_ceil(np)));
-            static const int per_cu = env_int("MIVI_GEMV_Q80_WG_PER_CU", 2);
-            const int grid = std::max(1, std::min((n + 4 * (64 / lpr) - 1) / (4 * (64 / lpr)), mivi::num_cus() * per_cu));
+            const int grid = std::max(1, std::min((n + 4 * (64 / lpr) - 1) / (4 * (64 / lpr)), mivi::num_cus() * 2));
 #define LQ(LPR, NC) hipLaunchKernelGGL((gemv_q80_pairs_kernel<LPR, NC, PRO>), dim3(grid), dim3(kWG), lds, s, a)
             if (np > 64) LQ(64, 2);
             else if (lpr == 64) LQ(64, 1);
@@ -3725,14 +3781,25 @@ int32_t launch_pro(int32_t t, const mivi::GemvArgs& a, int n, hipStream_t s) {
         const int cw = t == MIVI_GGML_F32 ? 4 : 8;
         const int nj = (K + 64 * cw - 1) / (64 * cw);
         const bool odd = K % cw != 0;
+        if (!dense_rows_wide(t == MIVI_GGML_F32 ? 4 : 2, K, n, odd)) {
+            const size_t lds = (size_t)K * 4;
+            const int grid = grid_for(n);
+#define LS(KIND) hipLaunchKernelGGL((gemv_short_rows_kernel<KIND, PRO>), dim3(grid), dim3(kWG), lds, s, a)
+            if (t == MIVI_GGML_F16) LS(RK_F16); else if (t == MIVI_GGML_BF16) LS(RK_BF16); else LS(RK_F32);
+#undef LS
+            break;
+        }
         bool even = true;  // (rows on odd bytes: ld16_a2 needs even ones)
         for (int i = 0; i < a.nseg; i++) even = even && (uintptr_t)a.seg[i].W % 2 == 0;
         // rows of up to two chunks a lane in groups of four, up to four
         // chunks in pairs, longer ones alone: eight loads a batch each way
         const int R = nj <= 2 ? 4 : nj <= 4 ? 2 : 1;
         const size_t lds = (size_t)(K + 3) / 4 * 16;
-        // two workgroups per CU: 25.2 us for bf16 65536 x 1024 (26.8 at four, 27.1 at eight)
-        static const int per_cu = env_int("MIVI_GEMV_ROWS_WG_PER_CU", 2);
+        // two workgroups per CU: 25.2 us for bf16 65536 x 1024 (26.8 at four,
+        // 27.1 at eight); three where a wave takes rows alone (bf16 4608
+        // columns, 16000 rows: 46.5 us at two, 44.7 at three; f32 2052 columns
+        // 28.8, 25.1, and 28.3 at four)
+        const int per_cu = R == 1 ? 3 : 2;
         const int grid = std::max(1, std::min(((n + R - 1) / R + 3) / 4, mivi::num_cus() * per_cu));
 #define LR(KIND, R, NJ, ODD) hipLaunchKernelGGL((gemv_rows_kernel<KIND, R, NJ, ODD, PRO>), dim3(grid), dim3(kWG), lds, s, a)
 #define LRS(KIND, ODD) \

@@ -803,6 +803,30 @@ def test_gemv_rows_any_depth(hip, oracle, torch_mod, t, rows, cols):
             assert np.all(np.abs(y[:rows].astype(np.float64) - ref) <= bound + 1e-40), (d, sh)
 
 
+@pytest.mark.parametrize("t", [F16, BF16, F32])
+@pytest.mark.parametrize("rows,cols", [(1, 1), (70, 3), (513, 255), (4096, 519), (4096, 520), (33000, 256), (33000, 264),
+                                       (70, 1023), (512, 2049), (2049, 2049), (4097, 2563), (20000, 769), (20000, 385)])
+def test_gemv_short_rows_and_odd_widths(hip, oracle, torch_mod, t, rows, cols):
+    # both sides of the choice between the value-by-value and the chunked
+    # streaming GEMV of F16 / BF16 / F32 rows, with
+    # guard values around the weights, against the f64 product: f32 sums of at
+    # most K / 64 + 10 steps a lane
+    torch = torch_mod
+    w = weights(t, rows, cols, 500 + cols)
+    x = hip.synth_normal(501, cols)
+    buf = torch.full((w.nbytes + 64,), 0xFF, dtype=torch.uint8, device="cuda")
+    buf[32:32 + w.nbytes].copy_(torch.from_numpy(w))
+    out = torch.full((rows + 1,), 7.0, dtype=torch.float32, device="cuda")
+    hip.quantized_matvec(out[:rows], t, buf[32:32 + w.nbytes], dev(torch, x), rows, cols)
+    torch.cuda.synchronize()
+    y = out.cpu().numpy()
+    assert y[-1] == 7.0
+    W = oracle.dequantize_slice(t, w, rows * cols)[1].reshape(rows, cols).astype(np.float64)
+    xd = x.astype(np.float64)
+    bound = (cols / 64 + 10) * 2.0 ** -23 * (np.abs(W) @ np.abs(xd))
+    assert np.all(np.abs(y[:rows].astype(np.float64) - W @ xd) <= bound + 1e-40)
+
+
 @pytest.mark.parametrize("t", [Q4_K, Q6_K, Q8_0, F16, BF16, F32])
 @pytest.mark.parametrize("n", [1, 3, 5, 37, 33000])
 def test_dequantize_runs_of_four_at_any_alignment(hip, oracle, torch_mod, t, n):
