@@ -776,7 +776,8 @@ def test_matmul_rows_any_depth_unaligned_and_captured(hip, torch_mod):
 
 @pytest.mark.parametrize("t", [Q8_0, F16, BF16, F32])
 @pytest.mark.parametrize("rows,cols", [(1, 64), (7, 96), (65, 320), (130, 512), (257, 1024), (9, 1088), (33, 2048),
-                                       (300, 4096), (5, 4160), (66, 8192), (3, 8256), (17, 12288)])
+                                       (300, 4096), (5, 4160), (66, 8192), (3, 8256), (17, 12288), (16384, 128),
+                                       (16385, 128), (20000, 64)])
 def test_gemv_rows_any_depth(hip, oracle, torch_mod, t, rows, cols):
     # the streaming GEMVs of Q8_0 (block pairs, 8 to 64 lanes a row, one or
     # two pairs a lane; single blocks past 8192 columns or off 4 bytes) and of
