@@ -17,7 +17,7 @@
 //
 // Order statistics run as radix searches over order-preserving 32-bit keys of
 // the floats (four 8-bit passes, 256-bin histograms in LDS); a top-k of at most
-// 64 by counting ranks first (select_kth). Probability
+// 62 by counting ranks first (select_kth). Probability
 // masses are accumulated as 2^-40 fixed-point integers, so every bin sum and
 // prefix is exact and the result does not depend on thread timing. The draw r
 // is bit-exact with the reference; the cumulative sums it is compared against
@@ -50,6 +50,7 @@ constexpr int kCandVPT = 8;               // candidates per thread of the pick w
 constexpr int kCapB = kST * kCandVPT;     // candidates a row may hold
 constexpr int kMaxChunks = kST;           // chunks the pick workgroup indexes
 constexpr int kSelMax = 256;              // elements the rank selection counts (select_kth)
+constexpr int kSelTop = 62;               // its largest k
 
 enum { kModeRow = 0, kModeGreedy = 1, kModeTopK = 2, kModeCat = 3 };
 
@@ -147,14 +148,17 @@ __device__ __forceinline__ void select_bin(const T* hist, T above, T target, uin
 }
 
 // The k-th largest active key of a workgroup of NT threads, VPT keys each
-// (1 <= k <= 64, at least k active elements, active keys > 0), in four
+// (1 <= k <= kSelTop, at least k active elements, active keys > 0), in four
 // barriers where the radix search takes twelve: the 64 maxima over the threads
 // t, t + 64, ... are distinct elements, so the k-th largest of them, T, bounds
 // the answer from below; the keys >= T (about 64 ln(64 / (64 - k)) of them
 // when the order is random) are gathered in LDS and ranked by counting. The
 // answer is the least key with fewer than k larger ones. False (in every
 // thread; K unset) where more than kSelMax keys reach T: ties, or the active
-// elements in fewer than k of the groups. Bound by its chain of barriers and
+// elements in fewer than k of the groups. At k = 64 about 300 keys reach the
+// least of the maxima, so the attempt is mostly lost (eight rows of 32000
+// logits, top-k 64: 34.7 us with it, 31.9 without); at 62 about 210 (30.4
+// against 31.8). Bound by its chain of barriers and
 // LDS round trips: eight rows of 65536 logits, default sampling (with the
 // logits' copies) 46.2 us on the radix searches, 40.4 with this in both
 // kernels and the row's zeros and generator state off the pick's chain. Called
@@ -305,7 +309,7 @@ struct CandRow {
     }
     // the key of the k-th largest candidate, where the rank selection can tell
     __device__ __forceinline__ bool kth(unsigned k, uint32_t* K) const {
-        if (k > 64) return false;
+        if (k > (unsigned)kSelTop) return false;
         uint32_t key[kCandVPT];
         bool act[kCandVPT];
 #pragma unroll
@@ -916,7 +920,7 @@ __global__ void __launch_bounds__(kCT) sample_chunk_kernel(float* logits, int64_
     unsigned nfin;
     bscan_excl<kCW>(nf, &nfin, sh.wtot);
     uint32_t K = 0;
-    if (nfin > k && !(k <= 64 && select_kth<kCT>(key, ok, k, sh.sel, &K))) {
+    if (nfin > k && !(k <= kSelTop && select_kth<kCT>(key, ok, k, sh.sel, &K))) {
         uint32_t prefix = 0, pmask = 0;
         unsigned above = 0;
         for (int pass = 0; pass < 4; pass++) {

@@ -208,11 +208,11 @@ def test_rows_ties(hip, oracle, torch_mod, scale):
     run_pair(hip, oracle, torch_mod, logits, [], cfg, 17, 16, "rows")
 
 
-@pytest.mark.parametrize("top_k", [1, 2, 40, 64, 65])
+@pytest.mark.parametrize("top_k", [1, 2, 40, 62, 63, 64, 65])
 @pytest.mark.parametrize("n,groups", [(66, 64), (1025, 64), (70001, 64), (65536, 32), (9000, 1)])
 def test_rank_selection_edges(hip, oracle, torch_mod, n, groups, top_k):
     """The rank selection of the top-k cutoff at the smallest k, its largest
-    (64; 65 takes the radix search), and with finite logits in 32 or one of the
+    (62; from 63 on the radix search), and with finite logits in 32 or one of the
     64 thread groups its lower bound comes from (fewer groups than top_k: the
     bound falls to zero and, with 32, more keys reach it than are ranked)."""
     rng = np.random.default_rng(n + top_k)
