@@ -741,6 +741,35 @@ def test_matmul_rows_matrix_cores_infinite_weights(hip, torch_mod, t, batch, row
     assert not np.isfinite(g[odd]).any() and np.isfinite(np.delete(g, odd)).all()
 
 
+def test_matmul_rows_on_many_streams(hip, torch_mod):
+    # six streams, more than the products have workspaces, over and over with
+    # inputs of their own and batches that make a workspace grow: every result
+    # equals the one the call gives alone
+    torch = torch_mod
+    cases = []
+    for i, (t, batch, rows, cols) in enumerate([(Q4_K, 20, 300, 2048), (Q8_0, 33, 500, 1024), (BF16, 64, 257, 1280),
+                                                (Q6_K, 17, 900, 8192), (F16, 200, 129, 1024), (Q4_K, 9, 640, 1280)]):
+        w, X = _rows_case(hip, t, batch, rows, cols)
+        dw, dX = dev(torch, w), dev(torch, X.reshape(-1))
+        alone = torch.empty(batch * rows, dtype=torch.float32, device="cuda")
+        hip.quantized_matmul_rows(alone, t, dw, dX, batch, rows, cols)
+        cases.append((t, dw, dX, batch, rows, cols, alone, torch.cuda.Stream()))
+    torch.cuda.synchronize()
+    outs = []
+    for r in range(12):
+        for i, (t, dw, dX, batch, rows, cols, alone, s) in enumerate(cases):
+            with torch.cuda.stream(s):
+                out = torch.full_like(alone, 3.0)
+                hip.quantized_matmul_rows(out, t, dw, dX, batch, rows, cols)
+                if r == 5 and i % 2:
+                    big = torch.empty(40 * batch * rows, dtype=torch.float32, device="cuda")
+                    hip.quantized_matmul_rows(big, t, dw, dX.repeat(40), 40 * batch, rows, cols)
+            outs.append((i, out))
+    torch.cuda.synchronize()
+    for i, out in outs:
+        assert torch.equal(out.view(torch.int32), cases[i][6].view(torch.int32)), i
+
+
 def test_matmul_rows_any_depth_unaligned_and_captured(hip, torch_mod):
     # inputs off a 16-byte boundary take the matrix cores too; under capture
     # (no workspace there) the GEMVs run, replay for replay equal to the matvecs
