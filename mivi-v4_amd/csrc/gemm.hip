@@ -1006,6 +1006,15 @@ static int rows_route(int32_t t, const GemvArgs& a) {
     return product < gemvs ? 2 : 0;
 }
 
+bool mivi::launch_rows_on_matrix_cores(int32_t t, size_t batch, size_t K) {
+    GemvArgs a = {};
+    a.seg[0].n = 1;
+    a.nseg = 1;
+    a.K = (int)std::min<size_t>(K, INT32_MAX);
+    a.ncol = (int)std::min<size_t>(batch, INT32_MAX - 64);
+    return rows_route(t, a) != 0;
+}
+
 // Workgroup shape of a product: WN column groups of 64 by KQ shares of the
 // depth, WN * KQ = 4 waves. Wider groups read the inputs fewer times; more
 // depth shares make more workgroups where the outputs alone would leave CUs

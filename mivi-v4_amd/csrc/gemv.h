@@ -107,6 +107,8 @@ int32_t launch_gemv_ex(int32_t ggml_type, int prologue, const GemvArgs& a, hipSt
 // seg[0].y) on the matrix cores only (else MIVI_ERR_UNSUPPORTED, nothing
 // launched).
 int32_t launch_rows(int32_t ggml_type, int prologue, const GemvArgs& a, hipStream_t s, const RowsWorkspace& ws = {});
+// Whether a product of `batch` rows of K columns runs on the matrix cores.
+bool launch_rows_on_matrix_cores(int32_t ggml_type, size_t batch, size_t K);
 // Workspace of a product of `batch` rows of K columns (longer batches run in slabs).
 size_t launch_rows_workspace(int32_t ggml_type, size_t batch, size_t K);
 

@@ -2494,10 +2494,18 @@ void enqueue_attn_prefill(const mivi_model_info& c, AttnArgs a, int pos0, int ro
 // against 4 x 72). The tile the caller set stays the least a pass takes, and
 // all of it for other models.
 constexpr size_t kPassRows = 2048;
+// f(the layers' projections)
+template <class F>
+void each_projection(const mivi_model* m, F f) {
+    for (const Layer& L : m->layers)
+        for (const Mat* x : {&L.wq, &L.wk, &L.wv, &L.wo, &L.in_proj, &L.out_proj, &L.gate, &L.up, &L.down})
+            if (x->w) f(*x);
+}
 size_t prefill_pass_rows(const mivi_model* m) {
     const mivi_model_info& c = m->info;
-    const bool wide = c.dim >= 1024 && c.dim % 256 == 0 && c.hidden_dim % 256 == 0 && c.hidden_dim <= 12288 &&
-                      m->prefill_tile >= kPfMinRows && attn_prefill_ok(c, m->kv_packed);
+    bool wide = c.dim >= 1024 && c.hidden_dim <= 12288 && m->prefill_tile >= kPfMinRows && attn_prefill_ok(c, m->kv_packed);
+    if (wide)
+        each_projection(m, [&](const Mat& x) { wide = wide && launch_rows_on_matrix_cores(x.type, kPfMinRows, x.cols); });
     return wide ? std::max(m->prefill_tile, kPassRows) : m->prefill_tile;
 }
 
@@ -2527,9 +2535,9 @@ int32_t prefill_buffers(mivi_model* m, size_t rows) {
     }
     parts *= c.n_heads;
     size_t ws = 0;
-    for (const Layer& L : m->layers)
-        for (const Mat* x : {&L.wq, &L.wk, &L.wv, &L.wo, &L.in_proj, &L.out_proj, &L.gate, &L.up, &L.down})
-            if (x->w) ws = std::max(ws, launch_rows_workspace(x->type, rows, x->cols));
+    each_projection(m, [&](const Mat& x) {
+        if (launch_rows_on_matrix_cores(x.type, rows, x.cols)) ws = std::max(ws, launch_rows_workspace(x.type, rows, x.cols));
+    });
     size_t off = 0;
     auto take = [&](size_t bytes) {
         const size_t o = off;

@@ -634,6 +634,26 @@ def test_prefill_tile_attention_matches_per_row_attention(hip, n_heads, n_kv, pr
         assert np.max(np.abs(ca - cb)) <= 1e-4 * np.max(np.abs(ca))
 
 
+def test_prefill_passes_keep_to_the_tile_without_matrix_cores(hip, torch_mod):
+    # tiles of 64 make up passes of 2048 rows only where every projection runs
+    # on the matrix cores: a model of F32 weights at their widths keeps its
+    # tiles, and their buffers stay small (1500 rows: about 100 MB)
+    from mivi_hip import GgmlType
+    from mivi_hip.synthmodel import build_hybrid
+    torch = torch_mod
+    img = build_hybrid(dim=1024, hidden=4608, n_layers=2, attn_layers=(1,), n_heads=16, n_kv=8, vocab=256, ctx_len=2048,
+                       seed=53, weight_type=GgmlType.F32)
+    m = hip.Model(img, max_ctx=2048)
+    m.set_prefill_strategy(64)
+    prompt = np.random.default_rng(54).integers(0, 256, 1500)
+    m.prefill(prompt[:70])
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    m.prefill(prompt)
+    torch.cuda.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] < 16 << 20
+
+
 def _patch_f32(img, name, f):
     """img with the F32 matrix `name` ([rows, cols]) changed in place by f."""
     from mivi_hip.gguf import read_tensor_index
