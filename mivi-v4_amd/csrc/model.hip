@@ -2186,7 +2186,10 @@ struct mivi_model {
     int32_t alloc(T** p, size_t count) {
         void* q = nullptr;
         hipError_t e = hipMalloc(&q, std::max<size_t>(1, count * sizeof(T)));
-        if (e != hipSuccess) return set_error(MIVI_ERR_HIP, "hipMalloc(%zu) failed: %s", count * sizeof(T), hipGetErrorString(e));
+        if (e != hipSuccess) {
+            (void)hipGetLastError();  // (the next launch's check would find it)
+            return set_error(MIVI_ERR_HIP, "hipMalloc(%zu) failed: %s", count * sizeof(T), hipGetErrorString(e));
+        }
         // zeroed on the model's stream and waited for: the stream is
         // non-blocking, so a null-stream memset could still be running (and
         // overwrite data) when the stream's next copy or kernel touches the
@@ -2509,20 +2512,9 @@ size_t prefill_pass_rows(const mivi_model* m) {
     return wide ? std::max(m->prefill_tile, kPassRows) : m->prefill_tile;
 }
 
-// Tile buffers for `rows` rows (grow-only), one allocation; a grown one takes
-// the old one's place.
-int32_t prefill_buffers(mivi_model* m, size_t rows) {
-    if (m->pf_cap >= rows) return MIVI_OK;
+// Tile buffers for `rows` rows, one allocation.
+int32_t prefill_buffers_for(mivi_model* m, size_t rows) {
     const mivi_model_info& c = m->info;
-    if (m->pf_base) {
-        // at least twice the rows, up to a whole pass: few regrowths
-        rows = std::max(rows, std::min(2 * m->pf_cap, prefill_pass_rows(m)));
-        MIVI_HIP_CHECK(hipStreamSynchronize(m->stream));
-        MIVI_HIP_CHECK(hipFree(m->pf_base));
-        m->allocs.erase(std::find(m->allocs.begin(), m->allocs.end(), (void*)m->pf_base));
-        m->pf_base = nullptr;
-        m->pf_cap = 0;
-    }
     const size_t D = c.dim, H = c.hidden_dim, KV = c.kv_dim;
     const size_t p1 = std::max({3 * D, D + 2 * KV, H});
     // attention partials: the per-row kernels' kPrefillSplits a row, or the
@@ -2558,6 +2550,24 @@ int32_t prefill_buffers(mivi_model* m, size_t rows) {
     m->pf_ws_bytes = ws;
     m->pf_cap = rows;
     return MIVI_OK;
+}
+
+// Tile buffers for at least `rows` rows (grow-only); grown ones take the old
+// ones' place.
+int32_t prefill_buffers(mivi_model* m, size_t rows) {
+    if (m->pf_cap >= rows) return MIVI_OK;
+    // at least twice the rows, up to a whole pass: few regrowths
+    const size_t most = std::max(rows, std::min(2 * m->pf_cap, prefill_pass_rows(m)));
+    if (m->pf_base) {
+        MIVI_HIP_CHECK(hipStreamSynchronize(m->stream));
+        MIVI_HIP_CHECK(hipFree(m->pf_base));
+        m->allocs.erase(std::find(m->allocs.begin(), m->allocs.end(), (void*)m->pf_base));
+        m->pf_base = nullptr;
+        m->pf_cap = 0;
+    }
+    int32_t rc = prefill_buffers_for(m, most);
+    if (rc && most > rows) rc = prefill_buffers_for(m, rows);  // no memory to spare: what the call needs
+    return rc;
 }
 
 // One prefill tile of sequence b: tokens (device) at positions p0 .. p0+rows-1
@@ -3248,7 +3258,6 @@ extern "C" int32_t mivi_hip_model_prefill(mivi_model* m, size_t seq, const uint3
         size_t tile = std::min(prefill_pass_rows(m), n);
         int32_t rc = prefill_buffers(m, tile);
         if (rc && tile > m->prefill_tile) {  // no memory for the long pass: the caller's tiles
-            (void)hipGetLastError();
             tile = std::min(m->prefill_tile, n);
             rc = prefill_buffers(m, tile);
         }

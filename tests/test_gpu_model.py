@@ -654,6 +654,51 @@ def test_prefill_passes_keep_to_the_tile_without_matrix_cores(hip, torch_mod):
     assert free - torch.cuda.mem_get_info()[0] < 16 << 20
 
 
+def test_prefill_buffers_regrow_with_little_memory(hip, torch_mod):
+    # a longer prompt grows the tile buffers (370 KB a row here) to twice their
+    # rows; with memory left for its own rows only, it takes those, and with
+    # less the call fails and the model goes on with shorter prompts
+    from mivi_hip.synthmodel import build_hybrid
+    torch = torch_mod
+    img = build_hybrid(dim=4096, hidden=2048, n_layers=1, attn_layers=(0,), n_heads=32, n_kv=8, vocab=256, ctx_len=4096,
+                       seed=55)
+    prompt = np.random.default_rng(56).integers(0, 256, 4000)
+
+    def run(m, n):
+        m.reset_context()
+        m.prefill(prompt[:n])
+        return m.forward(int(prompt[n]), n)
+
+    def model():
+        m = hip.Model(img, max_ctx=4096)
+        m.set_prefill_strategy(4096)
+        return m
+
+    m = model()
+    want = run(m, 2100)
+    m.close()
+    m = model()
+    short = run(m, 2000)
+    hold = more = None
+    try:
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        # 0.74 GB of buffers to come back, 0.78 needed, 1.48 for twice the rows
+        hold = torch.empty(torch.cuda.mem_get_info()[0] - (400 << 20), dtype=torch.uint8, device="cuda")
+        left = torch.cuda.mem_get_info()[0]
+        if left > 450 << 20:  # (the allocator keeps some of its own back)
+            more = torch.empty(left - (400 << 20), dtype=torch.uint8, device="cuda")
+        assert torch.cuda.mem_get_info()[0] < 500 << 20
+        assert np.array_equal(run(m, 2100), want)
+        with pytest.raises(hip.ModelError):
+            m.prefill(prompt[:3900])
+        assert np.array_equal(run(m, 2000), short)
+    finally:
+        hold = more = None
+        torch.cuda.empty_cache()
+    assert np.array_equal(run(m, 2100), want)
+
+
 def _patch_f32(img, name, f):
     """img with the F32 matrix `name` ([rows, cols]) changed in place by f."""
     from mivi_hip.gguf import read_tensor_index
