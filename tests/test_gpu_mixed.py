@@ -101,16 +101,17 @@ def test_mixed_token_path_matches_oracle(hip, oracle, mixed_img):
 
 @pytest.mark.parametrize("tile", [64, 512])
 def test_mixed_chunked_prefill_matches_oracle(hip, oracle, mixed_img, tile):
-    # PrefillStrategy::Chunked on a 600-token prompt (tile 512: 512 + 87
-    # rows, tile 64: nine tiles + 23 rows): the Q6_K ffn_down and v products
-    # on the matrix cores with the Q4_K ones; the next token's logits and 8
+    # PrefillStrategy::Chunked on a 600-token prompt in calls of `tile` tokens
+    # (512 + 87; nine of 64 and 23: one call would be one pass): the Q6_K
+    # ffn_down and v products on the matrix cores with the Q4_K ones; the next token's logits and 8
     # greedy tokens against the oracle's token path
     prompt = np.random.default_rng(63).integers(0, MIXED["vocab"], 600)
     lo, want = oracle_run(oracle, mixed_img, prompt, 8)
     m = hip.Model(mixed_img, max_ctx=1024)
     m.set_prefill_strategy(tile)
-    m.prefill(prompt[:-1])
     n = len(prompt) - 1
+    for p in range(0, n, tile):
+        m.prefill(prompt[p:min(p + tile, n)], p)
     lg = m.forward(int(prompt[-1]), n)
     assert rel_err(lg, lo) <= 1e-3, rel_err(lg, lo)
     assert int(np.argmax(lg)) == want[0]

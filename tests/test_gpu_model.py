@@ -247,9 +247,10 @@ def test_chunked_prefill_matches_token_prefill_and_oracle(hip, oracle, small_img
 
 
 def test_chunked_prefill_full_width_matrix_cores(hip):
-    # dim 2048: tiles of 64 rows run the projections on the MFMA GEMM (RMSNorm
-    # and SwiGLU in the activation split, residual adds in its store); the
-    # ragged last tile (8 rows) the batched GEMV
+    # dim 2048, in calls of 64 tokens (one call would be one pass of 200 rows):
+    # 64 rows run the projections on the matrix cores (RMSNorm in the
+    # activation split, SwiGLU and residual adds in the store), the ragged
+    # last 8 the batched GEMV
     from mivi_hip.synthmodel import build_hybrid
     img = build_hybrid(dim=2048, hidden=8192, n_layers=3, attn_layers=(1,), n_heads=32, n_kv=8, vocab=4096,
                        ctx_len=1024, seed=11)
@@ -259,7 +260,8 @@ def test_chunked_prefill_full_width_matrix_cores(hip):
     mt.prefill(prompt[:-1])
     mc = hip.Model(img, max_ctx=512)
     mc.set_prefill_strategy(64)
-    mc.prefill(prompt[:-1])
+    for p in range(0, n, 64):
+        mc.prefill(prompt[p:min(p + 64, n)], p)
     lt, lc = mt.forward(int(prompt[-1]), n), mc.forward(int(prompt[-1]), n)
     assert rel_err(lc, lt) <= 1e-3
     tok = int(np.argmax(lt))
@@ -571,8 +573,8 @@ def test_qk_norm_token_and_chunked_paths_match_oracle(hip, oracle, prec, oprec):
 @pytest.mark.parametrize("prec,oprec", [(2, 100), (1, 1)])
 def test_qk_norm_full_width_matches_oracle(hip, oracle, prec, oprec):
     # the decode shapes (dim 2048, 32 query heads over 8 kv heads, head_dim 64)
-    # with QK-norm: token path and tiles of 64 rows (the MFMA GEMM, a ragged
-    # last tile) against the oracle; the Q8_0 cache runs the matrix-core
+    # with QK-norm: token path and calls of 64 tokens (the matrix-core
+    # products, a ragged last call) against the oracle; the Q8_0 cache runs the matrix-core
     # attention and, as above, is checked code by code and then from the
     # device's own cache bytes
     from mivi_hip.synthmodel import build_hybrid
@@ -590,7 +592,8 @@ def test_qk_norm_full_width_matches_oracle(hip, oracle, prec, oprec):
     for tile in (0, 64):
         m = hip.Model(img, max_ctx=512, kv_precision=prec)
         m.set_prefill_strategy(tile)
-        m.prefill(prompt[:-1])
+        for p in range(0, n, tile or n):
+            m.prefill(prompt[p:min(p + (tile or n), n)], p)
         if prec == 1:
             row = m.kv_row_bytes()
             k, v, _ = m.export_state(n)
@@ -632,6 +635,70 @@ def test_prefill_tile_attention_matches_per_row_attention(hip, n_heads, n_kv, pr
             x, y = x.view(dt).astype(np.float64), y.view(dt).astype(np.float64)
             assert np.max(np.abs(x - y)) <= step * np.max(np.abs(x))
         assert np.max(np.abs(ca - cb)) <= 1e-4 * np.max(np.abs(ca))
+
+
+@pytest.mark.parametrize("prec,oprec", [(0, 0), (2, 100), (1, 1)])
+@pytest.mark.parametrize("cuts", [(70, 130, 9), (2057,), (2088,), (40, 2048, 300)])
+def test_prefill_passes_full_width_match_token_path(hip, oracle, prec, oprec, cuts):
+    # a model on the matrix cores at the decode shapes: prompts in several
+    # calls (pos0 > 0, the ShortConv state carried, buffers that grow), one
+    # pass of 2048 rows and a tail of 9 (batched GEMVs, per-row attention), of
+    # 40 (matrix cores, per-row attention) and of 300 rows; K and V, the
+    # ShortConv state and the next token's logits against the token path
+    # (Q8_0 caches: codes within a step of the token path's, logits against
+    # the oracle on the device's own cache)
+    from mivi_hip.synthmodel import build_hybrid
+    img = build_hybrid(dim=2048, hidden=8192, n_layers=3, attn_layers=(0, 2), n_heads=32, n_kv=8, vocab=512,
+                       ctx_len=4096, seed=57)
+    n = sum(cuts)
+    prompt = np.random.default_rng(58).integers(0, 512, n + 1)
+    mt = hip.Model(img, max_ctx=2500, kv_precision=prec)
+    mt.prefill(prompt[:n])
+    m = hip.Model(img, max_ctx=2500, kv_precision=prec)
+    m.set_prefill_strategy(64)
+    p = 0
+    for c in cuts:
+        m.prefill(prompt[p:p + c], p)
+        p += c
+    (kt, vt, ct), (k, v, conv) = mt.export_state(n), m.export_state(n)
+    # float arithmetic in another order, an fp16 step (2^-10), a Q8_0 code (1 /
+    # 127) of a cached value: what each may move the state by, of its largest
+    tol = {0: 1e-4, 2: 2.0 ** -10, 1: 1 / 127}[prec]
+    assert np.max(np.abs(ct - conv)) <= tol * np.max(np.abs(ct))
+    tok, row = int(prompt[n]), m.kv_row_bytes()
+    if prec == 1:
+        assert q8_rows_close(k, kt, n, 2, row) and q8_rows_close(v, vt, n, 2, row)
+        lo = oracle_from_device(oracle, img, m, n, oprec, 2500).forward(tok, n)
+    else:
+        dt = np.float32 if prec == 0 else np.float16
+        for x, y in ((k, kt), (v, vt)):
+            x, y = x.view(dt).astype(np.float64), y.view(dt).astype(np.float64)
+            assert np.max(np.abs(x - y)) <= tol * np.max(np.abs(y))
+        lo = mt.forward(tok, n)
+    assert rel_err(m.forward(tok, n), lo) <= 1e-3
+
+
+@pytest.mark.parametrize("t,hidden", [(1, 1000), (8, 1056), (8, 4608), (12, 4608)])
+def test_prefill_swiglu_store_off_its_tiles(hip, t, hidden):
+    # gate and up rows that do not fill the product's tiles of 32 pairs (F16),
+    # a down projection on the GEMVs (Q8_0, 1056 columns), and the
+    # loader's default widths: one pass against the token path
+    from mivi_hip import GgmlType
+    from mivi_hip.synthmodel import build_hybrid
+    img = build_hybrid(dim=1024, hidden=hidden, n_layers=3, attn_layers=(1,), n_heads=16, n_kv=8, vocab=512, ctx_len=512,
+                       seed=59, weight_type=GgmlType(t))
+    prompt = np.random.default_rng(60).integers(0, 512, 131)
+    n = len(prompt) - 1
+    mt, m = hip.Model(img, max_ctx=512), hip.Model(img, max_ctx=512)
+    mt.prefill(prompt[:n])
+    m.set_prefill_strategy(64)
+    m.prefill(prompt[:n])
+    (kt, vt, ct), (k, v, conv) = mt.export_state(n), m.export_state(n)
+    for x, y in ((k, kt), (v, vt)):
+        x, y = x.view(np.float32).astype(np.float64), y.view(np.float32).astype(np.float64)
+        assert np.max(np.abs(x - y)) <= 1e-4 * np.max(np.abs(y))
+    assert np.max(np.abs(ct - conv)) <= 1e-4 * np.max(np.abs(ct))
+    assert rel_err(m.forward(int(prompt[n]), n), mt.forward(int(prompt[n]), n)) <= 1e-4
 
 
 def test_prefill_passes_keep_to_the_tile_without_matrix_cores(hip, torch_mod):

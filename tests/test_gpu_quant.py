@@ -741,6 +741,27 @@ def test_matmul_rows_matrix_cores_infinite_weights(hip, torch_mod, t, batch, row
     assert not np.isfinite(g[odd]).any() and np.isfinite(np.delete(g, odd)).all()
 
 
+@pytest.mark.parametrize("t,batch,rows", [(BF16, 3584 + 5, 3), (Q4_K, 2 * 5248 + 70, 40)])
+def test_matmul_rows_in_slabs(hip, oracle, torch_mod, t, batch, rows):
+    # batches past the 256 MB of split inputs a launch takes (3584 and 5248
+    # rows of 12288 columns): several slabs through one workspace, a short last
+    # one; against the f64 product
+    torch = torch_mod
+    cols = 12288
+    w = hip.synth_random_weights(t, 65, rows, cols, 0.02) if t == Q4_K else weights(t, rows, cols, 65)
+    X = torch.randn(batch, cols, generator=torch.Generator(device="cuda").manual_seed(66), device="cuda")
+    X *= torch.exp(torch.linspace(-20, 20, batch, device="cuda"))[:, None]
+    out = torch.full((batch * rows + 1,), 5.0, dtype=torch.float32, device="cuda")
+    hip.quantized_matmul_rows(out[:-1], t, dev(torch, w), X.reshape(-1), batch, rows, cols)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    assert got[-1] == 5.0
+    W = oracle.dequantize_slice(t, w, rows * cols)[1].reshape(rows, cols).astype(np.float64)
+    ref = (X.double() @ torch.from_numpy(W).cuda().T).cpu().numpy()
+    bound = 1e-5 * X.double().norm(dim=1).cpu().numpy()[:, None] * np.linalg.norm(W, axis=1)[None, :]
+    assert np.all(np.abs(got[:-1].reshape(batch, rows) - ref) <= bound)
+
+
 def test_matmul_rows_on_many_streams(hip, torch_mod):
     # six streams, more than the products have workspaces, over and over with
     # inputs of their own and batches that make a workspace grow: every result

@@ -1,18 +1,18 @@
 """GPU parity at the decode benchmark's own workloads (BASELINE configs 4 and 5).
 
 Config 4: the 1.2B hybrid with an fp16 cache filled by a 4096-token chunked
-prefill (tiles of 512 rows, the matrix-core GEMM), working context 4352 (YaRN
+prefill (passes of 2048 rows, the matrix-core products), working context 4352 (YaRN
 scale 1.0625), then 256 greedy steps. The oracle continues from the state the
 GPU built (exported, then imported into the oracle's fp16-rounded cache mode),
 as the CPU leg of the benchmark does.
 
-Config 4's prefill itself: the GPU's tile-512 prefill of a 1024-token prompt
-at the config-4 working context (YaRN on) against the oracle's token path
+Config 4's prefill itself: the GPU's prefill of a 1024-token prompt in two
+passes of 512 rows at the config-4 working context (YaRN on) against the oracle's token path
 over the same prompt: every fp16 K/V value within one fp16 step, the
 ShortConv state within 1e-3, and the next token's logits.
 
 Config 5: 8 sequences, each a seeded uniform-random prompt of 32768 tokens
-prefilled in tiles of 512 rows into its own Q8_0 cache (working context
+prefilled in passes of 2048 rows into its own Q8_0 cache (working context
 32896, YaRN scale 8.03), stepped together through the batched path (one GEMV
 over the 8 columns per projection, one attention launch with the batch's
 split count). The oracle continues each sequence from the state the GPU
@@ -87,8 +87,8 @@ def test_config4_workload_matches_oracle(hip, oracle, img_1b2):
 
 
 def test_config4_prefill_matches_oracle_token_path(hip, oracle, img_1b2):
-    """The GPU's chunked prefill (tiles of 512 rows: the matrix-core GEMM,
-    the rows' attention) against the oracle's token path (the reference's
+    """The GPU's chunked prefill (two passes of 512 rows: the matrix-core
+    products, the tile attention) against the oracle's token path (the reference's
     default strategy) over a 1024-token prompt at the config-4 working context
     (4352, YaRN on). Both caches hold fp16 roundings of nearly the same
     floats, but the two paths' projections differ in their float arithmetic
@@ -108,7 +108,8 @@ def test_config4_prefill_matches_oracle_token_path(hip, oracle, img_1b2):
     m = hip.Model(img_1b2, max_ctx=ctx, kv_precision=hip.KvPrecision.F16)
     assert m.info.yarn == 1
     m.set_prefill_strategy(512)
-    m.prefill(prompt[:-1])
+    for p in range(0, n, 512):  # (one call would be one pass of 1024 rows)
+        m.prefill(prompt[p:p + 512], p)
     k, v, conv = m.export_state(n)
     mt = hip.Model(img_1b2, max_ctx=ctx, kv_precision=hip.KvPrecision.F16)
     mt.prefill(prompt[:-1])
