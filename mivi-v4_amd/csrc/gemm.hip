@@ -1180,6 +1180,14 @@ static int32_t rows_mfma(int32_t t, int pro, const GemvArgs& a, hipStream_t s, c
     GemmWorkspaces& all = gemm_workspaces(dev);
     std::lock_guard<std::mutex> lk(all.mu);
     GemmWorkspace* ws = &workspace_of(all, s);
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();
+    if (cap != hipStreamCaptureStatusNone && (ws->bytes < bytes || ws->stream == s)) {
+        // no allocation in a capture, and no wait for what the capturing
+        // stream itself ran before it: another stream's buffer, if one will do
+        for (GemmWorkspace& w : all.slot)
+            if (w.bytes >= bytes && w.stream != s) ws = &w;
+    }
     if (ws->bytes < bytes) {
         if (ws->ptr) {
             MIVI_HIP_CHECK(hipEventSynchronize(ws->done));

@@ -791,6 +791,33 @@ def test_matmul_rows_on_many_streams(hip, torch_mod):
         assert torch.equal(out.view(torch.int32), cases[i][6].view(torch.int32)), i
 
 
+def test_matmul_rows_captured_after_another_stream(hip, torch_mod):
+    # K-quants at the depths that always take the matrix cores, captured on a
+    # stream of its own after a call on another one (whose workspace the
+    # capture, which cannot allocate, goes on with): replays with eager calls
+    # in between
+    torch = torch_mod
+    batch, rows, cols = 64, 256, 2048
+    w, X = _rows_case(hip, Q4_K, batch, rows, cols)
+    dw, dX = dev(torch, w), dev(torch, X.reshape(-1))
+    ref = torch.empty(batch * rows, dtype=torch.float32, device="cuda")
+    out = torch.empty_like(ref)
+    hip.quantized_matmul_rows(ref, Q4_K, dw, dX, batch, rows, cols)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=torch.cuda.Stream()):
+        hip.quantized_matmul_rows(out, Q4_K, dw, dX, batch, rows, cols)
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref)
+        out.zero_()
+        hip.quantized_matmul_rows(out, Q4_K, dw, dX, batch, rows, cols)
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref)
+
+
 def test_matmul_rows_any_depth_unaligned_and_captured(hip, torch_mod):
     # inputs off a 16-byte boundary take the matrix cores too; under capture
     # (no workspace there) the GEMVs run, replay for replay equal to the matvecs
