@@ -106,9 +106,12 @@ int32_t mivi_hip_try_matvec_bf16(float* out, size_t out_len, const uint8_t* weig
  * matvec path (lib.rs:173-182). On the matrix cores: Q4_K and Q6_K with batch
  * >= 16 and cols a multiple of 2048; with cols another multiple of 256 from
  * 1024 to 12288 Q4_K and Q6_K with batch >= 4; with any of these cols Q8_0, F16
- * and BF16 from the batch on where that is faster (about 4 to 12); the last
- * two unless the stream is capturing. Other cases one GEMV per input row or
- * per few. */
+ * and BF16 from the batch on where that is faster (about 4 to 12; Q6_K of few
+ * and deep rows from 6 on); the last two unless the stream is capturing. Other
+ * cases one GEMV per input row or per few. On the matrix cores the order of a
+ * row's sums, and so its last bits, depends on the batch it is in. The products
+ * keep up to four workspaces per device (256 MB of split inputs each, at most,
+ * up to 4 M columns); calls may come from any thread and stream. */
 int32_t mivi_hip_quantized_matmul_rows(float* out, size_t out_len, int32_t ggml_type,
                                        const uint8_t* weights, size_t weights_len,
                                        const float* inputs, size_t inputs_len, size_t batch,
@@ -267,10 +270,11 @@ int32_t mivi_hip_model_generate_greedy(mivi_model* m, size_t batch, const uint32
  * PrefillStrategy::Token, forward_step(tokens[i], pos0 + i, false) per token;
  * after mivi_hip_model_set_prefill_tile(m, t > 1), PrefillStrategy::Chunked:
  * tiles of t tokens (from t = 64 on, as many as make up to 2048 tokens where
- * every product runs on the matrix cores) through every layer at once (model.rs:676-831,
+ * every projection's type and shape runs on the matrix cores; without memory
+ * for that, t) through every layer at once (model.rs:676-831,
  * attention_forward_tile transformer.rs:356-559, ssm_forward_tile
- * ssm.rs:174-387): row-batch products (matrix cores for Q4_K), K/V and the
- * ShortConv state left as the token path leaves them. Synchronous. */
+ * ssm.rs:174-387): row-batch products, K/V and the ShortConv state left as the
+ * token path leaves them. Synchronous. */
 int32_t mivi_hip_model_prefill(mivi_model* m, size_t seq, const uint32_t* tokens, size_t n,
                                size_t pos0);
 

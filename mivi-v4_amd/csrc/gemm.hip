@@ -51,7 +51,8 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // fp16 planes (P = 2): the row scaled by the power of two that puts its
 // largest finite |v| in [2^14, 2^15) (so the lo part of a value within 2^-15
 // of the largest is no denormal) and split v = hi + lo, each rounded to
-// nearest: v to about 2^-24 relative. bf16 planes (P = 3, bf16 weights, whose
+// nearest: v to 2^-23 relative, from 2^-17 of the largest down to 2^-39 of the
+// largest. bf16 planes (P = 3, bf16 weights, whose
 // range fp16 does not cover): v = hi + mid + lo unscaled. An infinite value
 // keeps its hi part only (no inf - inf).
 // Operand order: per 32 rows and 16-value k-step, one 1 KB block per plane,
@@ -977,11 +978,12 @@ static int rows_route(int32_t t, const GemvArgs& a) {
         const bool aligned = a16(a.x) && a16(a.x2) && a16(a.norm_w) && a.xs % 4 == 0;
         return a.ncol >= kMfmaMinBatch && aligned ? 1 : 0;
     }
-    // From 1024 columns, the narrowest of the loader's configurations: models
-    // narrower than that (test sizes) keep the GEMVs, whose chunked prefill
-    // then equals the token path bit for bit, as the tests over Q8_0 caches
-    // expect. The GEMVs stage one input row in LDS: longer ones than 12288 are
-    // refused there.
+    // Rows under 1024 columns (narrower than the loader's configurations) keep
+    // the GEMVs and with them each matvec's own bits: over a Q8_0 cache one
+    // flipped code shows in the logits of a small model. The product is the
+    // faster side there too (512 x 512, Q4_K: 4 inputs 18.6 us against 12.5, 128
+    // inputs 624 against 13). The GEMVs stage one input row in LDS: longer ones
+    // than 12288 are refused there.
     if (a.K < 1024 || a.K > 12288 || a.ncol < kMfmaMinBatchRows) return 0;
     if (t == MIVI_GGML_Q4_K) return 2;  // (4 inputs: 14-32 us against 24-46)
     if (t == MIVI_GGML_Q6_K) {
@@ -998,7 +1000,10 @@ static int rows_route(int32_t t, const GemvArgs& a) {
     // Q8_0, F16, BF16: a GEMV is near its bytes' time, so few inputs stay
     // with it. Fitted to both sides at 1024 to 8192 rows of 1024 to 4608
     // columns (f16 2048 x 2048: 4 inputs 18 us against 22, 6 inputs 26 against
-    // 23; Q8_0 1024 x 4608: 8 inputs 34 against 52, 12 inputs 50 against 52).
+    // 23; Q8_0 1024 x 4608: 8 inputs 34 against 52, 12 inputs 50 against 52);
+    // timed again at 1 to 8192 rows of 1024 to 12288 columns and 4 to 32
+    // inputs, it takes the faster side or one within 9 % of it but for Q8_0
+    // 4608 x 2048 at 6 inputs (29 us against 25).
     double bytes = 0;
     for (int i = 0; i < a.nseg; i++) bytes += (double)a.seg[i].n * a.K * (t == MIVI_GGML_Q8_0 ? 34.0 / 32 : 2.0);
     const double gemvs = a.ncol * (3.2 + bytes / 4.2e6);
@@ -1019,7 +1024,13 @@ bool mivi::launch_rows_on_matrix_cores(int32_t t, size_t batch, size_t K) {
 // depth, WN * KQ = 4 waves. Wider groups read the inputs fewer times; more
 // depth shares make more workgroups where the outputs alone would leave CUs
 // idle. Picks the least rounds(workgroups / CUs) * (fixed + super-blocks per
-// wave).
+// wave), one workgroup a CU. Against all three widths timed at seven shapes of
+// 512 to 16384 rows, 2048 to 8192 columns and 16 to 2048 inputs, within 6 % of
+// the fastest for 153 of 168; the rest up to 38 % over it, Q6_K, whose narrow
+// groups of 64 rows do better than this says (2048 x 8192, 1024 inputs: 203 us
+// wide, 147 narrow), and Q4_K at 512 rows and 2048 inputs (42 us, 31 at two
+// column groups). The shares change the order of a row's sums with the number
+// of inputs, so its last bits depend on the batch it is in.
 struct RowsTile {
     int wn, ntiles;
 };
@@ -1047,12 +1058,21 @@ template <int FMT>
 static void launch_rows_kernel(const RowsArgs& r, int wn, int mt, hipStream_t s) {
     const dim3 grid((unsigned)(r.ntiles * r.mtiles));
 #define LR(WN, MT, MID) hipLaunchKernelGGL((gemm_rows_kernel<FMT, WN, 4 / WN, MT, MID>), grid, dim3(256), 0, s, r)
+    // Without MID a chain runs over a whole super-block (Q4_K) and its sums go
+    // straight into the accumulators: the depths of the batched GEMVs, in
+    // workgroups of any width. Other depths replace f32 GEMVs, which the longer
+    // chains would not match (errors at 1024 to 12032 columns: Q4_K 3.7e-7 to
+    // 4.0e-7 without MID, 2.7e-7 to 3.3e-7 with it, the matvecs 3.0e-7 to
+    // 3.3e-7; Q6_K up to 3.3e-7, 2.4e-7, 2.7e-7), and with MID's sums wide
+    // groups of 64 rows do not fit the registers (100 to 3340 bytes a lane
+    // spilled).
     if constexpr (FMT == RF_Q4P || FMT == RF_Q4 || FMT == RF_Q6) {
         if (wn == 4) { if (mt == 1) LR(4, 1, false); else LR(4, 2, false); return; }
         if (wn == 2) { if (mt == 1) LR(2, 1, false); else LR(2, 2, false); return; }
-        if (r.K % 2048 == 0) { if (mt == 1) LR(1, 1, false); else LR(1, 2, false); return; }
+        // (the operand copy exists at these depths only)
+        if (FMT == RF_Q4P || r.K % 2048 == 0) { if (mt == 1) LR(1, 1, false); else LR(1, 2, false); return; }
     }
-    if (mt == 1) LR(1, 1, true); else LR(1, 2, true);
+    if constexpr (FMT != RF_Q4P) { if (mt == 1) LR(1, 1, true); else LR(1, 2, true); }
 #undef LR
 }
 
@@ -1327,11 +1347,10 @@ extern "C" int32_t mivi_hip_quantized_matmul_rows(float* out, size_t out_len, in
     clear_error();
     hipStream_t s = (hipStream_t)stream;
     if (rows > (size_t)INT32_MAX || cols > (size_t)INT32_MAX || batch > (size_t)INT32_MAX - 64) return err_overflow();
-    // Q4_K / Q6_K with batch >= kMfmaMinBatch and cols % 2048 == 0: the matrix cores;
-    // otherwise one GEMV over the batch's input rows as columns: the streaming
-    // kernel reads each weight row once per two inputs, with every input's
-    // result bit-identical to its own matvec (lib.rs:404-457); other shapes
-    // run one launch per input row
+    // The matrix cores where rows_route says so; otherwise the GEMVs, the
+    // batch's input rows as columns where the streaming kernels take several,
+    // else one launch per input row, with the matvecs' own bits (lib.rs:404-457)
+    // but on the Q4_K column kernels
     mivi::GemvArgs a = {};
     a.seg[0] = {w, out, (int)rows};
     a.nseg = 1;

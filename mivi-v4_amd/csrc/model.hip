@@ -1239,7 +1239,9 @@ __global__ void __launch_bounds__(64, 2) attn_f16_mfma_kernel(AttnArgs a) {
 // of its own, p as fp16 hi + lo, K and V as stored. Q8_0: K's and V's quants
 // are exact 16-bit integers; the scores' two blocks are scaled in f32, and p *
 // (V's block scale), whose range fp16 does not cover, enters as three bf16
-// parts. F32: every operand as three bf16 parts, the products up to 2^-24.
+// parts. F32: every operand as three bf16 parts, without the products below
+// 2^-24 of the largest (logits after 300 tokens against 64 bits, four seeds at
+// dim 1024: 0.9e-6 to 1.1e-6, with the per-row kernels 0.8e-6 to 1.1e-6).
 // The softmax reference moves only when a maximum exceeds it by 2^8.
 // A product of parts cannot carry an infinity or NaN (0 * inf, and a masked
 // token's p = 0 against its V): tiles that hold one in K or V (or, with F32
@@ -2457,9 +2459,12 @@ int32_t enqueue_batch_step(mivi_model* m, size_t batch, hipStream_t s) {
 }
 
 constexpr int kPrefillSplits = 16;  // attention splits per tile row, at most
-// Shorter tiles keep the per-row kernels of the decode: the tests hold
-// chunked prefill in short tiles over Q8_0 caches, where one code's flip
-// shows, to the token path's own bits.
+// Shorter tiles keep the per-row kernels of the decode and with them the token
+// path's own bits, which a Q8_0 cache shows (one flipped code moves the logits
+// of a small model). Three attention layers at dim 2048, 2000 cached tokens:
+// 63 rows 619 us a prefill on the per-row kernels, 490 on the tile's (F16; F32
+// 785, 556; Q8_0 532, 529), 32 rows 532, 489 (631, 565; 495, 532), 8 rows 385,
+// 383 (396, 461; 392, 426).
 constexpr size_t kPfMinRows = 64;
 
 // Splits of the cached tokens where the row blocks of a tile alone would leave
@@ -2495,7 +2500,8 @@ void enqueue_attn_prefill(const mivi_model_info& c, AttnArgs a, int pos0, int ro
 // CUs; a tile of 512 leaves them 64 workgroups wide ones, or the narrow ones
 // that re-read the inputs 32 times (down projection: 185 us for 2048 rows
 // against 4 x 72). The tile the caller set stays the least a pass takes, and
-// all of it for other models.
+// all of it for other models. (At dim 2048, hidden 8192 the buffers of 2048
+// rows take 0.25 GB.)
 constexpr size_t kPassRows = 2048;
 // f(the layers' projections)
 template <class F>

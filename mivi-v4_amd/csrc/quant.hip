@@ -32,7 +32,7 @@ constexpr size_t kMaxLdsK = 12288;  // x in LDS up to this many columns
 
 // A thread decodes runs of four consecutive values, stored as 16 bytes, past
 // the caches where the output would not fit them (one value a thread and
-// 4-byte stores before: 12289 x 2048 values, Q6_K 29.9 -> 18.2 us, Q4_K 57 ->
+// 4-byte stores before: 12289 x 2048 values, Q6_K 29.4 -> 18.0 us, Q4_K 57 ->
 // 17.6, Q8_0 54 -> 18.9, F16 57 -> 23.1, 6.5 to 6.7 TB/s; with stores through
 // the caches 23.6, 32.4, 24.7 and 30). Bytes come as 16-bit loads where blocks
 // lie on 2-byte boundaries.
