@@ -62,7 +62,7 @@ struct GemvArgs {
 
 // Row products: a caller's workspace for the inputs' operand planes
 // (launch_rows_workspace bytes, 16-byte aligned, used on the launches' stream
-// only); none: the device's shared one.
+// only); none: one of the device's.
 struct RowsWorkspace {
     void* p = nullptr;
     size_t bytes = 0;
