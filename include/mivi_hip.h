@@ -110,8 +110,9 @@ int32_t mivi_hip_try_matvec_bf16(float* out, size_t out_len, const uint8_t* weig
  * and deep rows from 6 on); the last two unless the stream is capturing. Other
  * cases one GEMV per input row or per few. On the matrix cores the order of a
  * row's sums, and so its last bits, depends on the batch it is in. The products
- * keep up to four workspaces per device (256 MB of split inputs each, at most,
- * up to 4 M columns); calls may come from any thread and stream. */
+ * keep up to four workspaces per device (each at most 256 MB of split inputs,
+ * or 64 inputs of up to 4 M columns); calls may come from any thread and
+ * stream. */
 int32_t mivi_hip_quantized_matmul_rows(float* out, size_t out_len, int32_t ggml_type,
                                        const uint8_t* weights, size_t weights_len,
                                        const float* inputs, size_t inputs_len, size_t batch,
